@@ -10,7 +10,7 @@ struct JacobiPlan {
   bool grouped = false;  // pairs only within [0, split) and [split, n)
   int split = 0;
   int npo = 0;  // pairs of the first group in every step (npairs when not grouped)
-  int max_inner = 2;  // inner Jacobi sweeps per 64x64 pair problem
+  int max_inner = 0;  // inner Jacobi sweeps per 64x64 pair problem (0: by the schedule)
   // Optional HIP-event timing of the solve and A-update launches.
   bool timing = false;
   double t_solve_ms = 0.0, t_apply_ms = 0.0, t_applyc_ms = 0.0;

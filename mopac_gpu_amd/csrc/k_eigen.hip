@@ -10,6 +10,8 @@
 // In the SCF the solver starts from the previous eigenvectors (A = C^T F C is
 // then nearly diagonal and one to three sweeps converge it); the first call
 // starts from C = I.  Stopping test: max |A_ij| (i != j) <= tol * max|A_ii|.
+#include <utility>
+
 #include "common.h"
 #include "k_eigen.h"
 #include "mfma.h"
@@ -169,133 +171,206 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve(
   if (tid == 0) active[pidx] = 1;
 }
 
-// Angle of the rotation that zeroes apq in [[app, apq], [apq, aqq]] (as in
-// pair_rotation), with t = tan: after it the diagonal is app - t apq,
-// aqq + t apq.
+// Angle of the rotation that zeroes apq in [[app, apq], [apq, aqq]], the
+// root t of h t^2 + 2 d t - h = 0 (d = aqq - app, h = 2 apq) of smaller
+// magnitude: after it the diagonal is app - t apq, aqq + t apq.  The root
+// comes from FP32 (reciprocal and square root in one instruction each) and
+// one FP64 Newton step, which leaves it good to about 1e-13; what an angle
+// error leaves of apq goes to the next sweep.  c = 1 / sqrt(1 + t^2) is
+// refined to the last bit in FP64, so c^2 + s^2 = 1 as for the exact angle.
+// About 25 dependent operations instead of the 100 of an FP64 division and
+// two square roots.
 __device__ __forceinline__ void rotation_of(double app, double aqq, double apq, double& c, double& sn,
                                             double& t) {
   c = 1.0;
   sn = 0.0;
   t = 0.0;
-  if (fabs(apq) > 1.0e-300 && fabs(apq) > 1.0e-18 * sqrt(fabs(app * aqq))) {
-    const double d = aqq - app, h = 2.0 * apq;
-    t = h / (fabs(d) + sqrt(d * d + h * h));
-    if (d < 0.0) t = -t;
-    c = rsqrt(t * t + 1.0);
+  const double d = aqq - app, h = 2.0 * apq;
+  const float df = (float)d, hf = (float)h;
+  // |apq| > 1e-18 sqrt|app aqq| compared as squares; below FP32's range an
+  // element is left as it is
+  if (fabsf(hf) >= 1.2e-38f && apq * apq > 1.0e-36 * fabs(app * aqq)) {
+    const float th = df * __builtin_amdgcn_rcpf(hf);
+    const float tf = copysignf(__builtin_amdgcn_rcpf(fabsf(th) + __builtin_amdgcn_sqrtf(fmaf(th, th, 1.0f))), th);
+    t = (double)tf;
+    const double f = fma(h, fma(t, t, -1.0), 2.0 * d * t);
+    const float fp = 2.0f * fmaf(hf, tf, df);
+    if (fabsf(fp) >= 1.2e-38f) t -= f * (double)__builtin_amdgcn_rcpf(fp);
+    const double u = fma(t, t, 1.0);
+    double y = (double)__builtin_amdgcn_rsqf((float)u);
+    const double e = fma(-u, y * y, 1.0);
+    c = fma(y * e, fma(e, 0.375, 0.5), y);
     sn = t * c;
   }
 }
 
-// Thread (k1, k2) of a round: rotation k1 on rows p1, q1 and k2 on columns
-// p2, q2 of the 2x2 block it owns, and on two rows of Q's columns p2, q2.
-// Returns the new S[p1][q2].
-__device__ __forceinline__ double round_update(double (*S)[LDSW], double (*Q)[LDSW], int k1, int p1,
-                                               int q1, double c1, double s1, int p2, int q2, double c2,
-                                               double s2) {
-  const double xpp = S[p1][p2], xpq = S[p1][q2], xqp = S[q1][p2], xqq = S[q1][q2];
-  const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
-  const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
-  const double npq = s2 * rpp + c2 * rpq;
-  S[p1][p2] = c2 * rpp - s2 * rpq;
-  S[p1][q2] = npq;
-  S[q1][p2] = c2 * rqp - s2 * rqq;
-  S[q1][q2] = s2 * rqp + c2 * rqq;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = 2 * k1 + h;
-    const double u = Q[row][p2], v = Q[row][q2];
-    Q[row][p2] = c2 * u - s2 * v;
-    Q[row][q2] = s2 * u + c2 * v;
+// The value of lane (lane ^ MASK) for the masks the cross rounds step by:
+// data-parallel-primitive moves inside a row of 16 lanes, a lane exchange
+// for 16.
+template <int MASK>
+__device__ __forceinline__ double lane_xor(double v) {
+  if constexpr (MASK == 16) {
+    return __shfl_xor(v, 16, 64);
+  } else {
+    constexpr int ctrl = MASK == 1 ? 0xB1 : MASK == 2 ? 0x4E : MASK == 7 ? 0x141 : 0x140;
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, ctrl, 0xF, 0xF, true),
+                            __builtin_amdgcn_update_dpp(0, lo, ctrl, 0xF, 0xF, true));
   }
-  return npq;
 }
 
-// round_update for the cross rounds, with the elements that stay with the
-// thread through them in registers: S[k1][k2] (sll) and Q's rows 2 k1,
-// 2 k1 + 1 of column k2 (ql0, ql1).  Only the moving row q1 and column q2
-// go through LDS; the arithmetic is round_update's, in the same order.
-__device__ __forceinline__ double round_update_x(double (*S)[LDSW], double (*Q)[LDSW], int k1, int q1,
-                                                 double c1, double s1, int p2, int q2, double c2, double s2,
-                                                 double& sll, double& ql0, double& ql1) {
-  const int p1 = k1;
-  const double xpp = sll, xpq = S[p1][q2], xqp = S[q1][p2], xqq = S[q1][q2];
-  const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
-  const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
-  const double npq = s2 * rpp + c2 * rpq;
-  sll = c2 * rpp - s2 * rpq;
-  S[p1][q2] = npq;
-  S[q1][p2] = c2 * rqp - s2 * rqq;
-  S[q1][q2] = s2 * rqp + c2 * rqq;
-  {
-    const double u = ql0, v = Q[2 * k1][q2];
-    ql0 = c2 * u - s2 * v;
-    Q[2 * k1][q2] = s2 * u + c2 * v;
+// Cross round R pairs local index k with 32 + (k ^ sigma(R)).  sigma walks
+// all of 0..31 in Gray order over the basis 1, 2, 7, 15, 16, so that the
+// partners of one round are those of the round before in the lane k ^ mask.
+constexpr int cross_mask(int r) {  // sigma(r + 1) ^ sigma(r)
+  return ((r + 1) & 1) ? 1 : ((r + 1) & 2) ? 2 : ((r + 1) & 4) ? 7 : ((r + 1) & 8) ? 15 : 16;
+}
+constexpr int cross_sigma(int r) {
+  int s = 0;
+  for (int i = 0; i < r; ++i) s ^= cross_mask(i);
+  return s;
+}
+
+// A thread's share of the 64x64 problem through the cross rounds: the 2x2
+// blocks (rows k, 32 + (k ^ sigma); columns k ^ d, 32 + (k ^ d ^ sigma)) for
+// d = g and g + 16, and four rows of Q's columns k and 32 + (k ^ sigma).
+struct CrossRegs {
+  double ll[2], rr[2];   // S[k][k ^ d], S[32 + (k ^ sigma)][32 + (k ^ d ^ sigma)]
+  double ql[4], qr[4];   // Q[4 g + j][k], Q[4 g + j][32 + (k ^ sigma)]
+};
+
+template <int R>
+__device__ __forceinline__ void cross_round(double (*S)[SB], double2 (*rot)[32], double (*dgl)[SB], int k, int g,
+                                            CrossRegs& v) {
+  constexpr int SG = cross_sigma(R), b = R & 1;
+  // keeps the compiler from computing all rounds' LDS addresses ahead of the
+  // sweep loop, which spilled 35 registers
+  asm volatile("" : "+v"(k));
+  const double2 r1 = rot[b][k];
+  const double c1 = r1.x, s1 = r1.y;
+  double npq[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int k2 = k ^ (g + 16 * j);
+    const double2 r2 = rot[b][k2];
+    const double c2 = r2.x, s2 = r2.y;
+    // S[q1][k2] is read from its mirror; the lane that owns the mirror is in
+    // this wave and writes it after this read
+    double* lr = &S[k][32 + (k2 ^ SG)];
+    const double xpp = v.ll[j], xpq = *lr, xqp = S[k2][32 + (k ^ SG)], xqq = v.rr[j];
+    const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
+    const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
+    v.ll[j] = c2 * rpp - s2 * rpq;
+    npq[j] = s2 * rpp + c2 * rpq;
+    v.rr[j] = s2 * rqp + c2 * rqq;
+    *lr = npq[j];
   }
-  {
-    const double u = ql1, v = Q[2 * k1 + 1][q2];
-    ql1 = c2 * u - s2 * v;
-    Q[2 * k1 + 1][q2] = s2 * u + c2 * v;
+  if constexpr (R < 31) {
+    // rotation k of the next round acts on S[k][32 + (k ^ SGN)], which is in
+    // the block of d = SGN ^ SG
+    constexpr int SGN = cross_sigma(R + 1), M = SG ^ SGN;
+    if (g == (M & 15)) {
+      const double apq = npq[M >> 4];
+      const double dp = dgl[b][k], dq = dgl[b][32 + (k ^ SGN)];
+      double c, sn, t;
+      rotation_of(dp, dq, apq, c, sn, t);
+      rot[b ^ 1][k] = make_double2(c, sn);
+      dgl[b ^ 1][k] = dp - t * apq;
+      dgl[b ^ 1][32 + (k ^ SGN)] = dq + t * apq;
+    }
   }
-  return npq;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const double x = v.ql[j], y = v.qr[j];
+    v.ql[j] = c1 * x - s1 * y;
+    v.qr[j] = s1 * x + c1 * y;
+  }
+  if constexpr (R < 31) {
+    constexpr int M = SG ^ cross_sigma(R + 1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) v.rr[j] = lane_xor<M>(v.rr[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v.qr[j] = lane_xor<M>(v.qr[j]);
+  }
+  __syncthreads();
+}
+
+template <int... R>
+__device__ __forceinline__ void cross_rounds(std::integer_sequence<int, R...>, double (*S)[SB], double2 (*rot)[32],
+                                             double (*dgl)[SB], int k, int g, CrossRegs& v) {
+  (cross_round<R>(S, rot, dgl, k, g, v), ...);
 }
 
 // The pair solve with cross rounds.  An inner sweep is, when intra[pair] is
 // set, 31 rounds inside each 32-wide half (circle order on 32 indices, both
-// halves at once), then 32 cross rounds: round r pairs local index k with
-// 32 + (k + r) % 32, so the 1024 index pairs across the two blocks are each
-// rotated once.  The sweep schedule sets intra once per sweep of the block's
-// group, so every index pair of the matrix is rotated once per sweep, in
-// about half the sequential rounds of a full 64-index inner sweep.
+// halves at once), then 32 cross rounds, in which the 1024 index pairs
+// across the two blocks are each rotated once.  The sweep schedule sets
+// intra once per sweep of the block's group, so every index pair of the
+// matrix is rotated once per sweep, in about half the sequential rounds of a
+// full 64-index inner sweep.
 //
-// Cross rounds need one barrier each: the element rotation k of round r + 1
-// acts on, S[k][32 + (k + r + 1) % 32], lies in the 2x2 block of thread
-// (k, k + 1) in round r, so that thread computes the next angle right after
-// its own update, from the diagonals tracked in dgl (a - t apq, d + t apq
-// per rotation), and publishes it in the other buffer.
-__global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve_x(
+// A cross round needs one barrier: the element that rotation k of the next
+// round acts on is in a block of this round, whose thread computes the next
+// angle right after its update, from the diagonals tracked in dgl
+// (a - t apq, d + t apq per rotation), and publishes it in the other buffer.
+// Of a block's four elements S[k][k2] stays in its thread's register and
+// S[q1][q2] moves between lanes of the wave with the partners; S[k][q2] goes
+// through LDS, and S[q1][k2] is read as its mirror.  Q's right columns move
+// between lanes as well, so Q stays in registers.  A round then moves 36 KB
+// through LDS; with all of S and Q's moving columns there it moved 112 KB,
+// in 2-way bank conflicts.  S is stored with row stride 64: the rounds' XOR
+// patterns put 16 consecutive lanes on 16 different bank pairs.
+// Latency bound: 22 us a launch at 1020 orbitals (32 rounds, one workgroup per
+// pair), 49 us before with two inner sweeps of 1.4 times longer rounds.
+constexpr int CROSS_THREADS = 512;
+__global__ __launch_bounds__(CROSS_THREADS) void k_jac_solve_x(
     const double* __restrict__ A, int lda, int nreal, const int* __restrict__ pairs,
     const int* __restrict__ intra, double* __restrict__ Qbuf, int* __restrict__ active, double tol,
     double skip_abs, int max_inner) {
-  __shared__ double S[SB][LDSW];
+  __shared__ double S[SB][SB];
   __shared__ double Q[SB][LDSW];
   __shared__ double2 rot[2][32];
   __shared__ double dgl[2][SB];
   __shared__ int rp[32], rq[32];
-  __shared__ double red_off[SOLVE_THREADS / 64], red_dg[SOLVE_THREADS / 64];
+  __shared__ double red_off[CROSS_THREADS / 64], red_dg[CROSS_THREADS / 64];
   const int pidx = blockIdx.x;
   const int I = pairs[2 * pidx], J = pairs[2 * pidx + 1];
   const bool do_intra = intra[pidx] != 0;
   const int tid = threadIdx.x;
-  // blocks by diagonal: thread t owns (k1, k2) = (t % 32, (t % 32 + d) % 32)
-  // with d = (t / 32 + 1) % 32, so the 32 blocks (k, k + 1) whose owners
-  // compute the next round's angles are threads 0..31: one wave runs that
-  // divergent code instead of every wave running it for two lanes
-  const int k1 = tid & 31, k2 = (k1 + (((tid >> 5) + 1) & 31)) & 31;
+  const int k = tid & 31, g = tid >> 5;
   {
-    // all four loads of this thread in flight before the first LDS store
-    constexpr int PER = SB * SB / SOLVE_THREADS;
+    // all loads of this thread in flight before the first LDS store; A is
+    // symmetric, so column c of it is row c of S
+    constexpr int PER = SB * SB / CROSS_THREADS;
     double v[PER];
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
-      const int e = tid + SOLVE_THREADS * it;
+      const int e = tid + CROSS_THREADS * it;
       v[it] = A[(size_t)gidx_dev(I, J, e % SB) + (size_t)gidx_dev(I, J, e / SB) * lda];
     }
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
-      const int e = tid + SOLVE_THREADS * it, r = e % SB, c = e / SB;
-      S[r][c] = v[it];
-      Q[r][c] = (r == c) ? 1.0 : 0.0;
+      const int e = tid + CROSS_THREADS * it;
+      S[e / SB][e % SB] = v[it];
     }
   }
   __syncthreads();
+  CrossRegs v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v.ql[j] = (4 * g + j == k) ? 1.0 : 0.0;
+    v.qr[j] = (4 * g + j == 32 + k) ? 1.0 : 0.0;
+  }
   for (int sw = 0; sw < max_inner; ++sw) {
     double off = 0.0, dg = 0.0;
-    for (int e = tid; e < SB * SB; e += SOLVE_THREADS) {
-      const int r = e % SB, c = e / SB;
+#pragma unroll
+    for (int e = tid; e < SB * SB; e += CROSS_THREADS) {
+      const int r = e / SB, c = e % SB;
+      const double x = fabs(S[r][c]);
       if (r == c) {
-        if (gidx_dev(I, J, r) < nreal) dg = fmax(dg, fabs(S[r][c]));
+        if (gidx_dev(I, J, r) < nreal) dg = fmax(dg, x);
       } else {
-        off = fmax(off, fabs(S[r][c]));
+        off = fmax(off, x);
       }
     }
     off = wave_max(off);
@@ -308,7 +383,7 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve_x(
     off = 0.0;
     dg = 0.0;
 #pragma unroll
-    for (int w = 0; w < SOLVE_THREADS / 64; ++w) {
+    for (int w = 0; w < CROSS_THREADS / 64; ++w) {
       off = fmax(off, red_off[w]);
       dg = fmax(dg, red_dg[w]);
     }
@@ -319,6 +394,12 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve_x(
     }
     if (off <= tol * fmax(dg, 1.0)) break;
     if (do_intra) {
+      // Q through LDS for these rounds
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        Q[4 * g + j][k] = v.ql[j];
+        Q[4 * g + j][32 + k] = v.qr[j];
+      }
       for (int round = 0; round < 31; ++round) {
         if (tid < 32) {
           // circle order on the 32 indices of half tid / 16
@@ -333,9 +414,36 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve_x(
           rq[tid] = q;
         }
         __syncthreads();
-        const double2 r1 = rot[0][k1], r2 = rot[0][k2];
-        (void)round_update(S, Q, k1, rp[k1], rq[k1], r1.x, r1.y, rp[k2], rq[k2], r2.x, r2.y);
+        const double2 r2 = rot[0][k];
+        const int p2 = rp[k], q2 = rq[k];
+        const double c2 = r2.x, s2 = r2.y;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int k1 = g + 16 * j;
+          const double2 r1 = rot[0][k1];
+          const int p1 = rp[k1], q1 = rq[k1];
+          const double c1 = r1.x, s1 = r1.y;
+          const double xpp = S[p1][p2], xpq = S[p1][q2], xqp = S[q1][p2], xqq = S[q1][q2];
+          const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
+          const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
+          S[p1][p2] = c2 * rpp - s2 * rpq;
+          S[p1][q2] = s2 * rpp + c2 * rpq;
+          S[q1][p2] = c2 * rqp - s2 * rqq;
+          S[q1][q2] = s2 * rqp + c2 * rqq;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int row = 4 * g + j;
+          const double x = Q[row][p2], y = Q[row][q2];
+          Q[row][p2] = c2 * x - s2 * y;
+          Q[row][q2] = s2 * x + c2 * y;
+        }
         __syncthreads();
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v.ql[j] = Q[4 * g + j][k];
+        v.qr[j] = Q[4 * g + j][32 + k];
       }
     }
     // cross rounds: angles of round 0 and the diagonals after it
@@ -348,37 +456,38 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve_x(
       dgl[0][p] = app - t * apq;
       dgl[0][q] = aqq + t * apq;
     }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      v.ll[j] = S[k][k ^ (g + 16 * j)];
+      v.rr[j] = S[32 + k][32 + (k ^ (g + 16 * j))];
+    }
     __syncthreads();
-    // row k1 and column k2 of this thread's block are the same in every
-    // cross round: their shared S element and Q's two elements of column k2
-    // stay in registers until the rounds end
-    double sll = S[k1][k2], ql0 = Q[2 * k1][k2], ql1 = Q[2 * k1 + 1][k2];
-    for (int r = 0; r < 32; ++r) {
-      const int b = r & 1;
-      const double2 r1 = rot[b][k1], r2 = rot[b][k2];
-      const int q1 = 32 + ((k1 + r) & 31), q2 = 32 + ((k2 + r) & 31);
-      const double npq = round_update_x(S, Q, k1, q1, r1.x, r1.y, k2, q2, r2.x, r2.y, sll, ql0, ql1);
-      if (r < 31 && tid < 32) {  // thread (k1, k1 + 1)
-        // rotation k1 of round r + 1 pairs k1 with q2
-        const double dp = dgl[b][k1], dq = dgl[b][q2];
-        double c, sn, t;
-        rotation_of(dp, dq, npq, c, sn, t);
-        rot[b ^ 1][k1] = make_double2(c, sn);
-        dgl[b ^ 1][k1] = dp - t * npq;
-        dgl[b ^ 1][q2] = dq + t * npq;
+    cross_rounds(std::make_integer_sequence<int, 32>{}, S, rot, dgl, k, g, v);
+    // Q's right columns back in order, and S whole again for another sweep
+    constexpr int SL = cross_sigma(31);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v.qr[j] = __shfl(v.qr[j], (tid & 32) | (k ^ SL), 64);
+    if (sw + 1 < max_inner) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int d = g + 16 * j;
+        S[k][k ^ d] = v.ll[j];
+        S[32 + (k ^ SL)][32 + (k ^ d ^ SL)] = v.rr[j];
+        S[32 + k][k ^ d] = S[k ^ d][32 + k];
       }
       __syncthreads();
     }
-    S[k1][k2] = sll;
-    Q[2 * k1][k2] = ql0;
-    Q[2 * k1 + 1][k2] = ql1;
-    __syncthreads();
   }
+  // to LDS, then out with consecutive lanes on consecutive rows
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    Q[4 * g + j][k] = v.ql[j];
+    Q[4 * g + j][32 + k] = v.qr[j];
+  }
+  __syncthreads();
   double* Qo = Qbuf + (size_t)pidx * SB * SB;
-  for (int e = tid; e < SB * SB; e += SOLVE_THREADS) {
-    const int r = e % SB, c = e / SB;
-    Qo[e] = Q[r][c];
-  }
+#pragma unroll
+  for (int e = tid; e < SB * SB; e += CROSS_THREADS) Qo[e] = Q[e % SB][e / SB];
   if (tid == 0) active[pidx] = 1;
 }
 
@@ -895,6 +1004,13 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
   const int lda = plan.npad;
   int done = 0;
   hipStream_t cs = plan.cstream;
+  // Inner sweeps per step.  Cross schedule: one; a second saves up to a fifth
+  // of the sweeps (54 instead of 66 in the plain SCF of 1020 orbitals) for
+  // twice the rounds (109 ms instead of 102; 16.6 instead of 15.2 ms at 174
+  // orbitals).  A matrix that is one pair problem is solved in one launch.
+  const bool cross = g_jacobi_schedule == 1;
+  const int inner = plan.max_inner > 0 ? plan.max_inner : !cross ? 2 : plan.npairs == 1 ? 16 : 1;
+  const double inner_tol = plan.npairs == 1 ? 0.5 * tol : 1.0e-14;
   // the C updates start after whatever the caller queued on C
   MHIP_CHECK(hipEventRecord(plan.ev_join, s));
   MHIP_CHECK(hipStreamWaitEvent(cs, plan.ev_join, 0));
@@ -938,11 +1054,11 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
       if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 0], s));
       if (g_jacobi_schedule == 1) {
         const int* fl = plan.intra.as<int>() + (size_t)step * plan.npairs;
-        hipLaunchKernelGGL(k_jac_solve_x, dim3(plan.npairs), dim3(SOLVE_THREADS), 0, s, A, lda, plan.n, pr, fl,
-                           q, act, 1.0e-14, skip_abs, plan.max_inner);
+        hipLaunchKernelGGL(k_jac_solve_x, dim3(plan.npairs), dim3(CROSS_THREADS), 0, s, A, lda, plan.n, pr, fl,
+                           q, act, inner_tol, skip_abs, inner);
       } else {
         hipLaunchKernelGGL(k_jac_solve, dim3(plan.npairs), dim3(SOLVE_THREADS), 0, s, A, lda, plan.n, pr, q,
-                           act, 1.0e-14, skip_abs, plan.max_inner);
+                           act, 1.0e-14, skip_abs, inner);
       }
       MHIP_LAUNCH_CHECK();
       if (plan.timing) {
@@ -995,7 +1111,7 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
           const long long per =
               g_jacobi_schedule == 1
                   ? 1024 + (plan.intra_host[(size_t)step * plan.npairs + first] ? 992 : 0)
-                  : 2016LL * plan.max_inner;
+                  : 2016LL * inner;
           plan.active_rotations += per * act[2 * step + g];
         }
         plan.active_tiles += (long long)ntiles - u0 * (u0 + 1) / 2 - u1 * (u1 + 1) / 2;
