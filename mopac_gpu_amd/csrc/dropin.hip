@@ -17,7 +17,7 @@ struct Implicit {
   bool init = false;
   int device = 0;
   hipStream_t s = nullptr;
-  DevBuf a, b, c, d, cols, rot, cnt;
+  DevBuf a, b, c, d, e, cols, rot, cnt;
   JacobiPlan plan;
   double* hs = nullptr;
   DevBuf scal;
@@ -31,7 +31,7 @@ int g_pair[2] = {0, 1};       // mhip_set_mozyme_gpu_pair (recorded; one GPU is 
 void release_implicit() {
   if (!g_imp.init) return;
   (void)hipSetDevice(g_imp.device);
-  for (DevBuf* b : {&g_imp.a, &g_imp.b, &g_imp.c, &g_imp.d, &g_imp.cols, &g_imp.rot, &g_imp.cnt,
+  for (DevBuf* b : {&g_imp.a, &g_imp.b, &g_imp.c, &g_imp.d, &g_imp.e, &g_imp.cols, &g_imp.rot, &g_imp.cnt,
                     &g_imp.scal})
     b->release();
   g_imp.plan.release();
@@ -162,14 +162,15 @@ void mhip_dsyevd(int n, double* a, int lda, double* w, int* info) {
     I.a.ensure(sizeof(double) * full.size());
     I.c.ensure(sizeof(double) * full.size());
     I.d.ensure(sizeof(double) * full.size());
+    I.e.ensure(sizeof(double) * full.size());
     I.b.ensure(sizeof(double) * np);
     MHIP_CHECK(hipMemcpyAsync(I.a.ptr, full.data(), sizeof(double) * full.size(), hipMemcpyHostToDevice, I.s));
     jacobi_set_identity(I.s, np, I.c.as<double>(), np);
     int sweeps = 0;
-    if (jacobi_sweeps(I.s, I.plan, I.a.as<double>(), I.c.as<double>(), 1.0e-12, 60, I.hs,
-                      I.scal.as<double>(), &sweeps) != 0)
+    double *A = I.a.as<double>(), *A2 = I.e.as<double>();
+    if (jacobi_sweeps(I.s, I.plan, A, A2, I.c.as<double>(), 1.0e-12, 60, I.hs, I.scal.as<double>(), &sweeps) != 0)
       *info = 1;
-    jacobi_sort(I.s, I.plan, I.a.as<double>(), I.c.as<double>(), I.d.as<double>(), I.b.as<double>());
+    jacobi_sort(I.s, I.plan, A, I.c.as<double>(), I.d.as<double>(), I.b.as<double>());
     MHIP_CHECK(hipMemcpy2DAsync(a, sizeof(double) * lda, I.d.ptr, sizeof(double) * np,
                                 sizeof(double) * n, n, hipMemcpyDeviceToHost, I.s));
     MHIP_CHECK(hipMemcpyAsync(w, I.b.ptr, sizeof(double) * n, hipMemcpyDeviceToHost, I.s));

@@ -20,39 +20,23 @@ struct JacobiPlan {
   std::vector<int> intra_host;                    // host copy of intra
   std::vector<hipEvent_t> ev;
   DevBuf pairs;  // nsteps x npairs x 2 block indices
-  DevBuf qbuf;   // npairs x 64 x 64 rotations of the current step
+  DevBuf qbuf;   // two steps x npairs x 64 x 64 rotations
+  DevBuf diag;   // two steps x nb x 32 x 32 diagonal blocks as the solves left them
+  DevBuf where;  // nsteps x nb: 2 x (pair of the block in the step) + half
   DevBuf part;   // reduction scratch
   DevBuf perm;   // sort permutation
-  DevBuf active; // per pair: 1 when Q != I this step
+  DevBuf active; // two steps x npairs: 1 when Q != I
   DevBuf intra;  // nsteps x npairs: 1 where the cross-round solve also
                  // rotates inside the two blocks (once per sweep of a group)
   DevBuf counts; // active pairs per step (timing mode)
-  // C <- C Q runs on its own stream, behind by up to a sweep: Q and the
-  // active flags have a slot per step, and events order each slot's C update
-  // after its step's A update and before the slot's next solve
-  hipStream_t cstream = nullptr;
-  std::vector<hipEvent_t> ev_solved, ev_cdone;
-  std::vector<char> cdone_pending;
-  hipEvent_t ev_join = nullptr;
   // split > 0 (a multiple of 32 leaving an even number of blocks on both
   // sides): rotations only within the leading split columns and within the
   // rest, for a matrix already block-diagonal in that partition.
   void build(int n, int split = 0);
   void release() {
-    if (cstream) (void)hipStreamSynchronize(cstream);
-    pairs.release(); qbuf.release(); part.release(); perm.release(); active.release();
-    intra.release(); counts.release();
+    for (DevBuf* b : {&pairs, &qbuf, &diag, &where, &part, &perm, &active, &intra, &counts}) b->release();
     for (auto e : ev) (void)hipEventDestroy(e);
     ev.clear();
-    for (auto e : ev_solved) (void)hipEventDestroy(e);
-    for (auto e : ev_cdone) (void)hipEventDestroy(e);
-    ev_solved.clear();
-    ev_cdone.clear();
-    cdone_pending.clear();
-    if (ev_join) (void)hipEventDestroy(ev_join);
-    ev_join = nullptr;
-    if (cstream) (void)hipStreamDestroy(cstream);
-    cstream = nullptr;
   }
 };
 
@@ -62,9 +46,10 @@ struct JacobiPlan {
 extern int g_jacobi_schedule;
 
 void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc);
-// Sweeps until max|offdiag| <= tol * max(1, max|diag|).  Returns 0 when
-// converged, 1 when max_sweeps ran out.
-int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double tol, int max_sweeps,
+// Sweeps until max|offdiag| <= tol * max(1, max|diag|).  A2 is scratch of A's
+// size; the steps go from one to the other, and A names the one that holds
+// the result on return.  Returns 0 when converged, 1 when max_sweeps ran out.
+int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
                   double* host_scal, double* dev_scal, int* sweeps_done);
 // eig_dev[k] = k-th smallest diagonal entry, Cout[:,k] = C[:,perm[k]].
 void jacobi_sort(hipStream_t s, JacobiPlan& plan, const double* A, const double* C, double* Cout,

@@ -171,37 +171,37 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve(
   if (tid == 0) active[pidx] = 1;
 }
 
-// Angle of the rotation that zeroes apq in [[app, apq], [apq, aqq]], the
-// root t of h t^2 + 2 d t - h = 0 (d = aqq - app, h = 2 apq) of smaller
-// magnitude: after it the diagonal is app - t apq, aqq + t apq.  The root
-// comes from FP32 (reciprocal and square root in one instruction each) and
-// one FP64 Newton step, which leaves it good to about 1e-13; what an angle
-// error leaves of apq goes to the next sweep.  c = 1 / sqrt(1 + t^2) is
-// refined to the last bit in FP64, so c^2 + s^2 = 1 as for the exact angle.
-// About 25 dependent operations instead of the 100 of an FP64 division and
-// two square roots.
+// Rotation by the smaller of the angles that zero apq in [[app, apq], [apq,
+// aqq]]: with d = aqq - app, h = 2 apq and r = sqrt(d^2 + h^2), c^2 = (1 +
+// |d| / r) / 2 and s = sign(d) h / (2 r c); t = s / c, and the diagonal after
+// it is app - t apq, aqq + t apq.  c and s start in FP32 (a reciprocal square
+// root is one instruction there), an FP64 step turns them by what they leave
+// of apq (angle good to about 1e-14), and they are scaled to c^2 + s^2 = 1 in
+// FP64 to the last bit.  Every round of a pair solve waits for this chain of
+// 17 dependent operations; FP64 division and square roots take 100.  With
+// apq and d both below 1e-15, far under any stopping threshold (they are
+// absolute), nothing is turned.
 __device__ __forceinline__ void rotation_of(double app, double aqq, double apq, double& c, double& sn,
                                             double& t) {
-  c = 1.0;
-  sn = 0.0;
-  t = 0.0;
-  const double d = aqq - app, h = 2.0 * apq;
-  const float df = (float)d, hf = (float)h;
-  // |apq| > 1e-18 sqrt|app aqq| compared as squares; below FP32's range an
-  // element is left as it is
-  if (fabsf(hf) >= 1.2e-38f && apq * apq > 1.0e-36 * fabs(app * aqq)) {
-    const float th = df * __builtin_amdgcn_rcpf(hf);
-    const float tf = copysignf(__builtin_amdgcn_rcpf(fabsf(th) + __builtin_amdgcn_sqrtf(fmaf(th, th, 1.0f))), th);
-    t = (double)tf;
-    const double f = fma(h, fma(t, t, -1.0), 2.0 * d * t);
-    const float fp = 2.0f * fmaf(hf, tf, df);
-    if (fabsf(fp) >= 1.2e-38f) t -= f * (double)__builtin_amdgcn_rcpf(fp);
-    const double u = fma(t, t, 1.0);
-    double y = (double)__builtin_amdgcn_rsqf((float)u);
-    const double e = fma(-u, y * y, 1.0);
-    c = fma(y * e, fma(e, 0.375, 0.5), y);
-    sn = t * c;
-  }
+  const double d = aqq - app;
+  const float df = (float)d, ad = fabsf(df), hh = (float)apq;
+  const float r2 = fmaf(4.0f * hh, hh, ad * ad);
+  const float rinv = __builtin_amdgcn_rsqf(r2);
+  const float c2 = fmaf(0.5f * ad, rinv, 0.5f);
+  const float cinv = __builtin_amdgcn_rsqf(c2);
+  const bool none = r2 < 1.0e-30f;
+  const float cf = none ? 1.0f : c2 * cinv, sf = none ? 0.0f : copysignf(1.0f, df) * hh * rinv * cinv;
+  double c0 = (double)cf, s0 = (double)sf;
+  // the off-diagonal element after the rotation, over sign(d) r
+  const double left = fma(fma(c0, c0, -s0 * s0), apq, -(c0 * s0) * d);
+  const double turn = left * (double)(none ? 0.0f : copysignf(rinv, df));
+  const double c1 = fma(-turn, s0, c0), s1 = fma(turn, c0, s0);
+  const double e = fma(-c1, c1, fma(-s1, s1, 1.0));
+  const double corr = fma(e, fma(e, 0.375, 0.5), 1.0);
+  c = c1 * corr;
+  sn = s1 * corr;
+  const double ci = none ? 1.0 : (double)cinv;
+  t = sn * (ci * fma(-c, ci, 2.0));  // s / c, 1 / c by a Newton step from FP32's
 }
 
 // The value of lane (lane ^ MASK) for the masks the cross rounds step by:
@@ -231,66 +231,114 @@ constexpr int cross_sigma(int r) {
   return s;
 }
 
-// A thread's share of the 64x64 problem through the cross rounds: the 2x2
-// blocks (rows k, 32 + (k ^ sigma); columns k ^ d, 32 + (k ^ d ^ sigma)) for
-// d = g and g + 16, and four rows of Q's columns k and 32 + (k ^ sigma).
+// A thread's share of the 64x64 problem through the cross rounds: one 2x2
+// block (rows k, q = 32 + (k ^ sigma); columns k ^ d, 32 + (k ^ d ^ sigma)),
+// and four rows of Q's columns k and q.  k is the lane in its half-wave g.
+// S is symmetric, so of the blocks (k, k ^ d) and (k ^ d, k) only one is
+// kept: the one whose k has the highest bit of d equal to d's lowest bit
+// (d > 1), which lets d and d + 1 share a half-wave.  d = 1 has a half-wave
+// to itself with both kept; the diagonal blocks (d = 0) are the rotated pairs
+// themselves, whose diagonals dgl tracks and whose off-diagonal becomes 0.
 struct CrossRegs {
-  double ll[2], rr[2];   // S[k][k ^ d], S[32 + (k ^ sigma)][32 + (k ^ d ^ sigma)]
-  double ql[4], qr[4];   // Q[4 g + j][k], Q[4 g + j][32 + (k ^ sigma)]
+  double ll, rr;         // S[k][k ^ d], S[32 + (k ^ sigma)][32 + (k ^ d ^ sigma)]
+  double ql[4], qr[4];   // Q[4 g + j][k], Q[4 g + j][32 + (k ^ sigma)], a round behind
+  double c, s;           // the rotation Q has still to take
+  int d, top;            // top: the highest bit of d; 0 where both blocks are kept
+  int own_rot, mate_rot; // LDS byte offsets of rot[0][k], rot[0][k ^ d]
+  int lr, rl;            // and of S[k][32 + (k ^ d)], S[k ^ d][32 + k]
+  int own_q;             // and of dgl[0][32 + k]
 };
+
+__device__ __forceinline__ void cross_setup(CrossRegs& v, int k, int g) {
+  if (g < 8) { v.top = 16; v.d = 16 + 2 * g + ((k >> 4) & 1); }
+  else if (g < 12) { v.top = 8; v.d = 8 + 2 * (g - 8) + ((k >> 3) & 1); }
+  else if (g < 14) { v.top = 4; v.d = 4 + 2 * (g - 12) + ((k >> 2) & 1); }
+  else if (g < 15) { v.top = 2; v.d = 2 + ((k >> 1) & 1); }
+  else { v.top = 0; v.d = 1; }
+  const int k2 = k ^ v.d;
+  v.own_rot = k * 16;
+  v.mate_rot = k2 * 16;
+  v.lr = (k * SB + 32 + k2) * 8;
+  v.rl = (k2 * SB + 32 + k) * 8;
+  v.own_q = (32 + k) * 8;
+}
+
+__device__ __forceinline__ void cross_turn_q(CrossRegs& v) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const double x = v.ql[j], y = v.qr[j];
+    v.ql[j] = v.c * x - v.s * y;
+    v.qr[j] = v.s * x + v.c * y;
+  }
+}
+
+template <class T>
+__device__ __forceinline__ T& lds_at(void* base, int off) {
+  return *reinterpret_cast<T*>(static_cast<char*>(base) + off);
+}
+
+// the half-wave that holds d = mask
+constexpr int mask_group(int m) { return m == 1 ? 15 : m == 2 ? 14 : m == 7 ? 13 : m == 15 ? 11 : 0; }
 
 template <int R>
 __device__ __forceinline__ void cross_round(double (*S)[SB], double2 (*rot)[32], double (*dgl)[SB], int k, int g,
                                             CrossRegs& v) {
   constexpr int SG = cross_sigma(R), b = R & 1;
+  // rotation k of the next round acts on S[k][32 + (k ^ SGN)], which is in
+  // this round's block of d = M
+  constexpr int SGN = R < 31 ? cross_sigma(R + 1) : 0, M = R < 31 ? SG ^ SGN : 0;
   // keeps the compiler from computing all rounds' LDS addresses ahead of the
-  // sweep loop, which spilled 35 registers
-  asm volatile("" : "+v"(k));
-  const double2 r1 = rot[b][k];
-  const double c1 = r1.x, s1 = r1.y;
-  double npq[2];
+  // sweep loop, which spilled registers
+  asm volatile("" : "+v"(v.lr), "+v"(v.rl), "+v"(v.own_q));
+  const int lr = v.lr ^ (SG * 8), rl = v.rl ^ (SG * 8), nq = v.own_q ^ (SGN * 8);
+  const double2 r1 = lds_at<double2>(rot[b], v.own_rot), r2 = lds_at<double2>(rot[b], v.mate_rot);
+  const double xpq = lds_at<double>(S, lr), xqp = lds_at<double>(S, rl);
+  const double dp = dgl[b][k], dq = lds_at<double>(dgl[b], nq);
+  // while those arrive: Q's turn of the round before, and its partners
+  if constexpr (R > 0) {
+    constexpr int MP = cross_sigma(R - 1) ^ SG;
+    cross_turn_q(v);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int k2 = k ^ (g + 16 * j);
-    const double2 r2 = rot[b][k2];
-    const double c2 = r2.x, s2 = r2.y;
-    // S[q1][k2] is read from its mirror; the lane that owns the mirror is in
-    // this wave and writes it after this read
-    double* lr = &S[k][32 + (k2 ^ SG)];
-    const double xpp = v.ll[j], xpq = *lr, xqp = S[k2][32 + (k ^ SG)], xqq = v.rr[j];
-    const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
-    const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
-    v.ll[j] = c2 * rpp - s2 * rpq;
-    npq[j] = s2 * rpp + c2 * rpq;
-    v.rr[j] = s2 * rqp + c2 * rqq;
-    *lr = npq[j];
+    for (int j = 0; j < 4; ++j) v.qr[j] = lane_xor<MP>(v.qr[j]);
   }
+  const double c1 = r1.x, s1 = r1.y, c2 = r2.x, s2 = r2.y;
+  v.c = c1;
+  v.s = s1;
+  const double xpp = v.ll, xqq = v.rr;
+  const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
+  const double rqp = s1 * xpp + c1 * xqp, rqq = s1 * xpq + c1 * xqq;
+  const double npq = s2 * rpp + c2 * rpq, nqp = c2 * rqp - s2 * rqq;
+  v.ll = c2 * rpp - s2 * rpq;
+  v.rr = s2 * rqp + c2 * rqq;
+  // the next round's pairs are zero after it, and not read in it
+  const bool next_pair = R < 31 && v.d == M;
+  lds_at<double>(S, lr) = next_pair ? 0.0 : npq;
+  lds_at<double>(S, rl) = next_pair ? 0.0 : nqp;
   if constexpr (R < 31) {
-    // rotation k of the next round acts on S[k][32 + (k ^ SGN)], which is in
-    // the block of d = SGN ^ SG
-    constexpr int SGN = cross_sigma(R + 1), M = SG ^ SGN;
-    if (g == (M & 15)) {
-      const double apq = npq[M >> 4];
-      const double dp = dgl[b][k], dq = dgl[b][32 + (k ^ SGN)];
+    if (g == mask_group(M)) {
+      // lane k of the half-wave takes rotation k: where the block kept is
+      // that of k ^ M, its S[q1][k2]
+      const double other = lane_xor<M>(nqp);
+      const double apq = v.d == M ? npq : other;
       double c, sn, t;
       rotation_of(dp, dq, apq, c, sn, t);
-      rot[b ^ 1][k] = make_double2(c, sn);
+      lds_at<double2>(rot[b ^ 1], v.own_rot) = make_double2(c, sn);
       dgl[b ^ 1][k] = dp - t * apq;
-      dgl[b ^ 1][32 + (k ^ SGN)] = dq + t * apq;
+      lds_at<double>(dgl[b ^ 1], nq) = dq + t * apq;
     }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const double x = v.ql[j], y = v.qr[j];
-    v.ql[j] = c1 * x - s1 * y;
-    v.qr[j] = s1 * x + c1 * y;
-  }
-  if constexpr (R < 31) {
-    constexpr int M = SG ^ cross_sigma(R + 1);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) v.rr[j] = lane_xor<M>(v.rr[j]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v.qr[j] = lane_xor<M>(v.qr[j]);
+    // S[q1][q2] of the partners to come, from lane k ^ M, or from its mirror
+    // where that lane keeps the other block
+    if constexpr (M == 16) {
+      v.rr = __shfl(v.rr, (threadIdx.x & 32) | (k ^ 16 ^ (v.top == 16 ? v.d : 0)), 64);
+    } else if constexpr (M == 1) {
+      v.rr = lane_xor<1>(v.rr);
+    } else {
+      constexpr int first = M == 2 ? 14 : M == 7 ? 12 : 8;  // half-waves from here on may turn
+      if (g >= first)
+        v.rr = __shfl(v.rr, (threadIdx.x & 32) | (k ^ M ^ ((v.top & M) ? v.d : 0)), 64);
+      else
+        v.rr = lane_xor<M>(v.rr);
+    }
   }
   __syncthreads();
 }
@@ -314,85 +362,78 @@ __device__ __forceinline__ void cross_rounds(std::integer_sequence<int, R...>, d
 // angle right after its update, from the diagonals tracked in dgl
 // (a - t apq, d + t apq per rotation), and publishes it in the other buffer.
 // Of a block's four elements S[k][k2] stays in its thread's register and
-// S[q1][q2] moves between lanes of the wave with the partners; S[k][q2] goes
-// through LDS, and S[q1][k2] is read as its mirror.  Q's right columns move
-// between lanes as well, so Q stays in registers.  A round then moves 36 KB
-// through LDS; with all of S and Q's moving columns there it moved 112 KB,
-// in 2-way bank conflicts.  S is stored with row stride 64: the rounds' XOR
-// patterns put 16 consecutive lanes on 16 different bank pairs.
-// Latency bound: 22 us a launch at 1020 orbitals (32 rounds, one workgroup per
-// pair), 49 us before with two inner sweeps of 1.4 times longer rounds.
+// S[q1][q2] moves between lanes of the wave with the partners; S[k][q2] and
+// S[q1][k2] = S[k2][q1] go through LDS.  Q's right columns move between lanes
+// as well, so Q stays in registers, and its turn waits for the next round's
+// loads.  With all of S and Q's moving columns in LDS a round moved 112 KB
+// through it, in 2-way bank conflicts; now 38 KB.  S is stored with row
+// stride 64: the rounds' XOR patterns put 16 consecutive lanes on 16
+// different bank pairs.
 constexpr int CROSS_THREADS = 512;
-__global__ __launch_bounds__(CROSS_THREADS) void k_jac_solve_x(
-    const double* __restrict__ A, int lda, int nreal, const int* __restrict__ pairs,
-    const int* __restrict__ intra, double* __restrict__ Qbuf, int* __restrict__ active, double tol,
-    double skip_abs, int max_inner) {
-  __shared__ double S[SB][SB];
-  __shared__ double Q[SB][LDSW];
-  __shared__ double2 rot[2][32];
-  __shared__ double dgl[2][SB];
-  __shared__ int rp[32], rq[32];
-  __shared__ double red_off[CROSS_THREADS / 64], red_dg[CROSS_THREADS / 64];
-  const int pidx = blockIdx.x;
-  const int I = pairs[2 * pidx], J = pairs[2 * pidx + 1];
-  const bool do_intra = intra[pidx] != 0;
+
+// LDS of one workgroup of the cross schedule: two 64 x 65 tiles, shared by
+// the pair solve (S with stride 64, then Q or its two operand halves) and
+// the update tiles.
+struct JacLds {
+  double m[2 * SB * LDSW];
+  double2 rot[2][32];
+  double dgl[2][SB];
+  int rp[32], rq[32];
+  double red_off[CROSS_THREADS / 64], red_dg[CROSS_THREADS / 64];
+  __device__ double (*s())[SB] { return reinterpret_cast<double (*)[SB]>(m); }
+  __device__ double (*q())[LDSW] { return reinterpret_cast<double (*)[LDSW]>(m + SB * SB); }
+};
+
+// What a pair solve reads besides its 64x64 problem and what it writes.
+struct JacSolve {
+  int nreal;
+  double* q;      // 64 x 64 rotation, column-major
+  int* active;
+  double* di;     // the two 32 x 32 diagonal blocks after the solve (may be null)
+  double* dj;
+  double tol, skip_abs;
+  int max_inner;
+};
+
+// Diagonalizes the problem in lds.s(): the upper right quadrant and the two
+// diagonal ones, and the lower left one where do_intra asks for it.
+__device__ __forceinline__ void pair_solve(JacLds& lds, int I, int J, bool do_intra, const JacSolve& p) {
+  double(*S)[SB] = lds.s();
+  double(*Q)[LDSW] = lds.q();
   const int tid = threadIdx.x;
   const int k = tid & 31, g = tid >> 5;
-  {
-    // all loads of this thread in flight before the first LDS store; A is
-    // symmetric, so column c of it is row c of S
-    constexpr int PER = SB * SB / CROSS_THREADS;
-    double v[PER];
-#pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int e = tid + CROSS_THREADS * it;
-      v[it] = A[(size_t)gidx_dev(I, J, e % SB) + (size_t)gidx_dev(I, J, e / SB) * lda];
-    }
-#pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int e = tid + CROSS_THREADS * it;
-      S[e / SB][e % SB] = v[it];
-    }
-  }
-  __syncthreads();
   CrossRegs v;
+  cross_setup(v, k, g);
+  const int k2 = k ^ v.d;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     v.ql[j] = (4 * g + j == k) ? 1.0 : 0.0;
     v.qr[j] = (4 * g + j == 32 + k) ? 1.0 : 0.0;
   }
-  for (int sw = 0; sw < max_inner; ++sw) {
-    double off = 0.0, dg = 0.0;
-#pragma unroll
-    for (int e = tid; e < SB * SB; e += CROSS_THREADS) {
-      const int r = e / SB, c = e % SB;
-      const double x = fabs(S[r][c]);
-      if (r == c) {
-        if (gidx_dev(I, J, r) < nreal) dg = fmax(dg, x);
-      } else {
-        off = fmax(off, x);
-      }
-    }
+  bool rotated = false;
+  for (int sw = 0; sw < p.max_inner; ++sw) {
+    v.ll = S[k][k2];
+    v.rr = S[32 + k][32 + k2];
+    double off = fmax(fabs(v.ll), fabs(v.rr)), dg = 0.0;
+    off = fmax(off, fmax(fabs(S[g][32 + k]), fabs(S[16 + g][32 + k])));
+    if (tid < SB && gidx_dev(I, J, tid) < p.nreal) dg = fabs(S[tid][tid]);
     off = wave_max(off);
     dg = wave_max(dg);
     if ((tid & 63) == 0) {
-      red_off[tid >> 6] = off;
-      red_dg[tid >> 6] = dg;
+      lds.red_off[tid >> 6] = off;
+      lds.red_dg[tid >> 6] = dg;
     }
     __syncthreads();
     off = 0.0;
     dg = 0.0;
 #pragma unroll
     for (int w = 0; w < CROSS_THREADS / 64; ++w) {
-      off = fmax(off, red_off[w]);
-      dg = fmax(dg, red_dg[w]);
+      off = fmax(off, lds.red_off[w]);
+      dg = fmax(dg, lds.red_dg[w]);
     }
     __syncthreads();
-    if (sw == 0 && off <= skip_abs) {
-      if (tid == 0) active[pidx] = 0;
-      return;
-    }
-    if (off <= tol * fmax(dg, 1.0)) break;
+    if ((sw == 0 && off <= p.skip_abs) || off <= p.tol * fmax(dg, 1.0)) break;
+    rotated = true;
     if (do_intra) {
       // Q through LDS for these rounds
 #pragma unroll
@@ -405,23 +446,23 @@ __global__ __launch_bounds__(CROSS_THREADS) void k_jac_solve_x(
           // circle order on the 32 indices of half tid / 16
           const int h = tid >> 4, kk = tid & 15;
           auto pos = [&](int slot) { return slot == 0 ? 0 : 1 + ((slot - 1 + round) % 31); };
-          int p = 32 * h + pos(kk), q = 32 * h + pos(31 - kk);
-          if (p > q) { const int x = p; p = q; q = x; }
+          int a = 32 * h + pos(kk), b = 32 * h + pos(31 - kk);
+          if (a > b) { const int x = a; a = b; b = x; }
           double c, sn, t;
-          rotation_of(S[p][p], S[q][q], S[p][q], c, sn, t);
-          rot[0][tid] = make_double2(c, sn);
-          rp[tid] = p;
-          rq[tid] = q;
+          rotation_of(S[a][a], S[b][b], S[a][b], c, sn, t);
+          lds.rot[0][tid] = make_double2(c, sn);
+          lds.rp[tid] = a;
+          lds.rq[tid] = b;
         }
         __syncthreads();
-        const double2 r2 = rot[0][k];
-        const int p2 = rp[k], q2 = rq[k];
+        const double2 r2 = lds.rot[0][k];
+        const int p2 = lds.rp[k], q2 = lds.rq[k];
         const double c2 = r2.x, s2 = r2.y;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int k1 = g + 16 * j;
-          const double2 r1 = rot[0][k1];
-          const int p1 = rp[k1], q1 = rq[k1];
+          const double2 r1 = lds.rot[0][k1];
+          const int p1 = lds.rp[k1], q1 = lds.rq[k1];
           const double c1 = r1.x, s1 = r1.y;
           const double xpp = S[p1][p2], xpq = S[p1][q2], xqp = S[q1][p2], xqq = S[q1][q2];
           const double rpp = c1 * xpp - s1 * xqp, rpq = c1 * xpq - s1 * xqq;
@@ -445,50 +486,86 @@ __global__ __launch_bounds__(CROSS_THREADS) void k_jac_solve_x(
         v.ql[j] = Q[4 * g + j][k];
         v.qr[j] = Q[4 * g + j][32 + k];
       }
+      v.ll = S[k][k2];
+      v.rr = S[32 + k][32 + k2];
     }
     // cross rounds: angles of round 0 and the diagonals after it
     if (tid < 32) {
-      const int p = tid, q = 32 + tid;
-      const double app = S[p][p], aqq = S[q][q], apq = S[p][q];
+      const double app = S[tid][tid], aqq = S[32 + tid][32 + tid], apq = S[tid][32 + tid];
       double c, sn, t;
       rotation_of(app, aqq, apq, c, sn, t);
-      rot[0][tid] = make_double2(c, sn);
-      dgl[0][p] = app - t * apq;
-      dgl[0][q] = aqq + t * apq;
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      v.ll[j] = S[k][k ^ (g + 16 * j)];
-      v.rr[j] = S[32 + k][32 + (k ^ (g + 16 * j))];
+      S[tid][32 + tid] = 0.0;
+      lds.rot[0][tid] = make_double2(c, sn);
+      lds.dgl[0][tid] = app - t * apq;
+      lds.dgl[0][32 + tid] = aqq + t * apq;
     }
     __syncthreads();
-    cross_rounds(std::make_integer_sequence<int, 32>{}, S, rot, dgl, k, g, v);
-    // Q's right columns back in order, and S whole again for another sweep
+    cross_rounds(std::make_integer_sequence<int, 32>{}, S, lds.rot, lds.dgl, k, g, v);
+    cross_turn_q(v);
+    // the moving columns back in order, and S whole again for another sweep
     constexpr int SL = cross_sigma(31);
 #pragma unroll
     for (int j = 0; j < 4; ++j) v.qr[j] = __shfl(v.qr[j], (tid & 32) | (k ^ SL), 64);
-    if (sw + 1 < max_inner) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int d = g + 16 * j;
-        S[k][k ^ d] = v.ll[j];
-        S[32 + (k ^ SL)][32 + (k ^ d ^ SL)] = v.rr[j];
-        S[32 + k][k ^ d] = S[k ^ d][32 + k];
-      }
+    // S whole again: the diagonal blocks here, the upper right one is there
+    const int last = 32 + (k ^ SL), last2 = 32 + (k2 ^ SL);
+    S[k][k2] = S[k2][k] = v.ll;
+    S[last][last2] = S[last2][last] = v.rr;
+    if (tid < SB) S[tid][tid] = lds.dgl[1][tid];
+    __syncthreads();
+    if (do_intra && sw + 1 < p.max_inner) {
+      S[32 + k][g] = S[g][32 + k];
+      S[32 + k][16 + g] = S[16 + g][32 + k];
       __syncthreads();
     }
   }
-  // to LDS, then out with consecutive lanes on consecutive rows
+  if (p.di) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = (g + 16 * j) * BS + k;
+      p.di[e] = S[g + 16 * j][k];
+      p.dj[e] = S[32 + g + 16 * j][32 + k];
+    }
+  }
+  if (tid == 0) *p.active = rotated ? 1 : 0;
+  if (!rotated) return;
+  // Q to LDS, then out with consecutive lanes on consecutive rows
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     Q[4 * g + j][k] = v.ql[j];
     Q[4 * g + j][32 + k] = v.qr[j];
   }
   __syncthreads();
-  double* Qo = Qbuf + (size_t)pidx * SB * SB;
 #pragma unroll
-  for (int e = tid; e < SB * SB; e += CROSS_THREADS) Qo[e] = Q[e % SB][e / SB];
-  if (tid == 0) active[pidx] = 1;
+  for (int e = tid; e < SB * SB; e += CROSS_THREADS) p.q[e] = Q[e % SB][e / SB];
+}
+
+// The pair solve on a matrix in memory.
+__global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_solve_x(
+    const double* __restrict__ A, int lda, int nreal, const int* __restrict__ pairs,
+    const int* __restrict__ intra, double* __restrict__ Qbuf, int* __restrict__ active, double* __restrict__ diag,
+    double tol, double skip_abs, int max_inner) {
+  __shared__ JacLds lds;
+  const int pidx = blockIdx.x;
+  const int I = pairs[2 * pidx], J = pairs[2 * pidx + 1];
+  const int tid = threadIdx.x;
+  // all loads of this thread in flight before the first LDS store; A is
+  // symmetric, so column c of it is row c of S
+  constexpr int PER = SB * SB / CROSS_THREADS;
+  double v[PER];
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + CROSS_THREADS * it;
+    v[it] = A[(size_t)gidx_dev(I, J, e % SB) + (size_t)gidx_dev(I, J, e / SB) * lda];
+  }
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + CROSS_THREADS * it;
+    lds.s()[e / SB][e % SB] = v[it];
+  }
+  __syncthreads();
+  pair_solve(lds, I, J, intra[pidx] != 0,
+             JacSolve{nreal, Qbuf + (size_t)pidx * SB * SB, active + pidx, diag ? diag + (size_t)I * BS * BS : nullptr,
+                      diag ? diag + (size_t)J * BS * BS : nullptr, tol, skip_abs, max_inner});
 }
 
 __device__ __forceinline__ int gidx(int pairI, int pairJ, int local) {
@@ -664,103 +741,125 @@ __device__ __forceinline__ void stage_q(double (&v)[SB * SB / UPD_NT], const dou
   }
 }
 
-// MFMA versions of the two update kernels (same data flow as above).
-__global__ __launch_bounds__(UPD_NT) void k_jac_apply_a_mfma(double* __restrict__ A, int lda,
-                                                          int npairs, int npo,
-                                                          const int* __restrict__ pairs,
-                                                          const double* __restrict__ Qbuf,
-                                                          const int* __restrict__ active) {
+// One launch of the cross schedule: step s applied to A and C, and step
+// s + 1's pair problems solved.
+struct JacStep {
+  const double* A;    // before the step
+  double* Ao;         // after it (A itself where the step solves nothing ahead)
+  double* C;
+  int lda, nreal, npairs, npo, ntiles;
+  const int* pairs;   // this step's pairs, rotations and active flags
+  const double* q;
+  const int* act;
+  const int* pairs_n; // the next step's
+  const int* intra_n;
+  const int* where;   // per block: 2 x (its pair in this step) + which half
+  double* qn;
+  int* actn;
+  const double* diag; // per block: its 32 x 32 diagonal block after this step
+  double* diag_n;     // and after the next one
+  double tol, skip_abs;
+  int max_inner;
+};
+
+// Tile (P1 <= P2) of A: Ao(rows of P1, cols of P2) = Q1^T A Q2, and its
+// mirror as the transpose, keeping A exactly symmetric.
+__device__ __forceinline__ void step_tile_a(double* lds, const JacStep& a, int tile) {
   int P1, P2;
-  tile_of(blockIdx.x, npairs, npo, P1, P2);
-  const bool a1 = active[P1] != 0, a2 = active[P2] != 0;
-  if (!a1 && !a2) return;
+  tile_of(tile, a.npairs, a.npo, P1, P2);
+  const bool a1 = a.act[P1] != 0, a2 = a.act[P2] != 0;
+  const int lda = a.lda;
+  if (!a1 && !a2 && a.A == a.Ao) return;
   // two 64 x 65 LDS tiles (66.5 KB) so two workgroups fit on a CU: the tile of
   // A, then Q1^T A, then the result; Q1, then Q2
-  __shared__ double At[SB][LDSW];
-  __shared__ double Qs[SB][LDSW];
-  const int I1 = pairs[2 * P1], J1 = pairs[2 * P1 + 1];
-  const int I2 = pairs[2 * P2], J2 = pairs[2 * P2 + 1];
+  double(*At)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds);
+  double(*Qs)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds + SB * LDSW);
+  const int I1 = a.pairs[2 * P1], J1 = a.pairs[2 * P1 + 1];
+  const int I2 = a.pairs[2 * P2], J2 = a.pairs[2 * P2 + 1];
   const int tid = threadIdx.x;
-  const double* q1 = Qbuf + (size_t)P1 * SB * SB;
-  const double* q2 = Qbuf + (size_t)P2 * SB * SB;
+  const double* q1 = a.q + (size_t)P1 * SB * SB;
+  const double* q2 = a.q + (size_t)P2 * SB * SB;
   // every global load of a stage is issued before the first LDS store, so a
   // thread waits for memory once per stage, not once per element; Q2 is
   // fetched into registers now and lands in LDS after the first product
   constexpr int PER = SB * SB / UPD_NT;  // element e = tid + 512 it: row tid % 64, column tid / 64 + 8 it
-  double va[PER], vq[PER], vq2[PER];
+  double va[PER];
 #pragma unroll
   for (int it = 0; it < PER; ++it) {
     const int e = tid + UPD_NT * it;
-    va[it] = A[(size_t)gidx(I1, J1, e % SB) + (size_t)gidx(I2, J2, e / SB) * lda];
+    va[it] = a.A[(size_t)gidx(I1, J1, e % SB) + (size_t)gidx(I2, J2, e / SB) * lda];
   }
-  stage_q(vq, q1, a1, tid);
-  if (P1 != P2) stage_q(vq2, q2, a2, tid);
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int e = tid + UPD_NT * it;
-    At[e % SB][e / SB] = va[it];
-    Qs[e % SB][e / SB] = vq[it];
-  }
-  __syncthreads();
-  d4_t acc[2];
-  for (int i = 0; i < 2; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
-  mfma_tile64_w8([&](int r, int k) { return Qs[k][r]; }, [&](int k, int c) { return At[k][c]; }, SB, acc);
-  __syncthreads();
-  mfma_tile64_w8_store(acc, [&](int r, int c, double v) { At[r][c] = v; });
-  if (P1 != P2) {
+  if (a1 || a2) {
+    double vq[PER], vq2[PER];
+    stage_q(vq, q1, a1, tid);
+    if (P1 != P2) stage_q(vq2, q2, a2, tid);
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int e = tid + UPD_NT * it;
-      Qs[e % SB][e / SB] = vq2[it];
+      At[e % SB][e / SB] = va[it];
+      Qs[e % SB][e / SB] = vq[it];
+    }
+    __syncthreads();
+    d4_t acc[2];
+    for (int i = 0; i < 2; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return Qs[k][r]; }, [&](int k, int c) { return At[k][c]; }, SB, acc);
+    __syncthreads();
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) { At[r][c] = v; });
+    if (P1 != P2) {
+#pragma unroll
+      for (int it = 0; it < PER; ++it) {
+        const int e = tid + UPD_NT * it;
+        Qs[e % SB][e / SB] = vq2[it];
+      }
+    }
+    __syncthreads();
+    for (int i = 0; i < 2; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return At[r][k]; }, [&](int k, int c) { return Qs[k][c]; }, SB, acc);
+    // stage the result in LDS and write both the tile and its mirror with
+    // consecutive lanes on consecutive rows of A
+    __syncthreads();
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) { At[r][c] = v; });
+  } else {
+    // nothing rotates here: the tile moves to the other buffer as it is
+#pragma unroll
+    for (int it = 0; it < PER; ++it) {
+      const int e = tid + UPD_NT * it;
+      At[e % SB][e / SB] = va[it];
     }
   }
-  __syncthreads();
-  for (int i = 0; i < 2; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
-  mfma_tile64_w8([&](int r, int k) { return At[r][k]; }, [&](int k, int c) { return Qs[k][c]; }, SB, acc);
-  // stage the result in LDS and write both the tile and its mirror with
-  // consecutive lanes on consecutive rows of A
-  __syncthreads();
-  mfma_tile64_w8_store(acc, [&](int r, int c, double v) { At[r][c] = v; });
   __syncthreads();
   if (P1 == P2) {
     for (int e = tid; e < SB * SB; e += UPD_NT) {
       const int r = e % SB, c = e / SB;
       const double v = (r == c) ? At[r][c] : 0.5 * (At[r][c] + At[c][r]);
-      A[(size_t)gidx(I1, J1, r) + (size_t)gidx(I2, J2, c) * lda] = v;
+      a.Ao[(size_t)gidx(I1, J1, r) + (size_t)gidx(I2, J2, c) * lda] = v;
     }
     return;
   }
   for (int e = tid; e < SB * SB; e += UPD_NT) {
     const int r = e % SB, c = e / SB;
-    A[(size_t)gidx(I1, J1, r) + (size_t)gidx(I2, J2, c) * lda] = At[r][c];
+    a.Ao[(size_t)gidx(I1, J1, r) + (size_t)gidx(I2, J2, c) * lda] = At[r][c];
   }
   for (int e = tid; e < SB * SB; e += UPD_NT) {
     const int c = e % SB, r = e / SB;
-    A[(size_t)gidx(I2, J2, c) + (size_t)gidx(I1, J1, r) * lda] = At[r][c];
+    a.Ao[(size_t)gidx(I2, J2, c) + (size_t)gidx(I1, J1, r) * lda] = At[r][c];
   }
 }
 
-__global__ __launch_bounds__(UPD_NT) void k_jac_apply_c_mfma(double* __restrict__ C, int ldc, int nrows,
-                                                          const int* __restrict__ pairs,
-                                                          const double* __restrict__ Qbuf,
-                                                          const int* __restrict__ active) {
-  const int P = blockIdx.y;
-  if (!active[P]) return;
-  __shared__ double Ct[SB][LDSW];
-  __shared__ double Qs[SB][LDSW];
-  const int row0 = blockIdx.x * SB;
-  const int I = pairs[2 * P], J = pairs[2 * P + 1];
-  const double* q = Qbuf + (size_t)P * SB * SB;
-  const int tid = threadIdx.x;
+// C(64 rows from row0, cols of pair P) <- C(...) Q_P
+__device__ __forceinline__ void step_tile_c(double* lds, const JacStep& a, int row0, int P) {
+  if (!a.act[P]) return;
+  double(*Ct)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds);
+  double(*Qs)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds + SB * LDSW);
+  const int I = a.pairs[2 * P], J = a.pairs[2 * P + 1];
+  const double* q = a.q + (size_t)P * SB * SB;
+  const int tid = threadIdx.x, ldc = a.lda;
   constexpr int PER = SB * SB / UPD_NT;
   double vc[PER], vq[PER];
-  {
-    const int gr = row0 + tid % SB;  // the same row for all of this thread's elements
 #pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int e = tid + UPD_NT * it;
-      vc[it] = (gr < nrows) ? C[(size_t)gr + (size_t)gidx(I, J, e / SB) * ldc] : 0.0;
-    }
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + UPD_NT * it;
+    vc[it] = a.C[(size_t)(row0 + e % SB) + (size_t)gidx(I, J, e / SB) * ldc];
   }
   stage_q(vq, q, true, tid);
 #pragma unroll
@@ -779,8 +878,138 @@ __global__ __launch_bounds__(UPD_NT) void k_jac_apply_c_mfma(double* __restrict_
   __syncthreads();
   for (int e = tid; e < SB * SB; e += UPD_NT) {
     const int r = e % SB, c = e / SB;
-    const int gr = row0 + r;
-    if (gr < nrows) C[(size_t)gr + (size_t)gidx(I, J, c) * ldc] = Ct[r][c];
+    a.C[(size_t)(row0 + r) + (size_t)gidx(I, J, c) * ldc] = Ct[r][c];
+  }
+}
+
+// The 32x32 block (X, Y) of A after this step, Qx^T A Qy with the columns of
+// X's and Y's pairs that belong to them, from A before it: 16x16 MFMA blocks,
+// left in the first four waves (rows 16 (w / 2), columns 16 (w % 2) of the
+// result).  A's operand is read from memory in the MFMA layout (16 lanes on
+// consecutive rows); lds is free for the two halves of Q and A Qy.
+__device__ __forceinline__ d4_t next_block(double* lds, const JacStep& a, int X, int Y) {
+  constexpr int LH = BS + 1;
+  double(*Tm)[LH] = reinterpret_cast<double (*)[LH]>(lds);
+  double(*Qx)[LH] = reinterpret_cast<double (*)[LH]>(lds + SB * SB);
+  double(*Qy)[LH] = reinterpret_cast<double (*)[LH]>(lds + SB * SB + SB * LH);
+  const int wx = a.where[X], wy = a.where[Y];
+  const int Px = wx >> 1, hx = wx & 1, Py = wy >> 1, hy = wy & 1;
+  const int Ix = a.pairs[2 * Px], Jx = a.pairs[2 * Px + 1], Iy = a.pairs[2 * Py], Jy = a.pairs[2 * Py + 1];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  double av[16];
+  {
+    const size_t row = gidx(Ix, Jx, 16 * (w >> 1) + li);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) av[i] = a.A[row + (size_t)gidx(Iy, Jy, 4 * i + lk) * a.lda];
+  }
+  constexpr int PER = SB * BS / CROSS_THREADS;
+  double vx[PER], vy[PER];
+  const double* qx = a.q + (size_t)Px * SB * SB + hx * SB * BS;
+  const double* qy = a.q + (size_t)Py * SB * SB + hy * SB * BS;
+  const bool ax = a.act[Px] != 0, ay = a.act[Py] != 0;
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + CROSS_THREADS * it, r = e % SB, c = e / SB;
+    vx[it] = ax ? qx[e] : (r == BS * hx + c ? 1.0 : 0.0);
+    vy[it] = ay ? qy[e] : (r == BS * hy + c ? 1.0 : 0.0);
+  }
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + CROSS_THREADS * it;
+    Qx[e % SB][e / SB] = vx[it];
+    Qy[e % SB][e / SB] = vy[it];
+  }
+  __syncthreads();
+  d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
+  const int cb = 16 * (w & 1);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc = mfma16x16x4(av[i], Qy[4 * i + lk][cb + li], acc);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) Tm[16 * (w >> 1) + lk + 4 * t][cb + li] = acc[t];
+  __syncthreads();
+  acc = d4_t{0.0, 0.0, 0.0, 0.0};
+  if (w < 4) {
+    const int rb = 16 * (w >> 1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc = mfma16x16x4(Qx[4 * i + lk][rb + li], Tm[4 * i + lk][cb + li], acc);
+  }
+  __syncthreads();
+  return acc;
+}
+
+// Pair p of the next step: its 64x64 problem is put together from this
+// step's rotations and A as it is before them, so the solve runs beside the
+// updates of A and C that the same launch makes.  The two diagonal blocks are
+// those the last solve of each block left; at the first step of a sweep they
+// are formed from A as well, so that nothing drifts over the sweeps.
+__device__ __forceinline__ void step_solve(JacLds& lds, const JacStep& a, int p) {
+  const int I = a.pairs_n[2 * p], J = a.pairs_n[2 * p + 1];
+  const bool do_intra = a.intra_n[p] != 0;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  double(*S)[SB] = lds.s();
+  constexpr int PER = BS * BS / CROSS_THREADS;
+  double vi[PER], vj[PER];
+  if (!do_intra) {
+#pragma unroll
+    for (int it = 0; it < PER; ++it) {
+      vi[it] = a.diag[(size_t)I * BS * BS + tid + CROSS_THREADS * it];
+      vj[it] = a.diag[(size_t)J * BS * BS + tid + CROSS_THREADS * it];
+    }
+  }
+  const d4_t lr = next_block(lds.m, a, I, J);
+  const int r0 = 16 * (w >> 1) + (lane >> 4), c0 = 16 * (w & 1) + (lane & 15);
+  if (do_intra) {
+    const d4_t ll = next_block(lds.m, a, I, I);
+    const d4_t rr = next_block(lds.m, a, J, J);
+    if (w < 4) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        S[r0 + 4 * t][c0] = ll[t];
+        S[32 + r0 + 4 * t][32 + c0] = rr[t];
+        S[32 + c0][r0 + 4 * t] = lr[t];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int it = 0; it < PER; ++it) {
+      const int e = tid + CROSS_THREADS * it;
+      S[e / BS][e % BS] = vi[it];
+      S[32 + e / BS][32 + e % BS] = vj[it];
+    }
+  }
+  if (w < 4) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) S[r0 + 4 * t][32 + c0] = lr[t];
+  }
+  __syncthreads();
+  pair_solve(lds, I, J, do_intra,
+             JacSolve{a.nreal, a.qn + (size_t)p * SB * SB, a.actn + p, a.diag_n + (size_t)I * BS * BS,
+                      a.diag_n + (size_t)J * BS * BS, a.tol, a.skip_abs, a.max_inner});
+}
+
+// Workgroups [0, npairs) solve the next step's pairs, the next ntiles update
+// A, the others C.  The solves are the longest and start first; they read A
+// before the step while the update writes the other buffer, so nothing in
+// the launch waits for anything else in it.
+//
+// Solving in a launch of its own left the chip to npairs workgroups for 22
+// of a step's 37 us at 1020 orbitals (with the A update behind it, and the C
+// update on a second stream, ordered by two events per step); this launch
+// takes 24 us, of which the solve's 32 rounds are 12 (each a chain of about
+// 940 cycles: LDS, the block, the next angle, a barrier) and putting its
+// problem together 4.  At 3072 orbitals the updates set it (48 us).
+__global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int base) {
+  static_assert(UPD_NT == CROSS_THREADS, "one workgroup size for every role");
+  __shared__ JacLds lds;
+  const int b = (int)blockIdx.x + base;
+  if (b < a.npairs) {
+    step_solve(lds, a, b);
+  } else if (b < a.npairs + a.ntiles) {
+    step_tile_a(lds.m, a, b - a.npairs);
+  } else {
+    const int c = b - a.npairs - a.ntiles, nrow = a.lda / SB;
+    step_tile_c(lds.m, a, (c % nrow) * SB, c / nrow);
   }
 }
 
@@ -924,9 +1153,6 @@ __global__ __launch_bounds__(256) void k_phase_lock(int n, double* __restrict__ 
 int g_jacobi_schedule = 1;
 
 void JacobiPlan::build(int n_in, int split) {
-  // buffers below may be re-allocated: no C update of an earlier solve may
-  // still be reading them
-  if (cstream) MHIP_CHECK(hipStreamSynchronize(cstream));
   n = n_in;
   npad = ((n + SB - 1) / SB) * SB;
   nb = npad / BS;
@@ -977,21 +1203,21 @@ void JacobiPlan::build(int n_in, int split) {
   intra_host = fl;
   intra.ensure(fl.size() * sizeof(int));
   MHIP_CHECK(hipMemcpy(intra.ptr, fl.data(), fl.size() * sizeof(int), hipMemcpyHostToDevice));
-  qbuf.ensure((size_t)nsteps * npairs * SB * SB * sizeof(double));
+  // where each block is in each step
+  std::vector<int> wh((size_t)nsteps * nb, 0);
+  for (int step = 0; step < nsteps; ++step)
+    for (int k = 0; k < npairs; ++k)
+      for (int half = 0; half < 2; ++half)
+        wh[(size_t)step * nb + h[((size_t)step * npairs + k) * 2 + half]] = 2 * k + half;
+  where.ensure(wh.size() * sizeof(int));
+  MHIP_CHECK(hipMemcpy(where.ptr, wh.data(), wh.size() * sizeof(int), hipMemcpyHostToDevice));
+  // rotations, flags and diagonal blocks of two consecutive steps
+  qbuf.ensure((size_t)2 * npairs * SB * SB * sizeof(double));
+  diag.ensure((size_t)2 * nb * BS * BS * sizeof(double));
+  active.ensure((size_t)2 * npairs * sizeof(int));
   part.ensure((size_t)2 * npad * sizeof(double) + 64);
   perm.ensure((size_t)npad * sizeof(int));
-  active.ensure((size_t)nsteps * npairs * sizeof(int));
-  if (!cstream) MHIP_CHECK(hipStreamCreateWithFlags(&cstream, hipStreamNonBlocking));
-  if (!ev_join) MHIP_CHECK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-  while ((int)ev_solved.size() < nsteps) {
-    hipEvent_t a, b;
-    MHIP_CHECK(hipEventCreateWithFlags(&a, hipEventDisableTiming));
-    MHIP_CHECK(hipEventCreateWithFlags(&b, hipEventDisableTiming));
-    ev_solved.push_back(a);
-    ev_cdone.push_back(b);
-  }
-  cdone_pending.assign(ev_cdone.size(), 0);
-  counts.ensure((size_t)2 * nb * sizeof(int));
+  counts.ensure((size_t)2 * nsteps * sizeof(int));
 }
 
 void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc) {
@@ -999,25 +1225,36 @@ void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc) {
   MHIP_LAUNCH_CHECK();
 }
 
-int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double tol, int max_sweeps,
+int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
                   double* host_scal, double* dev_scal, int* sweeps_done) {
   const int lda = plan.npad;
   int done = 0;
-  hipStream_t cs = plan.cstream;
   // Inner sweeps per step.  Cross schedule: one; a second saves up to a fifth
   // of the sweeps (54 instead of 66 in the plain SCF of 1020 orbitals) for
-  // twice the rounds (109 ms instead of 102; 16.6 instead of 15.2 ms at 174
+  // twice the rounds (72 ms instead of 58; 12.1 instead of 9.7 ms at 174
   // orbitals).  A matrix that is one pair problem is solved in one launch.
   const bool cross = g_jacobi_schedule == 1;
   const int inner = plan.max_inner > 0 ? plan.max_inner : !cross ? 2 : plan.npairs == 1 ? 16 : 1;
   const double inner_tol = plan.npairs == 1 ? 0.5 * tol : 1.0e-14;
-  // the C updates start after whatever the caller queued on C
-  MHIP_CHECK(hipEventRecord(plan.ev_join, s));
-  MHIP_CHECK(hipStreamWaitEvent(cs, plan.ev_join, 0));
-  // and the caller's later work on C waits for the last of them
-  auto join = [&] {
-    MHIP_CHECK(hipEventRecord(plan.ev_join, cs));
-    MHIP_CHECK(hipStreamWaitEvent(s, plan.ev_join, 0));
+  // every step's solves ride in the launch of the step before
+  const bool ahead = cross && g_kernel_variant == 1 && plan.npairs > 1;
+  const int npairs = plan.npairs, npv = npairs - plan.npo, nsteps = plan.nsteps;
+  const int ntiles = plan.npo * (plan.npo + 1) / 2 + npv * (npv + 1) / 2, nctiles = npairs * (plan.npad / SB);
+  int slot = 0;  // of the step at hand in the two-step buffers
+  auto qslot = [&](int k) { return plan.qbuf.as<double>() + (size_t)k * npairs * SB * SB; };
+  auto aslot = [&](int k) { return plan.active.as<int>() + (size_t)k * npairs; };
+  auto dslot = [&](int k) { return plan.diag.as<double>() + (size_t)k * plan.nb * BS * BS; };
+  auto pairs_of = [&](int step) { return plan.pairs.as<int>() + (size_t)step * npairs * 2; };
+  auto intra_of = [&](int step) { return plan.intra.as<int>() + (size_t)step * npairs; };
+  auto solve = [&](int step, double skip_abs) {
+    if (cross)
+      hipLaunchKernelGGL(k_jac_solve_x, dim3(npairs), dim3(CROSS_THREADS), 0, s, A, lda, plan.n, pairs_of(step),
+                         intra_of(step), qslot(slot), aslot(slot), ahead ? dslot(slot) : nullptr, inner_tol, skip_abs,
+                         inner);
+    else
+      hipLaunchKernelGGL(k_jac_solve, dim3(npairs), dim3(SOLVE_THREADS), 0, s, A, lda, plan.n, pairs_of(step),
+                         qslot(slot), aslot(slot), 1.0e-14, skip_abs, inner);
+    MHIP_LAUNCH_CHECK();
   };
   for (int sw = 0; sw <= max_sweeps; ++sw) {
     hipLaunchKernelGGL(k_offmax_partial, dim3(plan.n), dim3(256), 0, s, plan.n, A, lda,
@@ -1033,69 +1270,73 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
     // pairs whose whole 64x64 block is already this diagonal are left alone
     const double skip_abs = 0.1 * thr;
     if (sw == max_sweeps) {
-      join();
       if (sweeps_done) *sweeps_done = done;
       return 1;
     }
-    const int nsteps = plan.nsteps;
     if (plan.timing && plan.ev.size() < (size_t)(6 * nsteps)) {
       for (auto e : plan.ev) (void)hipEventDestroy(e);
       plan.ev.assign(6 * nsteps, nullptr);
       for (auto& e : plan.ev) MHIP_CHECK(hipEventCreate(&e));
     }
-    const int npv = plan.npairs - plan.npo;
-    const int ntiles = plan.npo * (plan.npo + 1) / 2 + npv * (npv + 1) / 2;
+    const bool timing = plan.timing && g_kernel_variant == 1;
+    // part k of the step's launch between events 2 k and 2 k + 1
+    auto mark = [&](int step, int k) {
+      if (timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + k], s));
+    };
+    // the first step's solve of a later sweep ran in the last launch of the
+    // sweep before
+    if (ahead && sw == 0) solve(0, skip_abs);
     for (int step = 0; step < nsteps; ++step) {
-      const int* pr = plan.pairs.as<int>() + (size_t)step * plan.npairs * 2;
-      double* q = plan.qbuf.as<double>() + (size_t)step * plan.npairs * SB * SB;
-      int* act = plan.active.as<int>() + (size_t)step * plan.npairs;
-      // the slot's previous C update (one sweep earlier) must have read it
-      if (plan.cdone_pending[step]) MHIP_CHECK(hipStreamWaitEvent(s, plan.ev_cdone[step], 0));
-      if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 0], s));
-      if (g_jacobi_schedule == 1) {
-        const int* fl = plan.intra.as<int>() + (size_t)step * plan.npairs;
-        hipLaunchKernelGGL(k_jac_solve_x, dim3(plan.npairs), dim3(CROSS_THREADS), 0, s, A, lda, plan.n, pr, fl,
-                           q, act, inner_tol, skip_abs, inner);
-      } else {
-        hipLaunchKernelGGL(k_jac_solve, dim3(plan.npairs), dim3(SOLVE_THREADS), 0, s, A, lda, plan.n, pr, q,
-                           act, 1.0e-14, skip_abs, inner);
+      if (!ahead) {
+        mark(step, 0);
+        solve(step, skip_abs);
+        mark(step, 1);
       }
-      MHIP_LAUNCH_CHECK();
-      if (plan.timing) {
-        MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 1], s));
-        hipLaunchKernelGGL(k_count_active, dim3(1), dim3(64), 0, s, plan.npairs, plan.npo, act,
+      if (timing)
+        hipLaunchKernelGGL(k_count_active, dim3(1), dim3(64), 0, s, npairs, plan.npo, aslot(slot),
                            plan.counts.as<int>() + 2 * step);
-      }
       if (g_kernel_variant == 1) {
-        if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 2], s));
-        hipLaunchKernelGGL(k_jac_apply_a_mfma, dim3(ntiles), dim3(UPD_NT), 0, s, A, lda, plan.npairs, plan.npo, pr, q,
-                           act);
-        MHIP_LAUNCH_CHECK();
-        if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 3], s));
-        // C <- C Q on the side stream once this step's A update is done, so
-        // it overlaps the next step's pair solves, which leave most CUs idle
-        MHIP_CHECK(hipEventRecord(plan.ev_solved[step], s));
-        MHIP_CHECK(hipStreamWaitEvent(cs, plan.ev_solved[step], 0));
-        if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 4], cs));
-        hipLaunchKernelGGL(k_jac_apply_c_mfma, dim3(plan.npad / SB, plan.npairs), dim3(UPD_NT), 0, cs, C, lda,
-                           plan.npad, pr, q, act);
-        MHIP_LAUNCH_CHECK();
-        if (plan.timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + 5], cs));
+        const int next = (step + 1) % nsteps, first = ahead ? 0 : npairs, total = npairs + ntiles + nctiles;
+        const JacStep a{A,          ahead ? A2 : A,  C,                lda,
+                        plan.n,     npairs,          plan.npo,         ntiles,
+                        pairs_of(step), qslot(slot), aslot(slot),      pairs_of(next),
+                        intra_of(next), plan.where.as<int>() + (size_t)step * plan.nb, qslot(slot ^ 1), aslot(slot ^ 1),
+                        dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
+                        inner};
+        auto launch = [&](int from, int to) {
+          hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), 0, s, a, from);
+          MHIP_LAUNCH_CHECK();
+        };
+        if (!timing) {
+          launch(first, total);
+        } else {
+          // the same work in a launch per part, for the parts' times
+          if (ahead) {
+            mark(step, 0);
+            launch(0, npairs);
+            mark(step, 1);
+          }
+          mark(step, 2);
+          launch(npairs, npairs + ntiles);
+          mark(step, 3);
+          mark(step, 4);
+          launch(npairs + ntiles, total);
+          mark(step, 5);
+        }
+        if (ahead) {
+          std::swap(A, A2);
+          slot ^= 1;
+        }
       } else {
-        hipLaunchKernelGGL(k_jac_apply_a, dim3(ntiles), dim3(256), 0, s, A, lda, plan.npairs, plan.npo, pr, q,
-                           act);
+        hipLaunchKernelGGL(k_jac_apply_a, dim3(ntiles), dim3(256), 0, s, A, lda, npairs, plan.npo, pairs_of(step),
+                           qslot(slot), aslot(slot));
         MHIP_LAUNCH_CHECK();
-        MHIP_CHECK(hipEventRecord(plan.ev_solved[step], s));
-        MHIP_CHECK(hipStreamWaitEvent(cs, plan.ev_solved[step], 0));
-        hipLaunchKernelGGL(k_jac_apply_c, dim3(plan.npad / SB, plan.npairs), dim3(256), 0, cs, C, lda,
-                           plan.npad, pr, q, act);
+        hipLaunchKernelGGL(k_jac_apply_c, dim3(plan.npad / SB, npairs), dim3(256), 0, s, C, lda, plan.npad,
+                           pairs_of(step), qslot(slot), aslot(slot));
         MHIP_LAUNCH_CHECK();
       }
-      MHIP_CHECK(hipEventRecord(plan.ev_cdone[step], cs));
-      plan.cdone_pending[step] = 1;
     }
-    if (plan.timing && g_kernel_variant == 1) {
-      MHIP_CHECK(hipStreamSynchronize(cs));
+    if (timing) {
       MHIP_CHECK(hipStreamSynchronize(s));
       std::vector<int> act(2 * nsteps);
       MHIP_CHECK(hipMemcpy(act.data(), plan.counts.ptr, sizeof(int) * 2 * nsteps, hipMemcpyDeviceToHost));
@@ -1107,21 +1348,18 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
         // plus 2 x 496 inside the blocks where the step's intra flag is set
         for (int g = 0; g < 2; ++g) {
           const int first = g == 0 ? 0 : plan.npo;
-          if (first >= plan.npairs) continue;
+          if (first >= npairs) continue;
           const long long per =
-              g_jacobi_schedule == 1
-                  ? 1024 + (plan.intra_host[(size_t)step * plan.npairs + first] ? 992 : 0)
-                  : 2016LL * inner;
+              cross ? 1024 + (plan.intra_host[(size_t)step * npairs + first] ? 992 : 0) : 2016LL * inner;
           plan.active_rotations += per * act[2 * step + g];
         }
         plan.active_tiles += (long long)ntiles - u0 * (u0 + 1) / 2 - u1 * (u1 + 1) / 2;
-        float a = 0.f, b = 0.f, c2 = 0.f;
-        MHIP_CHECK(hipEventElapsedTime(&a, plan.ev[6 * step + 0], plan.ev[6 * step + 1]));
-        MHIP_CHECK(hipEventElapsedTime(&b, plan.ev[6 * step + 2], plan.ev[6 * step + 3]));
-        MHIP_CHECK(hipEventElapsedTime(&c2, plan.ev[6 * step + 4], plan.ev[6 * step + 5]));
-        plan.t_solve_ms += a;
-        plan.t_apply_ms += b;
-        plan.t_applyc_ms += c2;
+        float t[3];
+        for (int k = 0; k < 3; ++k)
+          MHIP_CHECK(hipEventElapsedTime(&t[k], plan.ev[6 * step + 2 * k], plan.ev[6 * step + 2 * k + 1]));
+        plan.t_solve_ms += t[0];
+        plan.t_apply_ms += t[1];
+        plan.t_applyc_ms += t[2];
         plan.n_solve++;
         plan.n_apply++;
         plan.n_applyc++;
@@ -1129,7 +1367,6 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double* A, double* C, double 
     }
     ++done;
   }
-  join();
   if (sweeps_done) *sweeps_done = done;
   return 0;
 }

@@ -263,7 +263,8 @@ static void eigen_packed(mhip_ctx* c, double* fpacked, bool perturb, double tol 
     jacobi_set_identity(s, np, C, np);
   }
   int sweeps = 0;
-  const int rc = jacobi_sweeps(s, plan, A, C, tol, 40, c->hscal + 32,
+  double* A2 = c->T.as<double>();
+  const int rc = jacobi_sweeps(s, plan, A, A2, C, tol, 40, c->hscal + 32,
                                c->scal.as<double>() + 32, &sweeps);
   MHIP_REQUIRE(rc == 0, "block-Jacobi eigensolver did not converge in 40 sweeps");
   c->last_sweeps = sweeps;
