@@ -6,6 +6,11 @@
 // Y = Z (last).  Master weights stay FP32; the BF16 copies are refreshed after
 // every optimizer step.  Backward treats the BF16 rounding of activations as
 // the identity (straight-through), the usual mixed-precision convention.
+//
+// Every product runs on the BF16 matrix cores.  The forward operands are BF16
+// already.  The backward's FP32 operand dZ goes in as three BF16 parts that
+// add up to it exactly (8 significand bits each, by truncation), the leading
+// part and the two others summed separately in FP32, so no bit of it is lost.
 #include <vector>
 
 #include "common.h"
@@ -20,63 +25,295 @@ __device__ __forceinline__ unsigned short f2bf(float x) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return (unsigned short)(u >> 16);
 }
-__device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(((unsigned)h) << 16); }
 
-constexpr int T = 32;  // tile edge
+// x = p[0] + p[1] + p[2] in BF16, exactly (down to the smallest normal
+// numbers); an infinity or NaN stays in p[0]
+__device__ __forceinline__ void split3(float x, unsigned short p[3]) {
+  const unsigned u = __float_as_uint(x);
+  p[0] = (unsigned short)(u >> 16);
+  if ((u & 0x7f800000u) == 0x7f800000u) {
+    p[1] = p[2] = 0;
+    return;
+  }
+  const float r1 = x - __uint_as_float(u & 0xffff0000u);
+  const unsigned u1 = __float_as_uint(r1);
+  p[1] = (unsigned short)(u1 >> 16);
+  p[2] = (unsigned short)(__float_as_uint(r1 - __uint_as_float(u1 & 0xffff0000u)) >> 16);
+}
 
-// C[M x N] = op(A) * op(B) (+bias), FP32 accumulate.  A, B either BF16
-// (unsigned short) or FP32.  ta/tb select transposes of row-major storage:
-//   A row-major M x K (ta = 0) or K x M (ta = 1); B row-major K x N or N x K.
-template <class TA_, class TB_, bool TRA, bool TRB>
-__global__ __launch_bounds__(256) void k_mm(int M, int N, int K, const TA_* __restrict__ A,
-                                            const TB_* __restrict__ B, const float* __restrict__ bias,
-                                            float* __restrict__ C, int act, float beta) {
-  __shared__ float As[T][T + 1];
-  __shared__ float Bs[T][T + 1];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-  const int row0 = blockIdx.y * T, col0 = blockIdx.x * T;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  auto lda = [&](int m, int k) -> float {
-    if (m >= M || k >= K) return 0.f;
-    size_t idx = TRA ? (size_t)k * M + m : (size_t)m * K + k;
-    if constexpr (sizeof(TA_) == 2) return bf2f(A[idx]);
-    else return (float)A[idx];
-  };
-  auto ldb = [&](int k, int n) -> float {
-    if (k >= K || n >= N) return 0.f;
-    size_t idx = TRB ? (size_t)n * K + k : (size_t)k * N + n;
-    if constexpr (sizeof(TB_) == 2) return bf2f(B[idx]);
-    else return (float)B[idx];
-  };
-  for (int k0 = 0; k0 < K; k0 += T) {
-    for (int r = ty; r < T; r += 8) {
-      As[r][tx] = lda(row0 + r, k0 + tx);
-      Bs[r][tx] = ldb(k0 + r, col0 + tx);
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int kk = 0; kk < T; ++kk) {
-      const float b = Bs[kk][tx];
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+// v_mfma_f32_16x16x32_bf16: lane l gives A[l % 16][8 (l / 16) ..+7] and
+// B[8 (l / 16) ..+7][l % 16] and holds D[4 (l / 16) + t][l % 16].
+__device__ __forceinline__ f4_t mma(bf8_t a, bf8_t b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+constexpr int MLP_NT = 256;
+constexpr int MLP_BN = 256;  // output columns per workgroup: 64 per wave
+
+// C[M x N] = A[M x K] * B (+ epilogue), A row-major FP32, B given as BF16 rows
+// per output column, Kp long (K padded to 32 with zeros).  A tile of A is
+// converted once into LDS (PARTS = 1: rounded to BF16; 3: split exactly), B
+// is read from L2 in the operand layout.  One workgroup has BM rows and up to
+// 256 columns, so A is read from memory once.
+//   forward  (PARTS 1): C = act(A B + bias), act 1 = tanh
+//   backward (PARTS 3): C = A B (1 - act_in^2), act_in the tanh outputs
+// Bound by the FP32 activations it reads and writes: 28 us a layer on average
+// for 30000 rows of 168-256-256-256-16 (61 MB through memory for a 256 x 256
+// layer); FP32 vector tiles of 32x32, with a conversion pass before each
+// product, took 140 us.
+template <int BM, int PARTS>
+__global__ __launch_bounds__(MLP_NT) void k_layer(int M, int N, int K, int Kp, const float* __restrict__ A,
+                                                  const unsigned short* __restrict__ B,
+                                                  const float* __restrict__ bias, int act,
+                                                  const float* __restrict__ act_in, float* __restrict__ C) {
+  constexpr int KC = PARTS == 1 ? 256 : 128, LD = KC + 8;
+  __shared__ __align__(16) unsigned short as[PARTS][BM][LD];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * MLP_BN + 64 * w;
+  const bool vec = (K & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
+  f4_t big[BM / 16][4], corr[BM / 16][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = fmaf(As[ty + 8 * i][kk], b, acc[i]);
+  for (int i = 0; i < BM / 16; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) big[i][j] = corr[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  for (int kc = 0; kc < Kp; kc += KC) {
+    const int kk = min(KC, Kp - kc), quads = BM * (kk >> 2);
+    if (kc) __syncthreads();
+    constexpr int QPT = BM * KC / 4 / MLP_NT;
+    float4 v[QPT];
+#pragma unroll
+    for (int q = 0; q < QPT; ++q) {
+      const int idx = tid + MLP_NT * q;
+      v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (idx < quads) {
+        const int r = m0 + idx / (kk >> 2), k = kc + 4 * (idx % (kk >> 2));
+        if (r < M) {
+          const float* src = A + (size_t)r * K + k;
+          if (vec) {
+            if (k < K) v[q] = *reinterpret_cast<const float4*>(src);
+          } else {
+            if (k < K) v[q].x = src[0];
+            if (k + 1 < K) v[q].y = src[1];
+            if (k + 2 < K) v[q].z = src[2];
+            if (k + 3 < K) v[q].w = src[3];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < QPT; ++q) {
+      const int idx = tid + MLP_NT * q;
+      if (idx >= quads) continue;
+      const int r = idx / (kk >> 2), k = 4 * (idx % (kk >> 2));
+      const float x[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+      unsigned short p[4][3];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (PARTS == 1) p[t][0] = f2bf(x[t]);
+        else split3(x[t], p[t]);
+      }
+#pragma unroll
+      for (int pl = 0; pl < PARTS; ++pl)
+        *reinterpret_cast<ushort4*>(&as[pl][r][k]) = make_ushort4(p[0][pl], p[1][pl], p[2][pl], p[3][pl]);
     }
     __syncthreads();
+    if (n0 >= N) continue;
+    for (int k = 0; k < kk; k += 32) {
+      bf8_t b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int n = n0 + 16 * j + li;
+        b[j] = n < N ? *reinterpret_cast<const bf8_t*>(B + (size_t)n * Kp + kc + k + 8 * lg) : bf8_t{};
+      }
+#pragma unroll
+      for (int i = 0; i < BM / 16; ++i) {
+        bf8_t a[PARTS];
+#pragma unroll
+        for (int pl = 0; pl < PARTS; ++pl)
+          a[pl] = *reinterpret_cast<const bf8_t*>(&as[pl][16 * i + li][k + 8 * lg]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (PARTS == 3) {
+            corr[i][j] = mma(a[2], b[j], corr[i][j]);
+            corr[i][j] = mma(a[1], b[j], corr[i][j]);
+          }
+          big[i][j] = mma(a[0], b[j], big[i][j]);
+        }
+      }
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = row0 + ty + 8 * i, c = col0 + tx;
-    if (r >= M || c >= N) continue;
-    float v = acc[i] + (bias ? bias[c] : 0.f);
-    if (act == 1) v = tanhf(v);
-    float* dst = C + (size_t)r * N + c;
-    *dst = (beta == 0.f) ? v : v + beta * *dst;
+  for (int j = 0; j < 4; ++j) {
+    const int n = n0 + 16 * j + li;
+    if (n >= N) continue;
+    const float bn = bias ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < BM / 16; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = m0 + 16 * i + 4 * lg + t;
+        if (r >= M) continue;
+        const size_t at = (size_t)r * N + n;
+        if constexpr (PARTS == 1) {
+          const float z = big[i][j][t] + bn;
+          C[at] = act == 1 ? tanhf(z) : z;
+        } else {
+          const float x = act_in[at];
+          C[at] = (big[i][j][t] + corr[i][j][t]) * (1.f - x * x);
+        }
+      }
   }
 }
 
-__global__ void k_to_bf16(long long n, const float* __restrict__ x, unsigned short* __restrict__ y) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    y[i] = f2bf(x[i]);
+// One layer of the network, in the flat parameter vector and in the padded
+// BF16 copies: wt has out rows of inp (in padded to 32), wp in rows of outp.
+struct LayerDev {
+  int in, out, inp, outp;
+  long long woff, boff, wt, wp;
+  long long pre;  // sum of the widths before the layer's input
+  int tile0;      // first 64x64 tile of the layer in k_dw's grid
+};
+
+__device__ __forceinline__ const LayerDev& layer_of_tile(const LayerDev* __restrict__ L, int nl, int tile) {
+  int l = 0;
+  while (l + 1 < nl && tile >= L[l + 1].tile0) ++l;
+  return L[l];
+}
+
+// Every layer's dW = bf16(X)^T dZ and db = column sums of dZ, in one launch:
+// a workgroup has a 64x64 tile of one layer's dW and a slice of the batch
+// (blockIdx.y), whose part goes to part[slice] in the parameter layout.  X
+// and dZ are transposed on their way into LDS (a thread packs eight batch
+// rows of one column into 16 bytes), dZ in its three exact parts.
+// The matrix of a layer alone fills a few dozen workgroups, each over the
+// whole batch (171 us a layer at a batch of 2048, and 364 us for the column
+// sums of one thread per column); the slices fill the chip: 13 us for the
+// four layers of 96-256-256-256-16.
+__global__ __launch_bounds__(MLP_NT) void k_dw(int nl, const LayerDev* __restrict__ L, int batch, int rows,
+                                               const float* __restrict__ acts, const float* __restrict__ dz,
+                                               long long np, float* __restrict__ part) {
+  constexpr int LD = 40;
+  __shared__ __align__(16) unsigned short xs[64][LD], zs[3][64][LD];
+  __shared__ float red[4][64];
+  const LayerDev& y = layer_of_tile(L, nl, blockIdx.x);
+  const int tile = blockIdx.x - y.tile0, nj = (y.out + 63) / 64;
+  const int i0 = 64 * (tile / nj), j0 = 64 * (tile % nj);
+  const int in = y.in, out = y.out;
+  const float* X = acts + (size_t)batch * y.pre;
+  const float* Z = dz + (size_t)batch * (y.pre + in);
+  const int b0 = blockIdx.y * rows, b1 = min(batch, b0 + rows);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int wm = 32 * (w >> 1), wn = 32 * (w & 1);
+  const bool xi = i0 + lane < in, zj = j0 + lane < out;
+  f4_t big[2][2], corr[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) big[i][j] = corr[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  float sum = 0.f, xv[8], zv[8];
+  auto load = [&](int b) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int row = b + 8 * w + r;
+      xv[r] = xi && row < b1 ? X[(size_t)row * in + i0 + lane] : 0.f;
+      zv[r] = zj && row < b1 ? Z[(size_t)row * out + j0 + lane] : 0.f;
+    }
+  };
+  load(b0);
+  for (int b = b0; b < b1; b += 32) {
+    {
+      union { unsigned short h[8]; uint4 q; } x, z[3];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        x.h[r] = f2bf(xv[r]);
+        unsigned short p[3];
+        split3(zv[r], p);
+        z[0].h[r] = p[0];
+        z[1].h[r] = p[1];
+        z[2].h[r] = p[2];
+        sum += zv[r];
+      }
+      *reinterpret_cast<uint4*>(&xs[lane][8 * w]) = x.q;
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint4*>(&zs[pl][lane][8 * w]) = z[pl].q;
+    }
+    __syncthreads();
+    if (b + 32 < b1) load(b + 32);
+    bf8_t a[2], bz[2][3];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf8_t*>(&xs[wm + 16 * i + li][8 * lg]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl)
+        bz[j][pl] = *reinterpret_cast<const bf8_t*>(&zs[pl][wn + 16 * j + li][8 * lg]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        corr[i][j] = mma(a[i], bz[j][2], corr[i][j]);
+        corr[i][j] = mma(a[i], bz[j][1], corr[i][j]);
+        big[i][j] = mma(a[i], bz[j][0], big[i][j]);
+      }
+    __syncthreads();
+  }
+  float* o = part + (size_t)blockIdx.y * np;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = i0 + wm + 16 * i + 4 * lg + t, c = j0 + wn + 16 * j + li;
+        if (r < in && c < out) o[y.woff + (long long)r * out + c] = big[i][j][t] + corr[i][j][t];
+      }
+  if (i0 == 0) {
+    red[w][lane] = sum;
+    __syncthreads();
+    if (w == 0 && zj) o[y.boff + j0 + lane] = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+  }
+}
+
+// grad = sum of the batch slices' parts, in slice order; the first workgroup
+// also sums the loss's parts
+__global__ __launch_bounds__(256) void k_grad_sum(long long np, int slices, const float* __restrict__ part,
+                                                  float* __restrict__ grad, int nloss,
+                                                  const float* __restrict__ lpart, float scale,
+                                                  float* __restrict__ loss) {
+  const long long i = blockIdx.x * 256LL + threadIdx.x;
+  if (i < np) {
+    float s = 0.f;
+    for (int k = 0; k < slices; ++k) s += part[(size_t)k * np + i];
+    grad[i] = s;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    double s = 0.0;
+    for (int k = threadIdx.x; k < nloss; k += 64) s += lpart[k];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (threadIdx.x == 0) *loss = (float)(s * scale);
+  }
+}
+
+// both BF16 copies of every weight
+__global__ __launch_bounds__(256) void k_refresh(int nl, const LayerDev* __restrict__ L,
+                                                 const float* __restrict__ w, unsigned short* __restrict__ bf) {
+  const LayerDev y = L[blockIdx.y];
+  const long long len = (long long)y.in * y.out;
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < len; i += (long long)gridDim.x * 256) {
+    const int r = (int)(i / y.out), c = (int)(i % y.out);
+    const unsigned short h = f2bf(w[y.woff + i]);
+    bf[y.wt + (long long)c * y.inp + r] = h;
+    bf[y.wp + (long long)r * y.outp + c] = h;
+  }
+}
+
+__global__ void k_zero_u16(long long n, unsigned short* __restrict__ p) {
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += (long long)gridDim.x * 256) p[i] = 0;
 }
 
 // dY = (Y - T) * 2 / (B * nout); partial loss sums per block
@@ -97,32 +334,6 @@ __global__ __launch_bounds__(256) void k_mse(long long n, float scale, const flo
     __syncthreads();
   }
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-__global__ void k_sum_f(int n, const float* __restrict__ part, float scale, float* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    *out = (float)(s * scale);
-  }
-}
-
-// dZ = dX_next * (1 - tanh^2) where X_next = tanh(Z) is stored
-__global__ void k_tanh_back(long long n, const float* __restrict__ xn, float* __restrict__ d) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float a = xn[i];
-    d[i] *= (1.f - a * a);
-  }
-}
-
-// db[c] = sum_r dZ[r][c]
-__global__ void k_colsum(int rows, int cols, const float* __restrict__ dz, float* __restrict__ db) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += dz[(size_t)r * cols + c];
-  db[c] = s;
 }
 
 __global__ void k_adam(long long n, float* __restrict__ w, const float* __restrict__ g,
@@ -149,13 +360,15 @@ using namespace mhip;
 struct mhip_mlp {
   int nl = 0;
   std::vector<int> dims;
-  std::vector<size_t> woff, boff;  // offsets into the flat parameter vector
+  std::vector<LayerDev> lay;
+  int ntiles = 0;  // 64x64 tiles of all weight matrices
   size_t np = 0;
   hipStream_t s = nullptr;
-  DevBuf w32, wbf, grad, m, v;
-  DevBuf acts;  // X_0..X_nl (FP32) for the current batch
-  DevBuf xbf;   // BF16 copy of a layer input
-  DevBuf dbuf0, dbuf1, tgt, part, loss;
+  DevBuf w32, wbf, grad, m, v, layers;
+  DevBuf acts;   // X_0..X_nl (FP32) for the current batch
+  DevBuf dz;     // the gradients by the layers' outputs, laid out as acts
+  DevBuf gpart;  // the batch slices' parts of the gradient
+  DevBuf tgt, part, loss;
   int batch_cap = 0;
   long long step = 0;
 };
@@ -164,15 +377,9 @@ namespace {
 
 void mlp_ensure_batch(mhip_mlp* q, int batch) {
   if (batch <= q->batch_cap) return;
-  size_t tot = 0, mx = 0;
-  for (int l = 0; l <= q->nl; ++l) {
-    tot += (size_t)batch * q->dims[l];
-    mx = std::max(mx, (size_t)q->dims[l]);
-  }
+  size_t tot = 0;
+  for (int l = 0; l <= q->nl; ++l) tot += (size_t)batch * q->dims[l];
   q->acts.ensure(sizeof(float) * tot);
-  q->xbf.ensure(sizeof(unsigned short) * (size_t)batch * mx);
-  q->dbuf0.ensure(sizeof(float) * (size_t)batch * mx);
-  q->dbuf1.ensure(sizeof(float) * (size_t)batch * mx);
   q->tgt.ensure(sizeof(float) * (size_t)batch * q->dims[q->nl]);
   q->part.ensure(sizeof(float) * 1024);
   q->loss.ensure(sizeof(float) * 4);
@@ -186,25 +393,30 @@ float* act_ptr(mhip_mlp* q, int batch, int l) {
 }
 
 void refresh_bf16(mhip_mlp* q) {
-  hipLaunchKernelGGL(k_to_bf16, dim3(std::min(4096, cdiv(q->np, 256))), dim3(256), 0, q->s,
-                     (long long)q->np, q->w32.as<float>(), q->wbf.as<unsigned short>());
+  hipLaunchKernelGGL(k_refresh, dim3(128, q->nl), dim3(256), 0, q->s, q->nl, q->layers.as<LayerDev>(),
+                     q->w32.as<float>(), q->wbf.as<unsigned short>());
+  MHIP_LAUNCH_CHECK();
+}
+
+// rows per workgroup: 32 where that fills the chip twice over, else 16
+template <int PARTS>
+void layer(mhip_mlp* q, int M, int N, int K, int Kp, const float* A, const unsigned short* B, const float* bias,
+           int act, const float* act_in, float* C) {
+  const int ny = cdiv(N, MLP_BN);
+  if (cdiv(M, 32) * ny >= 512)
+    hipLaunchKernelGGL((k_layer<32, PARTS>), dim3(cdiv(M, 32), ny), dim3(MLP_NT), 0, q->s, M, N, K, Kp, A, B, bias,
+                       act, act_in, C);
+  else
+    hipLaunchKernelGGL((k_layer<16, PARTS>), dim3(cdiv(M, 16), ny), dim3(MLP_NT), 0, q->s, M, N, K, Kp, A, B, bias,
+                       act, act_in, C);
   MHIP_LAUNCH_CHECK();
 }
 
 void forward(mhip_mlp* q, int batch) {
   for (int l = 0; l < q->nl; ++l) {
-    const int in = q->dims[l], out = q->dims[l + 1];
-    float* X = act_ptr(q, batch, l);
-    float* Y = act_ptr(q, batch, l + 1);
-    hipLaunchKernelGGL(k_to_bf16, dim3(std::min(4096, cdiv((long long)batch * in, 256))), dim3(256), 0,
-                       q->s, (long long)batch * in, X, q->xbf.as<unsigned short>());
-    MHIP_LAUNCH_CHECK();
-    const unsigned short* W = q->wbf.as<unsigned short>() + q->woff[l];
-    const float* b = q->w32.as<float>() + q->boff[l];
-    hipLaunchKernelGGL((k_mm<unsigned short, unsigned short, false, false>),
-                       dim3(cdiv(out, T), cdiv(batch, T)), dim3(256), 0, q->s, batch, out, in,
-                       q->xbf.as<unsigned short>(), W, b, Y, (l + 1 < q->nl) ? 1 : 0, 0.f);
-    MHIP_LAUNCH_CHECK();
+    const LayerDev& y = q->lay[l];
+    layer<1>(q, batch, y.out, y.in, y.inp, act_ptr(q, batch, l), q->wbf.as<unsigned short>() + y.wt,
+             q->w32.as<float>() + y.boff, (l + 1 < q->nl) ? 1 : 0, nullptr, act_ptr(q, batch, l + 1));
   }
 }
 
@@ -212,45 +424,33 @@ void forward(mhip_mlp* q, int batch) {
 void backward(mhip_mlp* q, int batch) {
   const int nout = q->dims[q->nl];
   const long long ny = (long long)batch * nout;
-  float* Y = act_ptr(q, batch, q->nl);
+  size_t tot = 0;
+  for (int l = 0; l <= q->nl; ++l) tot += (size_t)batch * q->dims[l];
+  // slices of whole 32-row steps: enough of them to fill the chip, each at
+  // least 128 rows, at most 16 (each one writes and reads a gradient)
+  const int slices = std::max(1, std::min(16, batch / 128)), rows = cdiv(cdiv(batch, slices), 32) * 32;
+  const int nslice = cdiv(batch, rows);
+  q->dz.ensure(sizeof(float) * tot);
+  q->gpart.ensure(sizeof(float) * q->np * nslice);
+  float* dz = q->dz.as<float>();
+  auto dz_of = [&](int l) { return dz + (act_ptr(q, batch, l) - q->acts.as<float>()); };
   const int pb = std::min(1024, cdiv(ny, 256));
-  hipLaunchKernelGGL(k_mse, dim3(pb), dim3(256), 0, q->s, ny, 1.f / (float)ny, Y, q->tgt.as<float>(),
-                     q->dbuf0.as<float>(), q->part.as<float>());
+  hipLaunchKernelGGL(k_mse, dim3(pb), dim3(256), 0, q->s, ny, 1.f / (float)ny, act_ptr(q, batch, q->nl),
+                     q->tgt.as<float>(), dz_of(q->nl), q->part.as<float>());
   MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_f, dim3(1), dim3(64), 0, q->s, pb, q->part.as<float>(), 1.f / (float)ny,
+  // dZ of a layer's input: dZ W^T through that input's tanh
+  for (int l = q->nl - 1; l > 0; --l) {
+    const LayerDev& y = q->lay[l];
+    layer<3>(q, batch, y.in, y.out, y.outp, dz_of(l + 1), q->wbf.as<unsigned short>() + y.wp, nullptr, 0,
+             act_ptr(q, batch, l), dz_of(l));
+  }
+  hipLaunchKernelGGL(k_dw, dim3(q->ntiles, nslice), dim3(MLP_NT), 0, q->s, q->nl, q->layers.as<LayerDev>(), batch,
+                     rows, q->acts.as<float>(), dz, (long long)q->np, q->gpart.as<float>());
+  MHIP_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_grad_sum, dim3(cdiv(q->np, 256)), dim3(256), 0, q->s, (long long)q->np, nslice,
+                     q->gpart.as<float>(), q->grad.as<float>(), pb, q->part.as<float>(), 1.f / (float)ny,
                      q->loss.as<float>());
   MHIP_LAUNCH_CHECK();
-  float* dcur = q->dbuf0.as<float>();
-  float* dnext = q->dbuf1.as<float>();
-  for (int l = q->nl - 1; l >= 0; --l) {
-    const int in = q->dims[l], out = q->dims[l + 1];
-    float* X = act_ptr(q, batch, l);
-    if (l + 1 < q->nl) {
-      // hidden layer: through tanh
-      hipLaunchKernelGGL(k_tanh_back, dim3(std::min(4096, cdiv((long long)batch * out, 256))), dim3(256),
-                         0, q->s, (long long)batch * out, act_ptr(q, batch, l + 1), dcur);
-      MHIP_LAUNCH_CHECK();
-    }
-    // dW = bf16(X)^T dZ  (in x out), db = colsum(dZ)
-    hipLaunchKernelGGL(k_to_bf16, dim3(std::min(4096, cdiv((long long)batch * in, 256))), dim3(256), 0,
-                       q->s, (long long)batch * in, X, q->xbf.as<unsigned short>());
-    MHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_mm<unsigned short, float, true, false>), dim3(cdiv(out, T), cdiv(in, T)),
-                       dim3(256), 0, q->s, in, out, batch, q->xbf.as<unsigned short>(), dcur,
-                       (const float*)nullptr, q->grad.as<float>() + q->woff[l], 0, 0.f);
-    MHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_colsum, dim3(cdiv(out, 256)), dim3(256), 0, q->s, batch, out, dcur,
-                       q->grad.as<float>() + q->boff[l]);
-    MHIP_LAUNCH_CHECK();
-    if (l > 0) {
-      // dX = dZ W^T (batch x in), W in BF16
-      hipLaunchKernelGGL((k_mm<float, unsigned short, false, true>), dim3(cdiv(in, T), cdiv(batch, T)),
-                         dim3(256), 0, q->s, batch, in, out, dcur,
-                         q->wbf.as<unsigned short>() + q->woff[l], (const float*)nullptr, dnext, 0, 0.f);
-      MHIP_LAUNCH_CHECK();
-      std::swap(dcur, dnext);
-    }
-  }
 }
 
 template <class F>
@@ -292,17 +492,36 @@ int mhip_mlp_create(int nlayers, const int* dims, mhip_mlp** out) {
     auto* q = new mhip_mlp();
     q->nl = nlayers;
     q->dims.assign(dims, dims + nlayers + 1);
-    size_t off = 0;
+    long long off = 0, bf = 0, pre = 0;
     for (int l = 0; l < nlayers; ++l) {
-      q->woff.push_back(off);
-      off += (size_t)dims[l] * dims[l + 1];
-      q->boff.push_back(off);
-      off += dims[l + 1];
+      LayerDev y{};
+      y.in = dims[l];
+      y.out = dims[l + 1];
+      y.inp = cdiv(y.in, 32) * 32;
+      y.outp = cdiv(y.out, 32) * 32;
+      y.woff = off;
+      off += (long long)y.in * y.out;
+      y.boff = off;
+      off += y.out;
+      y.wt = bf;
+      bf += (long long)y.out * y.inp;
+      y.wp = bf;
+      bf += (long long)y.in * y.outp;
+      y.pre = pre;
+      pre += y.in;
+      y.tile0 = q->ntiles;
+      q->ntiles += cdiv(y.in, 64) * cdiv(y.out, 64);
+      q->lay.push_back(y);
     }
-    q->np = off;
+    q->np = (size_t)off;
     MHIP_CHECK(hipStreamCreateWithFlags(&q->s, hipStreamNonBlocking));
+    q->layers.ensure(sizeof(LayerDev) * nlayers);
+    MHIP_CHECK(hipMemcpyAsync(q->layers.ptr, q->lay.data(), sizeof(LayerDev) * nlayers, hipMemcpyHostToDevice, q->s));
     q->w32.ensure(sizeof(float) * off);
-    q->wbf.ensure(sizeof(unsigned short) * off);
+    // the padding stays zero: refreshes write the weights only
+    q->wbf.ensure(sizeof(unsigned short) * bf);
+    hipLaunchKernelGGL(k_zero_u16, dim3(256), dim3(256), 0, q->s, bf, q->wbf.as<unsigned short>());
+    MHIP_LAUNCH_CHECK();
     q->grad.ensure(sizeof(float) * off);
     q->m.ensure(sizeof(float) * off);
     q->v.ensure(sizeof(float) * off);
@@ -316,8 +535,8 @@ int mhip_mlp_create(int nlayers, const int* dims, mhip_mlp** out) {
 void mhip_mlp_destroy(mhip_mlp* q) {
   if (!q) return;
   (void)hipStreamSynchronize(q->s);
-  for (DevBuf* b : {&q->w32, &q->wbf, &q->grad, &q->m, &q->v, &q->acts, &q->xbf, &q->dbuf0, &q->dbuf1,
-                    &q->tgt, &q->part, &q->loss})
+  for (DevBuf* b : {&q->w32, &q->wbf, &q->grad, &q->m, &q->v, &q->layers, &q->acts, &q->dz, &q->gpart, &q->tgt,
+                    &q->part, &q->loss})
     b->release();
   (void)hipStreamDestroy(q->s);
   delete q;
