@@ -471,8 +471,8 @@ def _batch_oracle_worker(items):
 def run_batch(args):
     """The batched form: 4 096 molecules (seeded alkanes C1-C20 and water
     clusters of 1-30 molecules, 6-180 basis functions, SCFCRT 1e-6), PM7 RHF,
-    each molecule's iter loop on the device, one captured hipGraph replayed
-    until every molecule is done; the integrals resident before the timed
+    each molecule's iter loop on the device until every molecule is done; the
+    integrals resident before the timed
     region.  A seeded sample of 256 molecules is checked against the oracle
     (heat, iterations) and timed on the host cores as the CPU baseline."""
     import multiprocessing as mp
@@ -492,8 +492,8 @@ def run_batch(args):
         progress(f"timed {sec:.3f} s, {nconv} converged")
     escf, niter, conv = b.results()
     # roofline of the eigensolver (the dominant kernel): the same iterations
-    # as the timed run's graph launches, launched one by one with HIP events
-    # around each size class's eigensolver launch, flops counted on the device
+    # as the timed run's, launched phase by phase with HIP events around each
+    # size class's eigensolver, flops counted on the device
     iters = 20 * max(1, -(-(int(niter.max()) + 1) // 20))
     eig_ms, eig_fl, eig_rot = b.eig_profile(iters)
     b.close()
@@ -506,7 +506,7 @@ def run_batch(args):
     ach = float(eig_fl.sum()) / (float(eig_ms.sum()) * 1e-3) / 1e12
     roof = {"bound": "mfma", "pipe": "fp64 vector (no MFMA form: 2x2 rotations)", "achieved": round(ach, 3),
             "peak": 78.6, "unit": "TFLOP/s", "frac": round(ach / 78.6, 4), "traffic": None,
-            "kernel": "k_beig_lds (every size class)", "launch_ms_total": round(float(eig_ms.sum()), 2),
+            "kernel": "batched eigensolvers (every size class)", "launch_ms_total": round(float(eig_ms.sum()), 2),
             "launches": 4 * iters, "classes": classes}
     progress(f"eigensolver: {eig_ms.sum():.1f} ms over {iters} iterations, {eig_fl.sum() / 1e9:.1f} GFLOP, "
              f"{ach:.3f} TFLOP/s")
@@ -542,7 +542,7 @@ def run_batch(args):
                    "iters_per_graph": 20},
         "converged": int(conv.sum()), "mean_iterations": round(float(niter.mean()), 2),
         "oracle_check": check, "roofline": roof, "cpu_baseline": cpu,
-        "note": "one captured hipGraph per 20 iterations of every molecule; per-kernel times in "
+        "note": "one workgroup per molecule up to 64 orbitals, batched block-Jacobi steps above; per-kernel times in "
                 "profiles/batch4096_kernels.txt",
     }
     print(json.dumps(out), flush=True)

@@ -160,7 +160,7 @@ typedef struct {
 int mhip_scf(mhip_ctx* ctx, const mhip_scf_opts* opts, mhip_scf_result* res, double* p,
              double* f, double* c, double* eig);
 
-/* ---- batched SCF: many small molecules in one captured graph --------------
+/* ---- batched SCF: many small molecules at once ----------------------------
  * No single counterpart in the reference (it runs one molecule per job); each
  * molecule follows iter (src/SCF/iter.F90:16-1107, RHF, no PULAY) with its
  * control logic on the device.  Molecules up to 256 basis functions; the
@@ -181,11 +181,15 @@ typedef struct {
 typedef struct mhip_batch mhip_batch;
 int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** out);
 /* Eigensolver workgroup size per size class (n <= 32, 64, 128, 256):
- * 64, 128, 256, 512 or 1024 (chosen by the autotuner, mopac_gpu_amd/batch.py). */
+ * 64, 128, 256, 512 or 1024 (chosen by the autotuner, mopac_gpu_amd/batch.py),
+ * for the form with its matrices in global memory (mhip_batch_set_eig_lds);
+ * the default form's workgroups are all of 512. */
 int mhip_batch_set_tiles(mhip_batch* b, const int* tiles);
-/* Where the eigensolver keeps its matrices: lds = 1 (default) puts the
- * packed A = C^T F C, and C where both fit, in LDS; lds = 0 keeps both in
- * global memory (the same rotations, for comparison). */
+/* Which eigensolver: lds = 1 (default) diagonalizes a molecule of up to 64
+ * orbitals in one workgroup's LDS, where its whole SCF runs, and larger ones
+ * by block-Jacobi steps batched over all of them; lds = 0 runs every SCF in
+ * one workgroup with cyclic Jacobi on matrices in global memory (for
+ * comparison). */
 int mhip_batch_set_eig_lds(mhip_batch* b, int lds);
 /* Eigensolver profile: `iters` iterations of the batch from its starting
  * densities, launched one by one (no graph) with HIP events around the
@@ -194,8 +198,8 @@ int mhip_batch_set_eig_lds(mhip_batch* b, int lds);
  * rotation, 2 n^3 + n^2 (n+1) for a warm start, n (n+1) nocc for the
  * density); rotations[4] (may be NULL): applied rotations. */
 int mhip_batch_eig_profile(mhip_batch* b, int iters, double* ms, double* flops, long long* rotations);
-/* Capture iters_per_graph iterations of the whole batch into one hipGraph
- * and replay it (at most max_launches times) until every molecule is done. */
+/* Run the batch from its starting densities until every molecule is done,
+ * or each has made iters_per_graph * max_launches iterations. */
 int mhip_batch_run(mhip_batch* b, int iters_per_graph, int max_launches, double* seconds,
                    int* n_converged);
 /* Heats of formation (kcal/mol, without geometry-only terms), iterations and

@@ -4,14 +4,15 @@ generator, and the project's autotuner for the batched eigensolver.
 Workload (seed 4): half seeded random alkanes CnH2n+2 (n = 1..20), half
 water clusters (H2O)k (k = 1..30, 3.1 A lattice recipe), 8-180 basis
 functions each.  Every molecule runs iter's RHF loop (no PULAY) on the
-device; the whole batch is one captured hipGraph replayed until every
-molecule is done.
+device: one workgroup for a molecule up to 64 orbitals, batched block-Jacobi
+steps for the larger ones.
 
-Autotuner: the eigensolver (one workgroup per molecule) has a workgroup size
-per size class (n <= 32, 64, 128, 256).  `autotune` times the whole batched
-SCF for each candidate size of one class at a time (the others fixed), keeps
-the fastest, and writes the table to mopac_gpu_amd/tuning/batch_tiles.json,
-which `Batch` loads by default.
+Autotuner: the eigensolver's global-memory form (one workgroup per molecule,
+set_eig_lds(False)) has a workgroup size per size class (n <= 32, 64, 128,
+256).  `autotune` times the whole batched SCF in that form for each candidate
+size of one class at a time (the others fixed), keeps the fastest, and writes
+the table to mopac_gpu_amd/tuning/batch_tiles.json, which `Batch` loads by
+default.
 """
 import ctypes
 import json
@@ -85,7 +86,8 @@ class Batch:
         self.tiles = list(tiles)
 
     def set_eig_lds(self, on=True):
-        """Eigensolver matrices in LDS (default) or in global memory."""
+        """The LDS and block-Jacobi eigensolvers (default), or one workgroup per
+        molecule with its matrices in global memory."""
         L.check(self.lib.mhip_batch_set_eig_lds(self.h, 1 if on else 0))
 
     def eig_profile(self, iters):
@@ -132,7 +134,8 @@ def autotune(batch, repeats=2, write=True):
     """Coordinate search over the eigensolver workgroup size of each class."""
     best = list(batch.tiles)
     timings = {}
-    batch.run()  # warm the caches and the graph path once
+    batch.set_eig_lds(False)  # the form whose workgroups have a size to choose
+    batch.run()  # warm the caches once
     for cls in range(4):
         scores = {}
         for cand in CANDIDATES:
@@ -145,6 +148,7 @@ def autotune(batch, repeats=2, write=True):
         best[cls] = min(scores, key=scores.get)
         timings[f"class{cls}"] = scores
     batch.set_tiles(best)
+    batch.set_eig_lds(True)
     if write:
         os.makedirs(os.path.dirname(TILES_JSON), exist_ok=True)
         with open(TILES_JSON, "w") as fh:

@@ -26,6 +26,7 @@ SOURCES = [
     "k_split.hip",
     "k_mlp.hip",
     "k_batch.hip",
+    "k_batch_eig.hip",
     "k_guess.hip",
     "mozyme_scf.hip",
     "k_mozyme.hip",

@@ -48,6 +48,10 @@ struct mhip_ctx {
   // pseudo-diagonalization workspace
   mhip::PseudoWork pseudo;
   mhip::OccVirtWork ov;
+  // a small molecule's arguments and state, for the one-workgroup SCF: on the
+  // device and in pinned memory
+  mhip::DevBuf one;
+  void* hone = nullptr;
   // statistics of the last eigensolve
   int last_sweeps = 0;
   // Jacobi stopping tolerance (relative to max|diag|) inside the SCF loop;

@@ -1,52 +1,29 @@
-// Batched SCF: thousands of small molecules of uneven size in one captured
-// hipGraph.  Every kernel covers the whole batch (a workgroup per molecule,
-// or per (molecule, atom / row)); molecules that have converged drop out by a
-// flag, so the graph is the same for every replay.  The control logic of
-// iter (src/SCF/iter.F90:340-1041: level shift, convergence test, recompute
-// with shift 0, ready/iredy) runs on the device, one thread per molecule, so
-// no scalar returns to the host until the whole batch is done.
+// Batched SCF: thousands of small molecules of uneven size.  The control logic
+// of iter (src/SCF/iter.F90:340-1041: level shift, convergence test, recompute
+// with shift 0, ready/iredy) runs on the device for every molecule.
 //
-// Per iteration: control (shift, mode) -> fock2 (batched) -> helect ->
-// control (energy, test) -> eigensolve + density (one workgroup per
-// molecule: warm-started cyclic Jacobi in parallel order, the packed matrix
-// in LDS, and the eigenvectors too where they fit) -> cnvg (batched) -> control (PL, frontier levels, newdg) ->
-// Pa = P / 2.  The eigensolve's workgroup size per size class comes from a
-// measured table (mhip_batch_tune).
+// A molecule of up to 64 orbitals is one workgroup's from start to end
+// (k_bscf_lds): Fock build, energy, control, eigensolve and density in its
+// LDS, cnvg.  Larger ones iterate together, a launch per phase over all of
+// them: control (shift, mode) -> fock2 (batched) -> helect -> control
+// (energy, test) -> block-Jacobi eigensolve + density (k_batch_eig.hip) -> cnvg
+// (batched) -> control (PL, frontier levels, newdg) -> Pa = P / 2.  Molecules
+// that have converged drop out by a flag.
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
+#include "k_batch.h"
 #include "k_fock.h"
+#include "k_fock_body.h"
+#include "k_jacobi_step.h"
 
 namespace mhip {
 namespace {
-
-struct BatchMol {
-  int n, nocc, numat;
-  double* f;
-  double* p;
-  double* pa;
-  double* pold;
-  double* p1;
-  double* C;
-  double* A;
-  double* T;
-  double* eig;
-};
-
-struct BatchState {
-  int niter, iredy, ready, done, converged, newdg, oknewd, recompute, have_c, do_eig, mode, itrmax;
-  double ten, shift, shfmax, shfto, shftbo, shiftb, pl, eold, diff, sellim, escf, ee;
-  double eig_homo, eig_lumo, enuclr, atheat, selcon, pltest;
-  // eigensolver work of this molecule since the batch was reset: applied
-  // rotations, and FP64 flops of the method (12 n per rotation: 6 n on the
-  // symmetric A, 6 n on C; warm start 2 n^3 + 2 n tri(n); density
-  // 2 tri(n) nocc)
-  long long eig_rot;
-  double eig_flops;
-};
 
 __device__ __forceinline__ double beig_flops(int n, int nocc, long long nrot, bool warm) {
   const double dn = n, tn = 0.5 * dn * (dn + 1.0);
@@ -56,14 +33,7 @@ __device__ __forceinline__ double beig_flops(int n, int nocc, long long nrot, bo
 constexpr double kEnrgy = 23.060547830619029;  // fpc_9, eV -> kcal/mol
 
 // ---- control, part 1: shift and Fock mode (iter.F90:340-420) ---------------
-__global__ void k_bctl_pre(int nmol, BatchState* __restrict__ st, int* __restrict__ act,
-                           int* __restrict__ mode, int* __restrict__ niter_out,
-                           double* __restrict__ shift_out) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nmol) return;
-  BatchState s = st[m];
-  act[m] = !s.done;
-  if (s.done) return;
+__device__ void ctl_pre(BatchState& s) {
   if (s.recompute) {
     // label 320 again: F from H with the shift set to zero, same iteration
     s.mode = kInitH;
@@ -101,6 +71,18 @@ __global__ void k_bctl_pre(int nmol, BatchState* __restrict__ st, int* __restric
       s.mode = kInitShift;
     }
   }
+}
+
+__global__ void k_bctl_pre(int nmol, const int* __restrict__ list, BatchState* __restrict__ st, int* __restrict__ act,
+                           int* __restrict__ mode, int* __restrict__ niter_out,
+                           double* __restrict__ shift_out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nmol) return;
+  const int m = list[i];
+  BatchState s = st[m];
+  act[m] = !s.done;
+  if (s.done) return;
+  ctl_pre(s);
   mode[m] = s.mode;
   niter_out[m] = s.niter;
   shift_out[m] = s.shift;
@@ -108,27 +90,20 @@ __global__ void k_bctl_pre(int nmol, BatchState* __restrict__ st, int* __restric
 }
 
 // ---- control, part 2: energy and convergence test (iter.F90:640-700) -------
-__global__ void k_bctl_mid(int nmol, BatchState* __restrict__ st, const double* __restrict__ ee,
-                           int* __restrict__ do_eig) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nmol) return;
-  BatchState s = st[m];
-  do_eig[m] = 0;
-  if (s.done) return;
-  s.ee = ee[m];
+// Sets done, recompute (F again, with the shift at zero) or do_eig.
+__device__ void ctl_mid(BatchState& s, double ee) {
+  s.do_eig = 0;
+  s.ee = ee;
   if (!isfinite(s.ee)) {
     s.done = 1;
     s.converged = 0;
-    st[m] = s;
     return;
   }
   s.escf = (s.ee + s.enuclr) * kEnrgy + s.atheat;
   if (s.niter >= s.itrmax) {
     s.done = 1;
-    st[m] = s;
     return;
   }
-  const bool was_recompute = s.recompute != 0;
   s.recompute = 0;
   s.diff = s.escf - s.eold;
   if (s.diff > 0) s.ten = s.ten - 1.0;
@@ -138,20 +113,29 @@ __global__ void k_bctl_mid(int nmol, BatchState* __restrict__ st, const double* 
     if (fabs(s.shift) < 1e-10) {
       s.converged = 1;
       s.done = 1;
-      st[m] = s;
       return;
     }
     s.shift = 0.0;
     s.shiftb = 0.0;
     s.recompute = 1;
-    st[m] = s;
     return;
   }
-  (void)was_recompute;
   s.ready = s.iredy > 0 && (fabs(s.diff) < s.sellim * 10.0 || s.pl == 0.0);
   s.iredy += 1;
   s.eold = s.escf;
-  do_eig[m] = 1;
+  s.do_eig = 1;
+}
+
+__global__ void k_bctl_mid(int nmol, const int* __restrict__ list, BatchState* __restrict__ st, const double* __restrict__ ee,
+                           int* __restrict__ do_eig) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nmol) return;
+  const int m = list[i];
+  BatchState s = st[m];
+  do_eig[m] = 0;
+  if (s.done) return;
+  ctl_mid(s, ee[m]);
+  do_eig[m] = s.do_eig;
   st[m] = s;
 }
 
@@ -173,55 +157,44 @@ __device__ double wg_max(double v, double* red) {
   return r;
 }
 
-// maxima of two values over the workgroup: within each wave by lane
-// exchange, then across the NT / 64 waves through red (2 NT / 64 doubles)
-template <int NT>
-__device__ void wg_max2(double& a, double& b, double* red) {
-  for (int o = 32; o > 0; o >>= 1) {
-    a = fmax(a, __shfl_xor(a, o));
-    b = fmax(b, __shfl_xor(b, o));
-  }
-  constexpr int NW = NT / 64;
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    red[w] = a;
-    red[NW + w] = b;
-  }
-  __syncthreads();
-  a = red[0];
-  b = red[NW];
-  for (int i = 1; i < NW; ++i) {
-    a = fmax(a, red[i]);
-    b = fmax(b, red[NW + i]);
-  }
-  __syncthreads();
+// what one eigensolve did
+struct EigCount {
+  int nrot, sweeps;
+};
+
+__device__ __forceinline__ void eig_done(const BatchMol& M, BatchState& s, EigCount c, bool warm) {
+  if (threadIdx.x != 0) return;
+  s.eig_rot += c.nrot;
+  s.eig_flops += beig_flops(M.n, M.nocc, c.nrot, warm);
+  s.sweeps += c.sweeps;
+  s.last_sweeps = c.sweeps;
+  s.stuck |= c.sweeps >= kEigSweeps;
+  s.ndiag += 1;
+  s.have_c = 1;
 }
 
-constexpr int kMaxBatchN = 256;
-
+// Eigenvectors of M.f (warm: from M.C) into M.C, ascending, the levels into
+// M.eig, and, with nocc > 0, the packed density into M.p.  Matrices in global
+// memory.
 template <int NT>
-__global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, const int* __restrict__ do_eig,
-                                             BatchState* __restrict__ st, const int* __restrict__ list,
-                                             double tol) {
-  const int m = list[blockIdx.x];
-  if (!do_eig[m]) return;
-  const BatchMol& M = mols[m];
+__device__ EigCount beig_global(const BatchMol& M, double* f, bool warm, double tol, bool density) {
   const int n = M.n, tid = threadIdx.x;
   __shared__ double red[NT];
   __shared__ double cs[kMaxBatchN / 2], sn[kMaxBatchN / 2];
   __shared__ int pp[kMaxBatchN / 2], qq[kMaxBatchN / 2];
   __shared__ int rank[kMaxBatchN];
   __shared__ int nrot;
+  __syncthreads();
   if (tid == 0) nrot = 0;
+  int sweeps = 0;
   double* A = M.A;
   double* C = M.C;
   double* T = M.T;
-  const bool warm = st[m].have_c != 0;
   // eigenvectors_LAPACK: F(i,i) += i * 1e-10, in place
-  for (int i = tid; i < n; i += NT) M.f[(long long)i * (i + 1) / 2 + i] += (double)(i + 1) * 1.0e-10;
+  for (int i = tid; i < n; i += NT) f[(long long)i * (i + 1) / 2 + i] += (double)(i + 1) * 1.0e-10;
   __syncthreads();
   auto F = [&](int r, int c) -> double {
-    return r >= c ? M.f[(long long)r * (r + 1) / 2 + c] : M.f[(long long)c * (c + 1) / 2 + r];
+    return r >= c ? f[(long long)r * (r + 1) / 2 + c] : f[(long long)c * (c + 1) / 2 + r];
   };
   if (warm) {
     // T = F C, A = C^T T
@@ -248,7 +221,7 @@ __global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, 
   __syncthreads();
   const int np = (n + 1) & ~1;
   const int npair = np / 2;
-  for (int sweep = 0; sweep < 60; ++sweep) {
+  for (int sweep = 0; sweep < kEigSweeps; ++sweep) {
     double off = 0.0, dg = 0.0;
     for (int e = tid; e < n * n; e += NT) {
       const int r = e % n, c = e / n;
@@ -258,6 +231,7 @@ __global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, 
     off = wg_max<NT>(off, red);
     dg = wg_max<NT>(dg, red);
     if (off <= tol * fmax(dg, 1.0)) break;
+    ++sweeps;
     for (int r = 0; r < np - 1; ++r) {
       for (int k = tid; k < npair; k += NT) {
         int p = rr_index(k, r, np), q = rr_index(np - 1 - k, r, np);
@@ -325,6 +299,8 @@ __global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, 
   __syncthreads();
   for (int e = tid; e < n * n; e += NT) C[e] = T[e];
   __syncthreads();
+  const EigCount cnt{nrot, sweeps};
+  if (!density) return cnt;
   // P = 2 C_occ C_occ^T, packed
   const long long mp = (long long)n * (n + 1) / 2;
   for (long long q = tid; q < mp; q += NT) {
@@ -336,38 +312,20 @@ __global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, 
     for (int k = 0; k < M.nocc; ++k) s += C[r + k * n] * C[c + k * n];
     M.p[q] = 2.0 * s;
   }
-  if (tid == 0) {
-    st[m].eig_rot += nrot;
-    st[m].eig_flops += beig_flops(n, M.nocc, nrot, warm);
-    st[m].have_c = 1;
-  }
+  return cnt;
 }
 
-// LDS form of the batched eigensolver: the same warm-started cyclic Jacobi in
-// parallel (round-robin) order, with the working matrix A = C^T F C kept as
-// its lower triangle, packed, in LDS (np (np+1) / 2 doubles, np = n rounded
-// up to even; row n of an odd n is a zero row that no rotation touches), and
-// C in LDS too when both fit (CLDS).  One round is two phases: the angles of
-// its np / 2 disjoint pairs, then every 2x2 block (pair k1, pair k2) of A
-// turned by both rotations together (rows by k1, columns by k2), and, with
-// CLDS, the columns of C.  Without CLDS the rounds log their (c, s) in global
-// memory and C is turned once per sweep: A is parked in global memory, C
-// passes through the freed LDS in chunks of rows, each chunk taking the
-// sweep's rounds in order (the same operations on every element as turning
-// C round by round), then A comes back.
-// A rotation whose |a_pq| is under 1e-2 tol max(|diag|, 1) is skipped: the
-// sweep loop stops once every off-diagonal element is under tol max(|diag|,
-// 1), so such an element already meets it.  The warm start stages F in the
-// LDS that A later takes: T' = (F C)^T in global memory (lanes along rows of
-// F, C read as wave-uniform columns), then A = C^T T' with lanes along the
-// columns of T' (contiguous) and four rows per thread.
-__device__ __forceinline__ int tri(int i) { return (i * (i + 1)) >> 1; }
-// rr_index for idx, r < np - 1 (the sum wraps at most once)
-__device__ __forceinline__ int rr_pos(int idx, int r, int np) {
-  if (idx == 0) return 0;
-  const int t = r + idx - 1;
-  return 1 + (t >= np - 1 ? t - (np - 1) : t);
+template <int NT>
+__global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, const int* __restrict__ do_eig,
+                                             BatchState* __restrict__ st, const int* __restrict__ list,
+                                             double tol) {
+  const int m = list[blockIdx.x];
+  if (!do_eig[m]) return;
+  const bool warm = st[m].have_c != 0;
+  eig_done(mols[m], st[m], beig_global<NT>(mols[m], mols[m].f, warm, tol, true), warm);
 }
+
+__device__ __forceinline__ int tri(int i) { return (i * (i + 1)) >> 1; }
 __device__ __forceinline__ int sym_at(int a, int b) { return a >= b ? tri(a) + b : tri(b) + a; }
 // row of packed lower-triangle index e (exact for e < 2^22)
 __device__ __forceinline__ int tri_row(int e) {
@@ -377,347 +335,132 @@ __device__ __forceinline__ int tri_row(int e) {
   return i;
 }
 
-// C <- C R^T for the logged rounds of one sweep, in chunks of at most NT rows
-// staged in LDS (ch, room doubles, column-major per chunk); thread (row,
-// slot) turns its row for the pairs slot, slot + NT / rows, ... of every
-// round, while the pairs of the next round are staged.
-template <int NT>
-__device__ void beig_flush_c(double* __restrict__ C, const double* __restrict__ lg, int n, int np, double* ch,
-                             int room, double2 (*csn2)[kMaxBatchN / 2], int2 (*off2)[kMaxBatchN / 2]) {
-  const int tid = threadIdx.x, npair = np / 2, nround = np - 1;
-  const int R = min(min(n, room / n), NT);
-  for (int r0 = 0; r0 < n; r0 += R) {
-    const int rows = min(R, n - r0);
-    // round r's (c, s) for the pairs k = tid + j NT are fetched into
-    // registers two rounds ahead and put into LDS one round ahead
-    constexpr int KP = (kMaxBatchN / 2 + NT - 1) / NT;
-    double fc[KP], fs[KP];
-    auto fetch = [&](int r) {
+// Molecules up to kMaxLdsN orbitals are one pair problem of the block-Jacobi
+// steps (k_jacobi_step.h), padded to 64 with decoupled large entries: the
+// whole eigensolve in one workgroup's LDS, the products with C on the matrix
+// cores.  C is 64 x 64 in memory (M.C, identity in the padding).
+// A cyclic Jacobi over the packed A, with C beside it in LDS and two barriers
+// a round, took 3400 cycles a round at 26 orbitals and 4350 at 60, its chain
+// of LDS reads; a round here takes 940 in the level of 32 rounds, and about 1700 with
+// the levels between them.
+// Larger molecules go to the steps over several workgroups of k_batch_eig.hip.
+static_assert(kMaxLdsN == SB, "one pair problem");
+constexpr int kLdsThreads = CROSS_THREADS;
+
+__device__ __noinline__ EigCount beig_lds(JacLds& lds, const BatchMol& M, double* f, bool warm, double tol, bool density) {
+  const int n = M.n, tid = threadIdx.x;
+  __shared__ int rank[SB];
+  double(*S)[SB] = lds.s();
+  double(*X)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds.m);
+  double(*Y)[LDSW] = reinterpret_cast<double (*)[LDSW]>(lds.m + SB * LDSW);
+  double* C = M.C;
+  constexpr int PER = SB * SB / kLdsThreads;
+  __syncthreads();
+  // eigenvectors_LAPACK: F(i,i) += i * 1e-10, in place
+  if (tid < n) f[tri(tid) + tid] += (double)(tid + 1) * 1.0e-10;
+  __syncthreads();
+  auto fp = [&](int r, int c) -> double {
+    return r < n && c < n ? f[sym_at(r, c)] : (r == c ? 1.0e4 + r : 0.0);
+  };
+  d4_t acc[2];
+  if (warm) {
+    // A = C^T (F C)
 #pragma unroll
-      for (int j = 0; j < KP; ++j) {
-        const int k = tid + j * NT;
-        if (k < npair) {
-          fc[j] = lg[2 * (r * npair + k)];
-          fs[j] = lg[2 * (r * npair + k) + 1];
-        }
-      }
-    };
-    auto put = [&](int r) {
-      const int b = r & 1;
-#pragma unroll
-      for (int j = 0; j < KP; ++j) {
-        const int k = tid + j * NT;
-        if (k < npair) {
-          int p = rr_pos(k, r, np), q = rr_pos(np - 1 - k, r, np);
-          if (p > q) { const int t = p; p = q; q = t; }
-          csn2[b][k] = make_double2(fc[j], q < n ? fs[j] : 0.0);
-          off2[b][k] = make_int2(p * rows, q * rows);
-        }
-      }
-    };
-    for (int e = tid; e < rows * n; e += NT) {
-      const int row = e % rows, col = e / rows;
-      ch[row + col * rows] = C[r0 + row + (size_t)col * n];
-    }
-    fetch(0);
-    put(0);
-    if (nround > 1) fetch(1);
-    __syncthreads();
-    const int kstep = NT / rows, row = tid % rows, slot = tid / rows;
-    for (int r = 0; r < nround; ++r) {
-      if (r + 1 < nround) put(r + 1);
-      if (r + 2 < nround) fetch(r + 2);
-      const int b = r & 1;
-      if (slot < kstep) {
-        for (int k = slot; k < npair; k += kstep) {
-          const double2 a = csn2[b][k];
-          if (a.y != 0.0) {
-            const int2 o = off2[b][k];
-            double* cp = ch + o.x + row;
-            double* cq = ch + o.y + row;
-            const double u = *cp, v = *cq;
-            *cp = a.x * u - a.y * v;
-            *cq = a.y * u + a.x * v;
-          }
-        }
-      }
-      __syncthreads();
-    }
-    for (int e = tid; e < rows * n; e += NT) {
-      const int row2 = e % rows, col = e / rows;
-      C[r0 + row2 + (size_t)col * n] = ch[row2 + col * rows];
+    for (int it = 0; it < PER; ++it) {
+      const int e = tid + kLdsThreads * it;
+      X[e % SB][e / SB] = fp(e % SB, e / SB);
+      Y[e % SB][e / SB] = C[e];
     }
     __syncthreads();
+    acc[0] = acc[1] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return X[r][k]; }, [&](int k, int c) { return Y[k][c]; }, SB, acc);
+    __syncthreads();
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) { X[r][c] = v; });
+    __syncthreads();
+    acc[0] = acc[1] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return Y[k][r]; }, [&](int k, int c) { return X[k][c]; }, SB, acc);
+    __syncthreads();
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) { S[r][c] = v; });
+  } else {
+#pragma unroll
+    for (int it = 0; it < PER; ++it) {
+      const int e = tid + kLdsThreads * it;
+      S[e / SB][e % SB] = fp(e / SB, e % SB);
+    }
   }
+  __syncthreads();
+  const int sweeps = pair_solve(lds, 0, 1, true, JacSolve{n, nullptr, nullptr, nullptr, nullptr, tol, 0.0, kEigSweeps});
+  // ascending order, ties by index; the padding stays where it is
+  if (tid < SB) {
+    const double d = S[tid][tid];
+    int rk = tid;
+    if (tid < n) {
+      rk = 0;
+      for (int j = 0; j < n; ++j) {
+        const double o = S[j][j];
+        rk += (o < d || (o == d && j < tid)) ? 1 : 0;
+      }
+      M.eig[rk] = d;
+    }
+    rank[tid] = rk;
+  }
+  __syncthreads();
+  // C Q in the order of the levels, by rows of C's transpose
+  double(*Ct)[SB] = lds.s();
+  double(*Q)[LDSW] = lds.q();
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + kLdsThreads * it, r = e % SB, c = e / SB;
+    Ct[c][r] = warm ? C[e] : (r == c ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  if (sweeps > 0) {
+    acc[0] = acc[1] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return Ct[k][r]; }, [&](int k, int c) { return Q[k][c]; }, SB, acc);
+    __syncthreads();
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) { X[rank[c]][r] = v; });
+  } else {
+    double v[PER];
+#pragma unroll
+    for (int it = 0; it < PER; ++it) v[it] = Ct[(tid + kLdsThreads * it) / SB][(tid + kLdsThreads * it) % SB];
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < PER; ++it)
+      X[rank[(tid + kLdsThreads * it) / SB]][(tid + kLdsThreads * it) % SB] = v[it];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < PER; ++it) {
+    const int e = tid + kLdsThreads * it;
+    C[e] = X[e / SB][e % SB];
+  }
+  if (density) {
+    // P = 2 C_occ C_occ^T, packed
+    const int nocc = M.nocc;
+    acc[0] = acc[1] = d4_t{0.0, 0.0, 0.0, 0.0};
+    mfma_tile64_w8([&](int r, int k) { return k < nocc ? X[k][r] : 0.0; },
+                   [&](int k, int c) { return X[k][c]; }, (nocc + 3) & ~3, acc);
+    mfma_tile64_w8_store(acc, [&](int r, int c, double v) {
+      if (r < n && c <= r) M.p[tri(r) + c] = 2.0 * v;
+    });
+  }
+  return EigCount{sweeps * (n * (n - 1) / 2), sweeps};
 }
 
-template <int NT, bool CLDS>
-__global__ __launch_bounds__(NT) void k_beig_lds(const BatchMol* __restrict__ mols, const int* __restrict__ do_eig,
-                                                 BatchState* __restrict__ st, const int* __restrict__ list,
-                                                 double tol, int room) {
+__global__ __launch_bounds__(kLdsThreads, 4) void k_beig_lds(const BatchMol* __restrict__ mols,
+                                                             const int* __restrict__ do_eig,
+                                                             BatchState* __restrict__ st,
+                                                             const int* __restrict__ list, double tol) {
+  __shared__ JacLds lds;
   const int m = list[blockIdx.x];
   if (!do_eig[m]) return;
-  const BatchMol& M = mols[m];
-  const int n = M.n, tid = threadIdx.x;
-  const int np = (n + 1) & ~1;
-  const int npair = np / 2;
-  __shared__ double red[2 * (NT / 64)];
-  __shared__ double2 csn2[2][kMaxBatchN / 2];  // (c, s) of every pair; two buffers for the flush
-  __shared__ int4 pq4[kMaxBatchN / 2];         // p, q, tri(p), tri(q)
-  __shared__ int2 off2[2][kMaxBatchN / 2];     // the flush's column offsets
-  __shared__ int rank[kMaxBatchN];
-  __shared__ int rotated, nrot;
-  if (tid == 0) nrot = 0;
-  double2* csn = csn2[0];
-  extern __shared__ double dyn[];
-  double* A = dyn;                               // tri(np) packed lower triangle
-  double* C = CLDS ? dyn + tri(np) : M.C;        // n x n, column-major
-  double* Tt = M.T;                              // n x n scratch, global
   const bool warm = st[m].have_c != 0;
-  const int na = tri(np);
-  // without CLDS: the sweep's (c, s) log, np (np-1) doubles, then A parked
-  double* lg = M.A;
-  double* park = M.A + (size_t)np * (np - 1);
-  // eigenvectors_LAPACK: F(i,i) += i * 1e-10, in place
-  for (int i = tid; i < n; i += NT) M.f[tri(i) + i] += (double)(i + 1) * 1.0e-10;
-  __syncthreads();
-  // F (packed, same layout as A's first n rows) into LDS, zero row n
-  for (int e = tid; e < na; e += NT) A[e] = e < tri(n) ? M.f[e] : 0.0;
-  if (CLDS && warm)
-    for (int e = tid; e < n * n; e += NT) C[e] = M.C[e];
-  __syncthreads();
-  if (warm) {
-    // T'(c, r) = sum_k F(r, k) C(k, c): four columns c per thread (the
-    // columns past n repeat column n - 1 and are not stored)
-    const int ncb = (n + 3) >> 2;
-    for (int w = tid; w < n * ncb; w += NT) {
-      const int r = w % n, c0 = (w / n) * 4;
-      const int rb = tri(r);
-      const double* q0 = C + (size_t)c0 * n;
-      const double* q1 = C + (size_t)min(c0 + 1, n - 1) * n;
-      const double* q2 = C + (size_t)min(c0 + 2, n - 1) * n;
-      const double* q3 = C + (size_t)min(c0 + 3, n - 1) * n;
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll 4
-      for (int k = 0; k < n; ++k) {
-        const double f = A[k <= r ? rb + k : tri(k) + r];
-        s0 += f * q0[k];
-        s1 += f * q1[k];
-        s2 += f * q2[k];
-        s3 += f * q3[k];
-      }
-      double* t = Tt + c0 + (size_t)r * n;
-      t[0] = s0;
-      if (c0 + 1 < n) t[1] = s1;
-      if (c0 + 2 < n) t[2] = s2;
-      if (c0 + 3 < n) t[3] = s3;
-    }
-    __syncthreads();
-    // A(i, j) = sum_k C(k, i) T'(j, k), j <= i: rows i0..i0+3 per thread
-    const int nib = (n + 3) >> 2;
-    for (int w = tid; w < n * nib; w += NT) {
-      const int j = w % n, i0 = (w / n) * 4;
-      if (j > i0 + 3) continue;
-      const double* c0 = C + (size_t)i0 * n;
-      const double* c1 = C + (size_t)min(i0 + 1, n - 1) * n;
-      const double* c2 = C + (size_t)min(i0 + 2, n - 1) * n;
-      const double* c3 = C + (size_t)min(i0 + 3, n - 1) * n;
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll 4
-      for (int k = 0; k < n; ++k) {
-        const double t = Tt[j + (size_t)k * n];
-        s0 += c0[k] * t;
-        s1 += c1[k] * t;
-        s2 += c2[k] * t;
-        s3 += c3[k] * t;
-      }
-      if (j <= i0) A[tri(i0) + j] = s0;
-      if (i0 + 1 < n && j <= i0 + 1) A[tri(i0 + 1) + j] = s1;
-      if (i0 + 2 < n && j <= i0 + 2) A[tri(i0 + 2) + j] = s2;
-      if (i0 + 3 < n && j <= i0 + 3) A[tri(i0 + 3) + j] = s3;
-    }
-  } else {
-    for (int e = tid; e < n * n; e += NT) {
-      const int r = e % n, c = e / n;
-      C[e] = (r == c) ? 1.0 : 0.0;
-    }
-  }
-  __syncthreads();
-  const int nblk = tri(npair);  // 2x2 blocks (k1 >= k2)
-  // the blocks of this thread, k1 | k2 << 8, kept in registers
-  constexpr int KB = NT >= 256 ? (kMaxBatchN / 2 * (kMaxBatchN / 2 + 1) / 2 + NT - 1) / NT : 1;
-  int blk[KB];
-  if constexpr (NT >= 256) {
-#pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      const int b = tid + j * NT;
-      const int k1 = b < nblk ? tri_row(b) : 0;
-      blk[j] = b < nblk ? k1 | ((b - tri(k1)) << 8) : -1;
-    }
-  }
-  // A <- R A R^T on the block (pair k1 rows, pair k2 columns), R = [c -s; s c]
-  auto turn_block = [&](int k1, int k2) {
-    const double2 a1 = csn[k1], a2 = csn[k2];
-    if (a1.y == 0.0 && a2.y == 0.0) return;
-    const double c1 = a1.x, s1 = a1.y, c2 = a2.x, s2 = a2.y;
-    const int4 i1 = pq4[k1];
-    if (k1 == k2) {
-      const int ip = i1.z + i1.x, iq = i1.w + i1.y, ipq = i1.w + i1.x;
-      const double x = A[ip], y = A[ipq], v = A[iq];
-      // rows, then columns
-      const double x1 = c1 * x - s1 * y, y1 = s1 * x + c1 * y;
-      const double u1 = c1 * y - s1 * v, v1 = s1 * y + c1 * v;
-      A[ip] = c1 * x1 - s1 * u1;
-      A[iq] = s1 * y1 + c1 * v1;
-      A[ipq] = 0.0;
-    } else {
-      const int4 i2 = pq4[k2];
-      const int ixx = i1.x >= i2.x ? i1.z + i2.x : i2.z + i1.x;
-      const int iyx = i1.y >= i2.x ? i1.w + i2.x : i2.z + i1.y;
-      const int ixu = i1.x >= i2.y ? i1.z + i2.y : i2.w + i1.x;
-      const int iyu = i1.y >= i2.y ? i1.w + i2.y : i2.w + i1.y;
-      const double x = A[ixx], y = A[iyx], u = A[ixu], v = A[iyu];
-      const double x1 = c1 * x - s1 * y, y1 = s1 * x + c1 * y;
-      const double u1 = c1 * u - s1 * v, v1 = s1 * u + c1 * v;
-      A[ixx] = c2 * x1 - s2 * u1;
-      A[ixu] = s2 * x1 + c2 * u1;
-      A[iyx] = c2 * y1 - s2 * v1;
-      A[iyu] = s2 * y1 + c2 * v1;
-    }
-  };
-  const int stepk = NT / n, stepr = NT % n;
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    double off = 0.0, dg = 0.0;
-    for (int e = tid; e < tri(n); e += NT) {
-      const int i = tri_row(e);
-      const double v = fabs(A[e]);
-      if (e == tri(i) + i) dg = fmax(dg, v);
-      else off = fmax(off, v);
-    }
-    if (tid == 0) rotated = 0;
-    wg_max2<NT>(off, dg, red);
-    const double lim = tol * fmax(dg, 1.0);
-    if (off <= lim) break;
-    const double skip = 1.0e-2 * lim;
-    for (int r = 0; r < np - 1; ++r) {
-      for (int k = tid; k < npair; k += NT) {
-        int p = rr_pos(k, r, np), q = rr_pos(np - 1 - k, r, np);
-        if (p > q) { const int t = p; p = q; q = t; }
-        double c = 1.0, s = 0.0;
-        if (q < n) {
-          const double app = A[tri(p) + p], aqq = A[tri(q) + q], apq = A[tri(q) + p];
-          // |a_pq| > 1e-18 sqrt|a_pp a_qq| compared as squares
-          if (fabs(apq) > skip && apq * apq > 1.0e-36 * fabs(app * aqq)) {
-            const double theta = (aqq - app) / (2.0 * apq);
-            const double t = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-            c = rsqrt(t * t + 1.0);
-            s = t * c;
-            atomicAdd(&nrot, 1);
-          }
-        }
-        csn[k] = make_double2(c, s);
-        pq4[k] = make_int4(p, q, tri(p), tri(q));
-        if (!CLDS) {
-          lg[2 * (r * npair + k)] = c;
-          lg[2 * (r * npair + k) + 1] = s;
-          if (s != 0.0) rotated = 1;
-        }
-      }
-      __syncthreads();
-      if constexpr (NT >= 256) {
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-          if (blk[j] < 0) break;
-          turn_block(blk[j] & 0xff, blk[j] >> 8);
-        }
-      } else {
-        for (int b = tid; b < nblk; b += NT) {
-          const int k1 = tri_row(b);
-          turn_block(k1, b - tri(k1));
-        }
-      }
-      // C <- C R^T on columns (p, q)
-      if (CLDS) {
-        int k = tid / n, row = tid % n;
-        for (int e = tid; e < npair * n; e += NT) {
-          const double2 a = csn[k];
-          if (a.y != 0.0) {
-            const int4 iq = pq4[k];
-            double* cp = C + iq.x * n + row;
-            double* cq = C + iq.y * n + row;
-            const double u = *cp, v = *cq;
-            *cp = a.x * u - a.y * v;
-            *cq = a.y * u + a.x * v;
-          }
-          k += stepk;
-          row += stepr;
-          if (row >= n) { row -= n; ++k; }
-        }
-      }
-      __syncthreads();
-    }
-    // every thread reads the flag before thread 0 may clear it for the next sweep
-    const bool pending = !CLDS && rotated != 0;
-    __syncthreads();
-    if (pending) {
-      for (int e = tid; e < na; e += NT) park[e] = A[e];
-      __syncthreads();
-      beig_flush_c<NT>(C, lg, n, np, dyn, room, csn2, off2);
-      for (int e = tid; e < na; e += NT) A[e] = park[e];
-      __syncthreads();
-    }
-  }
-  // ascending order, ties by index
-  for (int i = tid; i < n; i += NT) {
-    const double ai = A[tri(i) + i];
-    int rk = 0;
-    for (int j = 0; j < n; ++j) {
-      const double aj = A[tri(j) + j];
-      rk += (aj < ai || (aj == ai && j < i)) ? 1 : 0;
-    }
-    rank[i] = rk;
-  }
-  __syncthreads();
-  double* sorted = CLDS ? M.C : Tt;
-  for (int e = tid; e < n * n; e += NT) {
-    const int r = e % n, c = e / n;
-    sorted[r + rank[c] * n] = C[e];
-  }
-  for (int i = tid; i < n; i += NT) M.eig[rank[i]] = A[tri(i) + i];
-  __syncthreads();
-  if (!CLDS)
-    for (int e = tid; e < n * n; e += NT) M.C[e] = Tt[e];
-  __syncthreads();
-  // P = 2 C_occ C_occ^T, packed, with C_occ staged in LDS where it fits
-  const int nocc = M.nocc;
-  const double* Cg = M.C;
-  if (n * nocc <= room) {
-    for (int e = tid; e < n * nocc; e += NT) dyn[e] = Cg[e];
-    Cg = dyn;
-    __syncthreads();
-  }
-  for (int q = tid; q < tri(n); q += NT) {
-    const int r = tri_row(q), c = q - tri(r);
-    double s = 0.0;
-#pragma unroll 4
-    for (int k = 0; k < nocc; ++k) s += Cg[r + k * n] * Cg[c + k * n];
-    M.p[q] = 2.0 * s;
-  }
-  if (tid == 0) {
-    st[m].eig_rot += nrot;
-    st[m].eig_flops += beig_flops(n, M.nocc, nrot, warm);
-    st[m].have_c = 1;
-  }
+  eig_done(mols[m], st[m], beig_lds(lds, mols[m], mols[m].f, warm, tol, true), warm);
 }
 
 // ---- control, part 3: PL, frontier levels, newdg (iter.F90:1030-1041) -------
-__global__ void k_bctl_post(int nmol, const BatchMol* __restrict__ mols, BatchState* __restrict__ st,
-                            const int* __restrict__ do_eig, const double* __restrict__ scal) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nmol || !do_eig[m]) return;
-  BatchState s = st[m];
-  const BatchMol& M = mols[m];
-  s.pl = scal[2 * m];
+__device__ void ctl_post(BatchState& s, const BatchMol& M, double pl) {
+  s.pl = pl;
   const int ih = max(M.nocc, 1);
   if (ih < M.n) {
     s.eig_homo = M.eig[ih - 1];
@@ -727,7 +470,386 @@ __global__ void k_bctl_post(int nmol, const BatchMol* __restrict__ mols, BatchSt
   s.oknewd = (s.pl < s.sellim) || s.oknewd;
   s.newdg = ((s.pl < trans) && s.oknewd) || s.newdg;
   if (s.pl < trans * 0.3333) s.oknewd = 1;
+}
+
+__global__ void k_bctl_post(int nmol, const int* __restrict__ list, const BatchMol* __restrict__ mols, BatchState* __restrict__ st,
+                            const int* __restrict__ do_eig, const double* __restrict__ scal) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nmol) return;
+  const int m = list[i];
+  if (!do_eig[m]) return;
+  BatchState s = st[m];
+  ctl_post(s, mols[m], scal[2 * m]);
   st[m] = s;
+}
+
+// ---- the whole SCF of a molecule in one workgroup ----------------------------
+// The Fock build of a small molecule (n <= kMaxLdsN) by the workgroup, from P
+// and Pa staged in LDS (ps: 2 tri(n) doubles): four lanes per element of the
+// diagonal atom blocks (its Coulomb field over every partner, and the
+// one-centre terms), a thread per element between two atoms (its exchange
+// sum of at most 16 terms).  No partial sums go through memory, and no wave
+// is left with an atom's three or four partners: the row and column passes
+// of k_fock.hip, a wave per atom, took 95 of 105 thousand cycles beside the
+// eigensolve at 26 orbitals, this takes TODO.
+template <int NT>
+__device__ void fock_small(const FockArgs& a, const int* atom_of, double* ps) {
+  const int n = a.sys.norbs, tid = threadIdx.x, mp = tri(n), numat = a.sys.numat;
+  double* pas = ps + mp;
+  for (int q = tid; q < mp; q += NT) {
+    ps[q] = a.p[q];
+    pas[q] = a.pa[q];
+  }
+  __syncthreads();
+  auto pr = [](int u, int v) { return u >= v ? tri(u) + v : tri(v) + u; };
+  const double* __restrict__ W = a.sys.w;
+  // diagonal blocks: element e is pair ab of atom i
+  const int nd = (int)a.sys.wcum[numat - 1] + (a.sys.norb[numat - 1] == 4 ? 10 : 1);
+  for (int base = 0; base < nd; base += NT / 4) {
+    const int e = base + (tid >> 2), part = tid & 3;
+    int i = 0;
+    double g = 0.0;
+    if (e < nd) {
+      // the last atom whose first element is not after e
+      int lo = 0, hi = numat - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.sys.wcum[mid] <= e) lo = mid;
+        else hi = mid - 1;
+      }
+      i = lo;
+      const int ab = e - (int)a.sys.wcum[i], limi = a.sys.norb[i] == 4 ? 10 : 1;
+      for (int j = part; j < numat; j += 4) {
+        if (j == i) continue;
+        const int fj = a.sys.nf0[j], nj = a.sys.norb[j], limj = nj == 4 ? 10 : 1;
+        // element (ab of i, cd of j) of the pair's block
+        const double* wb;
+        int step;
+        if (j < i) {
+          wb = W + a.sys.woff[i] + (long long)limi * a.sys.wcum[j] + ab * limj;
+          step = 1;
+        } else {
+          wb = W + a.sys.woff[j] + (long long)limj * a.sys.wcum[i] + ab;
+          step = limi;
+        }
+        if (nj == 4) {
+          double w[10];
+#pragma unroll
+          for (int cd = 0; cd < 10; ++cd) w[cd] = wb[cd * step];
+#pragma unroll
+          for (int cd = 0; cd < 10; ++cd) {
+            const int x = c_pa[cd], y = c_pb[cd];
+            g += w[cd] * ps[tri(fj + x) + fj + y] * (x == y ? 1.0 : 2.0);
+          }
+        } else {
+          g += wb[0] * ps[tri(fj) + fj];
+        }
+      }
+    }
+    g += __shfl_xor(g, 1, 64);
+    g += __shfl_xor(g, 2, 64);
+    if (e < nd && part == 0) {
+      const int ab = e - (int)a.sys.wcum[i], ni = a.sys.norb[i], fi = a.sys.nf0[i], lim = ni == 4 ? 10 : 1;
+      const int x = c_pa[ab], y = c_pb[ab];
+      // one-centre terms (fock1.F90:38-88)
+      const double* __restrict__ w1 = W + a.sys.w1off[i];
+      for (int k = 0; k < ni; ++k)
+        for (int l = 0; l < ni; ++l) {
+          const int q = sym_at(fi + k, fi + l);
+          g += ps[q] * w1[pr(k, l) * lim + ab] - pas[q] * w1[pr(l, x) * lim + pr(k, y)];
+        }
+      const int q = tri(fi + x) + fi + y;
+      a.f[q] = finit(a, q, x == y) + g;
+    }
+  }
+  // elements between two atoms
+  for (int q = tid; q < mp; q += NT) {
+    const int r = tri_row(q), c = q - tri(r);
+    const int i = atom_of[r], j = atom_of[c];
+    if (i == j) continue;
+    const int fi = a.sys.nf0[i], fj = a.sys.nf0[j], ni = a.sys.norb[i], nj = a.sys.norb[j];
+    const int x = r - fi, u = c - fj, limi = ni == 4 ? 10 : 1, limj = nj == 4 ? 10 : 1;
+    const double* __restrict__ wb = W + a.sys.woff[i] + (long long)limi * a.sys.wcum[j];
+    double k = 0.0;
+    for (int y = 0; y < ni; ++y) {
+      const double* row = wb + pr(x, y) * limj;
+      const double* pa = pas + tri(fi + y) + fj;
+      if (nj == 4) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) k += pa[v] * row[pr(u, v)];
+      } else {
+        k += pa[0] * row[0];
+      }
+    }
+    a.f[q] = finit(a, q, false) - k;
+  }
+}
+
+// Column pass of the Fock build for atom j by one wave (k_fock.hip has the
+// workgroup form).
+__device__ void fock_cols_wave(const FockArgs& a, const int j, const int lane) {
+  const int nj = a.sys.norb[j];
+  const int lim = (nj == 4) ? 10 : 1;
+  const long long fj = a.sys.nf0[j];
+  const int m = (a.sys.numat - 1 - j) * lim;
+  const double* __restrict__ src = a.jcol + a.sys.ccol[j];
+  double s = 0.0;
+  if (lim == 10) {
+    if (lane < 60)
+      for (int idx = lane; idx < m; idx += 60) s += src[idx];
+    // the six lanes of pair index lane % 10
+    double t = s;
+#pragma unroll
+    for (int k = 1; k < 6; ++k) t += __shfl(s, lane + 10 * k, 64);
+    s = t;
+  } else {
+    for (int idx = lane; idx < m; idx += 64) s += src[idx];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  }
+  if (lane >= lim) return;
+  const int x = c_pa[lane], y = c_pb[lane];
+  // one-centre terms (fock1.F90:38-88)
+  const double* __restrict__ w1 = a.sys.w + a.sys.w1off[j];
+  auto pr = [](int u, int v) { return u >= v ? u * (u + 1) / 2 + v : v * (v + 1) / 2 + u; };
+  double g = 0.0;
+  for (int k = 0; k < nj; ++k)
+    for (int l = 0; l < nj; ++l) {
+      const long long q = pk(fj + k, fj + l);
+      g += a.p[q] * w1[pr(k, l) * lim + lane] - a.pa[q] * w1[pr(l, x) * lim + pr(k, y)];
+    }
+  const long long q = pk(fj + x, fj + y);
+  a.f[q] = finit(a, q, x == y) + a.jrow[(long long)j * 10 + lane] + s + g;
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+__device__ __forceinline__ double wave_fmax(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// cnvg's diagonal steps (src/SCF/cnvg.F90:16-145, as in k_fock.hip) by one
+// wave; returns PL and the extrapolation factor.
+__device__ double2 cnvg_diag_wave(int n, double* __restrict__ pnew, double* __restrict__ pold,
+                                  double* __restrict__ p1, int niter, int lane) {
+  const double rhfuhf = 2.0;
+  const double damp = (niter > 3) ? 0.05 : 1.0e10;
+  const bool extrap = (niter % 3) != 0;
+  double sum1 = 0.0, pl = 0.0, faca = 0.0, facb = 0.0;
+  for (int i = lane; i < n; i += 64) {
+    const int k = tri(i) + i;
+    const double a = pnew[k], o = pold[k];
+    sum1 += a;
+    const double sa = fabs(a - o);
+    pl = fmax(pl, sa);
+    if (!extrap) {
+      faca += sa * sa;
+      const double t = a - 2.0 * o + p1[i];
+      facb += t * t;
+    }
+    p1[i] = o;
+    pold[k] = a;
+  }
+  sum1 = wave_sum(sum1);
+  pl = wave_fmax(pl);
+  faca = wave_sum(faca);
+  facb = wave_sum(facb);
+  double fac = 0.0;
+  if (facb > 1.0e-10 && faca < 100.0 * facb) fac = sqrt(faca / facb);
+  double sum2 = 0.0;
+  for (int i = lane; i < n; i += 64) {
+    const int k = tri(i) + i;
+    double v = pold[k];
+    const double o = p1[i];
+    if (fabs(v - o) > damp) v = o + ((v - o) >= 0.0 ? damp : -damp);
+    else v = v + fac * (v - o);
+    v = fmin(rhfuhf, fmax(v, 0.0));
+    pold[k] = v;
+    pnew[k] = v;
+    sum2 += v;
+  }
+  sum2 = wave_sum(sum2);
+  const double sum0 = sum1;
+  for (int it = 0; it < 1000; ++it) {
+    const double sc = (sum2 > 1.0e-3) ? sum1 / sum2 : 0.0;
+    sum1 = sum0;
+    if (sum2 < 1.0e-3 || fabs(sc - 1.0) < 1.0e-5) break;
+    double s2 = 0.0, nclamp = 0.0;
+    for (int i = lane; i < n; i += 64) {
+      const int k = tri(i) + i;
+      double v = fmax(pold[k] * sc + 1.0e-20, 0.0);
+      if (v > rhfuhf) {
+        v = rhfuhf;
+        nclamp += 1.0;
+      } else {
+        s2 += v;
+      }
+      pold[k] = v;
+      pnew[k] = v;
+    }
+    sum2 = wave_sum(s2);
+    sum1 -= rhfuhf * wave_sum(nclamp);
+  }
+  return make_double2(pl, fac);
+}
+
+// The SCF of molecule list[blockIdx.x] (entry 0 without a list), from the
+// state and densities in memory until it is done or `cap` Fock builds have
+// run.  No molecule waits for another: in lockstep, a launch per phase over
+// all molecules, every iteration took the longest eigensolve of its size
+// class and twenty launches, and 64 molecules took 109 ms where they now take
+// 15 (400: 137 -> 25, 4096: 403 -> 222).  With M.fexit, a finished molecule is
+// diagonalized once more to 1e-12, as iter does at its exit, and phase_lock'ed
+// if asked.
+template <int NT, bool LDS>
+__device__ __forceinline__ void scf_body(JacLds* lds, const FockArgs* __restrict__ args,
+                                         const BatchMol* __restrict__ mols, BatchState* __restrict__ st,
+                                         const int* __restrict__ list, double tol, int cap, int lock) {
+  constexpr int NW = NT / 64;
+  __shared__ BatchState s;
+  __shared__ double red[NW];
+  __shared__ double2 plfac;
+  const int m = list ? list[blockIdx.x] : 0;
+  const BatchMol M = mols[m];
+  FockArgs a = args[m];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = M.n;
+  auto eig = [&](double* f, bool warm, double t, bool density) {
+    if constexpr (LDS) return beig_lds(*lds, M, f, warm, t, density);
+    else return beig_global<NT>(M, f, warm, t, density);
+  };
+  if (tid == 0) s = st[m];
+  __shared__ int atom_of[kMaxLdsN];
+  if constexpr (LDS)
+    for (int i = tid; i < M.numat; i += NT)
+      for (int k = 0; k < a.sys.norb[i]; ++k) atom_of[a.sys.nf0[i] + k] = i;
+  __syncthreads();
+  for (int pass = 0; pass < cap; ++pass) {
+    if (s.done) break;
+    __syncthreads();
+    if (tid == 0) ctl_pre(s);
+    __syncthreads();
+    a.init_mode = s.mode;
+    a.shift = s.shift;
+    if constexpr (LDS) {
+      fock_small<NT>(a, atom_of, lds->m);
+    } else {
+      for (int i = M.numat - 1 - w; i >= 0; i -= NW) fock_rows_body<64>(a, i, lane);
+      __syncthreads();
+      for (int j = w; j < M.numat; j += NW) fock_cols_wave(a, j, lane);
+    }
+    __syncthreads();
+    double e = 0.0;
+    for (int r = w; r < n; r += NW)
+      for (int c = lane; c <= r; c += 64) {
+        const int q = tri(r) + c;
+        const double v = a.pa[q] * (a.h[q] + a.f[q]);
+        e += (c == r) ? 0.5 * v : v;
+      }
+    e = wave_sum(e);
+    if (lane == 0) red[w] = e;
+    __syncthreads();
+    if (tid == 0) {
+      e = red[0];
+      for (int i = 1; i < NW; ++i) e += red[i];
+      ctl_mid(s, 2.0 * e);
+    }
+    __syncthreads();
+    if (s.done) break;
+    if (!s.do_eig) continue;
+    const bool warm = s.have_c != 0;
+    double t = tol;
+    if (s.adaptive && s.pl > 10.0 * s.pltest) t = fmax(tol, fmin(1.0e-5, 1.0e-3 * s.pl));
+    const EigCount cnt = eig(M.f, warm, t, true);
+    __syncthreads();
+    eig_done(M, s, cnt, warm);
+    if (w == 0) {
+      const double2 r = cnvg_diag_wave(n, M.p, M.pold, M.p1, s.niter, lane);
+      if (lane == 0) plfac = r;
+    }
+    __syncthreads();
+    const double fac = plfac.y;
+    for (int r = w; r < n; r += NW)
+      for (int c = lane; c <= r; c += 64) {
+        const int q = tri(r) + c;
+        double v = M.p[q];
+        if (c < r) {
+          v += fac * (v - M.pold[q]);
+          M.pold[q] = v;
+          M.p[q] = v;
+        }
+        M.pa[q] = 0.5 * v;
+      }
+    if (tid == 0) ctl_post(s, M, plfac.x);
+    __syncthreads();
+  }
+  if (M.fexit && s.done && isfinite(s.ee)) {
+    for (int q = tid; q < tri(n); q += NT) M.fexit[q] = M.f[q];
+    __syncthreads();
+    const bool warm = s.have_c != 0;
+    const EigCount cnt = eig(M.fexit, warm, 1.0e-12, false);
+    __syncthreads();
+    eig_done(M, s, cnt, warm);
+    if (lock) {
+      // the largest coefficient of each column positive (the first of equals)
+      for (int col = w; col < n; col += NW) {
+        double* v = M.C + (size_t)col * (LDS ? SB : n);
+        double best = 0.0, sgn = 0.0;
+        int bi = n;
+        for (int r = lane; r < n; r += 64) {
+          const double x = fabs(v[r]);
+          if (x > best) { best = x; sgn = v[r]; bi = r; }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+          const double b2 = __shfl_xor(best, o, 64), s2 = __shfl_xor(sgn, o, 64);
+          const int i2 = __shfl_xor(bi, o, 64);
+          if (b2 > best || (b2 == best && i2 < bi)) { best = b2; sgn = s2; bi = i2; }
+        }
+        if (sgn < 0.0)
+          for (int r = lane; r < n; r += 64) v[r] = -v[r];
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) st[m] = s;
+}
+
+__global__ __launch_bounds__(kLdsThreads, 4) void k_bscf_lds(const FockArgs* __restrict__ args,
+                                                             const BatchMol* __restrict__ mols,
+                                                             BatchState* __restrict__ st,
+                                                             const int* __restrict__ list, double tol, int cap,
+                                                             int lock) {
+  __shared__ JacLds lds;
+  scf_body<kLdsThreads, true>(&lds, args, mols, st, list, tol, cap, lock);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_bscf(const FockArgs* __restrict__ args, const BatchMol* __restrict__ mols,
+                                             BatchState* __restrict__ st, const int* __restrict__ list, double tol,
+                                             int cap, int lock) {
+  scf_body<NT, false>(nullptr, args, mols, st, list, tol, cap, lock);
+}
+
+// The starting densities (iter.F90:269-300): P the atoms' diagonal, Pa its
+// share of one spin, the previous density and diagonal those of Pa.
+__global__ __launch_bounds__(256) void k_binit(const BatchMol* __restrict__ mols, const double* __restrict__ pdiag,
+                                               const long long* __restrict__ orb_off, int* __restrict__ act,
+                                               int* __restrict__ do_eig) {
+  const BatchMol M = mols[blockIdx.x];
+  if (threadIdx.x == 0) act[blockIdx.x] = do_eig[blockIdx.x] = 0;
+  const double* d = pdiag + orb_off[blockIdx.x];
+  const double w1 = M.nocc / (M.nocc + 1.0e-6 + M.nocc), share = w1 < 1e-6 ? 0.5 : w1;
+  for (int q = threadIdx.x; q < tri(M.n); q += 256) {
+    const int r = tri_row(q);
+    const double v = q == tri(r) + r ? d[r] : 0.0;
+    M.p[q] = v;
+    M.pa[q] = M.pold[q] = v * share;
+  }
+  for (int i = threadIdx.x; i < M.n; i += 256) M.p1[i] = d[i] * share;
 }
 
 // Pa = P / 2 for the molecules that stepped
@@ -758,141 +880,118 @@ struct mhip_batch {
   DevBuf w, h, f, p, pa, pold, p1, C, A, T, eig, jrow, jcol;
   DevBuf nf0, norb, woff, wcum, w1off, ccol, heavy, light, nhb, nlb;
   DevBuf args, mols, cnv, st, act, doeig, mode, niter, shift, ee, partial, scal, orboff;
-  std::vector<double> p0, pa0, p1h;  // starting densities, restored by every run
+  DevBuf pdiag, st0;  // starting diagonals and control states, where every run begins
+  hipStream_t cs[4] = {};  // a stream per size class: the classes fill each other's tails
+  hipEvent_t ev[5] = {};
   DevBuf atom_mol, atom_idx, row_mol, row_idx;
   int n_atom_blk = 0, n_row_blk = 0;
   // molecules by eigensolver class (workgroup size), in launch order
   std::vector<int> cls_count, cls_nmax;
-  int eig_form[4] = {0, 0, 0, 0};  // 0 global, 1 A in LDS, 2 A and C in LDS
-  size_t eig_lds[4] = {0, 0, 0, 0};
+  BatchJacobi* bj = nullptr;         // the classes above kMaxLdsN
+  int small_atoms = 0, small_rows = 0;  // workgroups of the others in the atom and row lists, which they begin
   bool force_global_eig = false;
   DevBuf cls_list;
   int tile[4] = {64, 128, 256, 256};   // workgroup size per class (n <= 32, 64, 128, 256)
   double tol = 1.0e-10;
   std::vector<BatchState> init_state;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
   // eager timing of the eigensolver launches per size class
   hipEvent_t eig_ev[4][2] = {};
   bool eig_timing = false;
-  int graph_iters = 0;
 };
 
 namespace {
 
 int size_class(int n) { return n <= 32 ? 0 : (n <= 64 ? 1 : (n <= 128 ? 2 : 3)); }
 
-// LDS bytes a workgroup can take beyond the kernel's static arrays
-size_t lds_room(const void* fn) {
-  int dev = 0, lds_max = 0;
-  MHIP_CHECK(hipGetDevice(&dev));
-  MHIP_CHECK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  hipFuncAttributes fa{};
-  MHIP_CHECK(hipFuncGetAttributes(&fa, fn));
-  return lds_max > (int)fa.sharedSizeBytes ? (size_t)lds_max - fa.sharedSizeBytes : 0;
-}
-
-// Eigensolver form of a size class (its largest n, workgroup size NT): A and
-// C in LDS when both fit (2), else A in LDS (1), else the global-memory
-// kernel (0); the LDS forms get their dynamic LDS limit raised here, before
-// any capture.  Returns the form and sets the dynamic LDS bytes.
-template <int NT>
-int plan_beig(int nmax, size_t* lds) {
-  const size_t np = (size_t)((nmax + 1) & ~1);
-  const size_t a = sizeof(double) * (np * (np + 1) / 2), c = sizeof(double) * (size_t)nmax * nmax;
-  const void* f2 = (const void*)k_beig_lds<NT, true>;
-  const void* f1 = (const void*)k_beig_lds<NT, false>;
-  if (a + c <= lds_room(f2)) {
-    MHIP_CHECK(hipFuncSetAttribute(f2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(a + c)));
-    *lds = a + c;
-    return 2;
-  }
-  if (a <= lds_room(f1)) {
-    MHIP_CHECK(hipFuncSetAttribute(f1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)a));
-    *lds = a;
-    return 1;
-  }
-  *lds = 0;
-  return 0;
-}
-
-template <int NT>
-void launch_beig(hipStream_t s, int form, size_t lds, int nblk, const BatchMol* mols, const int* doeig,
-                 BatchState* st, const int* list, double tol) {
-  const int room = (int)(lds / sizeof(double));
-  if (form == 2)
-    hipLaunchKernelGGL((k_beig_lds<NT, true>), dim3(nblk), dim3(NT), lds, s, mols, doeig, st, list, tol, room);
-  else if (form == 1)
-    hipLaunchKernelGGL((k_beig_lds<NT, false>), dim3(nblk), dim3(NT), lds, s, mols, doeig, st, list, tol, room);
-  else
-    hipLaunchKernelGGL(k_beig<NT>, dim3(nblk), dim3(NT), 0, s, mols, doeig, st, list, tol);
-  MHIP_LAUNCH_CHECK();
-}
-
-void plan_eig_classes(mhip_batch* b) {
-  for (int c = 0; c < 4; ++c) {
-    size_t lds = 0;
-    int form = 0;
-    if (b->cls_nmax[c] > 0) {
-      switch (b->tile[c]) {
-        case 64: form = plan_beig<64>(b->cls_nmax[c], &lds); break;
-        case 128: form = plan_beig<128>(b->cls_nmax[c], &lds); break;
-        case 512: form = plan_beig<512>(b->cls_nmax[c], &lds); break;
-        case 1024: form = plan_beig<1024>(b->cls_nmax[c], &lds); break;
-        default: form = plan_beig<256>(b->cls_nmax[c], &lds); break;
-      }
-    }
-    b->eig_form[c] = b->force_global_eig ? 0 : form;
-    b->eig_lds[c] = b->force_global_eig ? 0 : lds;
+// fn(std::integral_constant<int, NT>) for the workgroup size `tile`
+template <class F>
+void with_tile(int tile, F&& fn) {
+  switch (tile) {
+    case 64: fn(std::integral_constant<int, 64>()); break;
+    case 128: fn(std::integral_constant<int, 128>()); break;
+    case 512: fn(std::integral_constant<int, 512>()); break;
+    case 1024: fn(std::integral_constant<int, 1024>()); break;
+    default: fn(std::integral_constant<int, 256>()); break;
   }
 }
 
+// Classes 0 and 1 in LDS, a workgroup to a molecule; with the matrices in
+// memory (the comparison form) every class.
 void launch_eig_class(mhip_batch* b, int cls, int offset, int count) {
   if (count <= 0) return;
-  const int* list = b->cls_list.as<int>() + offset;
   auto* mols = b->mols.as<BatchMol>();
   auto* st = b->st.as<BatchState>();
+  const int* list = b->cls_list.as<int>() + offset;
   const int* de = b->doeig.as<int>();
-  const int f = b->eig_form[cls];
-  const size_t l = b->eig_lds[cls];
-  switch (b->tile[cls]) {
-    case 64: launch_beig<64>(b->s, f, l, count, mols, de, st, list, b->tol); break;
-    case 128: launch_beig<128>(b->s, f, l, count, mols, de, st, list, b->tol); break;
-    case 512: launch_beig<512>(b->s, f, l, count, mols, de, st, list, b->tol); break;
-    case 1024: launch_beig<1024>(b->s, f, l, count, mols, de, st, list, b->tol); break;
-    default: launch_beig<256>(b->s, f, l, count, mols, de, st, list, b->tol); break;
-  }
+  if (!b->force_global_eig)
+    hipLaunchKernelGGL(k_beig_lds, dim3(count), dim3(kLdsThreads), 0, b->s, mols, de, st, list, b->tol);
+  else
+    with_tile(b->tile[cls], [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      hipLaunchKernelGGL(k_beig<NT>, dim3(count), dim3(NT), 0, b->s, mols, de, st, list, b->tol);
+    });
+  MHIP_LAUNCH_CHECK();
 }
 
-void one_iteration(mhip_batch* b) {
+void launch_scf_class(mhip_batch* b, hipStream_t s, int cls, int offset, int cap) {
+  auto* args = b->args.as<FockArgs>();
+  auto* mols = b->mols.as<BatchMol>();
+  auto* st = b->st.as<BatchState>();
+  const int* list = b->cls_list.as<int>() + offset;
+  const int n = b->cls_count[cls];
+  if (!b->force_global_eig)
+    hipLaunchKernelGGL(k_bscf_lds, dim3(n), dim3(kLdsThreads), 0, s, args, mols, st, list, b->tol, cap, 0);
+  else
+    with_tile(b->tile[cls], [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      hipLaunchKernelGGL(k_bscf<NT>, dim3(n), dim3(NT), 0, s, args, mols, st, list, b->tol, cap, 0);
+    });
+  MHIP_LAUNCH_CHECK();
+}
+
+// One iteration of every molecule (the eigensolver profile), or of those of
+// the block-Jacobi classes alone (big_only), a launch per phase over all of
+// them; returns how many of the latter are not done.
+int one_iteration(mhip_batch* b, bool big_only) {
   hipStream_t s = b->s;
-  const int nm = b->nmol;
+  const int l0 = big_only ? b->cls_count[0] + b->cls_count[1] : 0, nm = b->nmol - l0;
+  const int a0 = big_only ? b->small_atoms : 0, na = b->n_atom_blk - a0;
+  const int r0 = big_only ? b->small_rows : 0, nr = b->n_row_blk - r0;
+  const int* list = b->cls_list.as<int>() + l0;
+  const int* row_mol = b->row_mol.as<int>() + r0;
+  const int* row_idx = b->row_idx.as<int>() + r0;
   const int cb = cdiv(nm, 64);
-  hipLaunchKernelGGL(k_bctl_pre, dim3(cb), dim3(64), 0, s, nm, b->st.as<BatchState>(), b->act.as<int>(),
+  hipLaunchKernelGGL(k_bctl_pre, dim3(cb), dim3(64), 0, s, nm, list, b->st.as<BatchState>(), b->act.as<int>(),
                      b->mode.as<int>(), b->niter.as<int>(), b->shift.as<double>());
   MHIP_LAUNCH_CHECK();
-  fock_build_batch(s, b->args.as<FockArgs>(), b->n_atom_blk, b->atom_mol.as<int>(), b->atom_idx.as<int>(),
+  fock_build_batch(s, b->args.as<FockArgs>(), na, b->atom_mol.as<int>() + a0, b->atom_idx.as<int>() + a0,
                    b->act.as<int>(), b->mode.as<int>(), b->shift.as<double>());
-  helect_batch(s, b->args.as<FockArgs>(), nm, b->n_row_blk, b->row_mol.as<int>(), b->row_idx.as<int>(),
-               b->act.as<int>(), b->orboff.as<long long>(), b->partial.as<double>(), 2.0, b->ee.as<double>());
-  hipLaunchKernelGGL(k_bctl_mid, dim3(cb), dim3(64), 0, s, nm, b->st.as<BatchState>(), b->ee.as<double>(),
+  helect_batch(s, b->args.as<FockArgs>(), b->nmol, nr, row_mol, row_idx, b->act.as<int>(),
+               b->orboff.as<long long>(), b->partial.as<double>(), 2.0, b->ee.as<double>());
+  hipLaunchKernelGGL(k_bctl_mid, dim3(cb), dim3(64), 0, s, nm, list, b->st.as<BatchState>(), b->ee.as<double>(),
                      b->doeig.as<int>());
   MHIP_LAUNCH_CHECK();
-  int off = 0;
-  for (int c = 0; c < 4; ++c) {
+  int open = 0, off = 0;
+  for (int c = big_only ? 2 : 0; c < 4; ++c) {
     if (b->eig_timing) MHIP_CHECK(hipEventRecord(b->eig_ev[c][0], s));
-    launch_eig_class(b, c, off, b->cls_count[c]);
+    if (c < 2 || b->force_global_eig) launch_eig_class(b, c, off, b->cls_count[c]);
+    else if (b->bj && (!big_only || c == 2))
+      // by itself only for its own time
+      open += bj_solve(b->bj, s, b->st.as<BatchState>(), b->doeig.as<int>(), b->tol, big_only || c == 2 ? 128 : 192,
+                       !big_only && c == 2 ? 128 : 256);
     if (b->eig_timing) MHIP_CHECK(hipEventRecord(b->eig_ev[c][1], s));
     off += b->cls_count[c];
   }
-  cnvg_batch(s, b->cnv.as<BatchCnvg>(), nm, b->n_row_blk, b->row_mol.as<int>(), b->row_idx.as<int>(),
-             b->doeig.as<int>(), b->niter.as<int>(), b->scal.as<double>());
-  hipLaunchKernelGGL(k_bctl_post, dim3(cb), dim3(64), 0, s, nm, b->mols.as<BatchMol>(), b->st.as<BatchState>(),
+  if (big_only && open == 0) return 0;
+  cnvg_batch(s, b->cnv.as<BatchCnvg>(), b->nmol, nr, row_mol, row_idx, b->doeig.as<int>(), b->niter.as<int>(),
+             b->scal.as<double>());
+  hipLaunchKernelGGL(k_bctl_post, dim3(cb), dim3(64), 0, s, nm, list, b->mols.as<BatchMol>(), b->st.as<BatchState>(),
                      b->doeig.as<int>(), b->scal.as<double>());
   MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bhalf, dim3(b->n_row_blk), dim3(256), 0, s, b->mols.as<BatchMol>(), b->row_mol.as<int>(),
-                     b->row_idx.as<int>(), b->doeig.as<int>());
+  hipLaunchKernelGGL(k_bhalf, dim3(nr), dim3(256), 0, s, b->mols.as<BatchMol>(), row_mol, row_idx,
+                     b->doeig.as<int>());
   MHIP_LAUNCH_CHECK();
+  return open;
 }
 
 template <class F>
@@ -908,6 +1007,35 @@ int bguard(F&& fn) {
 
 }  // namespace
 
+namespace mhip {
+
+BatchState batch_start(double enuclr, double atheat, double scfcrt, int itrmax) {
+  BatchState z{};
+  z.itrmax = itrmax > 0 ? itrmax : 2000;
+  z.ten = -80.0;
+  z.shift = 1.0;
+  z.shfmax = 20.0;
+  z.pl = 1.0;
+  z.eold = 100.0;
+  z.iredy = 1;
+  z.enuclr = enuclr;
+  z.atheat = atheat;
+  const double scf = std::max(scfcrt > 0 ? scfcrt : 1.0e-4, 1e-12);
+  z.selcon = std::min(std::min(scf * 100.0, 0.1), scf);
+  z.pltest = 0.05 * std::sqrt(std::fabs(z.selcon));
+  return z;
+}
+
+bool scf_one_workgroup(hipStream_t s, int n, const FockArgs* args, const BatchMol* mol, BatchState* st, double tol,
+                       int phase_lock) {
+  if (n > kMaxLdsN) return false;
+  hipLaunchKernelGGL(k_bscf_lds, dim3(1), dim3(kLdsThreads), 0, s, args, mol, st, nullptr, tol, INT_MAX, phase_lock);
+  MHIP_LAUNCH_CHECK();
+  return true;
+}
+
+}  // namespace mhip
+
 extern "C" {
 
 int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** out) {
@@ -916,6 +1044,8 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     auto* b = new mhip_batch();
     b->nmol = nmol;
     MHIP_CHECK(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking));
+    for (auto& c : b->cs) MHIP_CHECK(hipStreamCreateWithFlags(&c, hipStreamNonBlocking));
+    for (auto& e : b->ev) MHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // ---- host tables, then one upload per array
     std::vector<long long> o_w(nmol), o_mp(nmol), o_nn(nmol), o_n(nmol), o_at(nmol), o_cc(nmol), o_a(nmol);
     long long tw = 0, tmp = 0, tnn = 0, tn = 0, tat = 0, tcc = 0, ta = 0;
@@ -962,14 +1092,9 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
       MHIP_REQUIRE(nf0_all.back() + norb_all.back() == n, "mhip_batch_create: nlast(numat) != norbs");
       tw += kr;
       tmp += (long long)n * (n + 1) / 2;
-      tnn += (long long)n * n;
-      {
-        // the eigensolver's A: n x n (global form), or the LDS form's
-        // rotation log of one sweep and parked A
-        const long long np = (n + 1) & ~1;
-        o_a[m] = ta;
-        ta += std::max((long long)n * n, np * (np - 1) + np * (np + 1) / 2);
-      }
+      tnn += std::max<long long>((long long)n * n, SB * SB);  // the LDS form's C is padded
+      o_a[m] = ta;
+      ta += (long long)n * n;
       tn += n;
       tat += na;
       tcc += std::max(cc, 1LL);
@@ -1018,6 +1143,21 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     upv(b->light, light_all.data(), sizeof(int) * light_all.size());
     upv(b->nhb, nhb_all.data(), sizeof(int) * nhb_all.size());
     upv(b->nlb, nlb_all.data(), sizeof(int) * nlb_all.size());
+    // molecules grouped by eigensolver class
+    std::vector<int> order;
+    b->cls_count.assign(4, 0);
+    b->cls_nmax.assign(4, 0);
+    for (int c = 0; c < 4; ++c)
+      for (int m = 0; m < nmol; ++m)
+        if (size_class(b->n_h[m]) == c) {
+          order.push_back(m);
+          b->cls_count[c]++;
+          b->cls_nmax[c] = std::max(b->cls_nmax[c], b->n_h[m]);
+        }
+    // the largest of each class first: they take the longest
+    for (int c = 0, o = 0; c < 4; o += b->cls_count[c++])
+      std::stable_sort(order.begin() + o, order.begin() + o + b->cls_count[c],
+                       [&](int x, int y) { return b->n_h[x] > b->n_h[y]; });
     // per-molecule argument blocks
     std::vector<FockArgs> args(nmol);
     std::vector<BatchMol> bm(nmol);
@@ -1025,8 +1165,7 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     std::vector<long long> orboff(nmol);
     std::vector<int> atom_mol, atom_idx, row_mol, row_idx;
     b->init_state.resize(nmol);
-    // initial densities (iter.F90:269-300 with pdiag)
-    std::vector<double> p0(tmp, 0.0), pa0(tmp, 0.0), p1h(tn, 0.0);
+    std::vector<double> pdiag;
     for (int m = 0; m < nmol; ++m) {
       const mhip_batch_molecule& M = mols[m];
       const int n = M.norbs;
@@ -1067,35 +1206,23 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
       q.eig = b->eig.as<double>() + o_n[m];
       cv[m] = BatchCnvg{n, q.p, q.pold, q.p1};
       orboff[m] = o_n[m];
-      for (int i = 0; i < M.numat; ++i) {
+      pdiag.insert(pdiag.end(), M.pdiag, M.pdiag + n);
+      b->init_state[m] = batch_start(M.enuclr, M.atheat, M.scfcrt, M.itrmax);
+    }
+    for (int k = 0; k < nmol; ++k) {
+      const int m = order[k];
+      if (k == b->cls_count[0] + b->cls_count[1]) {
+        b->small_atoms = (int)atom_mol.size();
+        b->small_rows = (int)row_mol.size();
+      }
+      for (int i = 0; i < mols[m].numat; ++i) {
         atom_mol.push_back(m);
         atom_idx.push_back(i);
       }
-      for (int r = 0; r < n; ++r) {
+      for (int r = 0; r < mols[m].norbs; ++r) {
         row_mol.push_back(m);
         row_idx.push_back(r);
       }
-      const double w1 = M.nclose / (M.nclose + 1.0e-6 + M.nclose);
-      for (int i = 0; i < n; ++i) {
-        const long long d = o_mp[m] + (long long)i * (i + 1) / 2 + i;
-        p0[d] = M.pdiag[i];
-        pa0[d] = M.pdiag[i] * (w1 < 1e-6 ? 0.5 : w1);
-        p1h[o_n[m] + i] = pa0[d];  // pold2 = diagonal of pold (= Pa)
-      }
-      BatchState& z = b->init_state[m];
-      z = BatchState{};
-      z.itrmax = M.itrmax > 0 ? M.itrmax : 2000;
-      z.ten = -80.0;
-      z.shift = 1.0;
-      z.shfmax = 20.0;
-      z.pl = 1.0;
-      z.eold = 100.0;
-      z.iredy = 1;
-      z.enuclr = M.enuclr;
-      z.atheat = M.atheat;
-      const double scf = std::max(M.scfcrt > 0 ? M.scfcrt : 1.0e-4, 1e-12);
-      z.selcon = std::min(std::min(scf * 100.0, 0.1), scf);
-      z.pltest = 0.05 * std::sqrt(std::fabs(z.selcon));
     }
     b->n_atom_blk = (int)atom_mol.size();
     b->n_row_blk = (int)row_mol.size();
@@ -1112,24 +1239,12 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     for (DevBuf* x : {&b->shift, &b->ee}) x->ensure(sizeof(double) * nmol);
     b->scal.ensure(sizeof(double) * 2 * nmol);
     b->partial.ensure(sizeof(double) * tn);
-    // the starting P, Pa, Pold, p1, uploaded by every mhip_batch_run
-    b->p0 = std::move(p0);
-    b->pa0 = std::move(pa0);
-    b->p1h = std::move(p1h);
-    // molecules grouped by eigensolver class
-    std::vector<int> order;
-    b->cls_count.assign(4, 0);
-    b->cls_nmax.assign(4, 0);
-    for (int c = 0; c < 4; ++c)
-      for (int m = 0; m < nmol; ++m)
-        if (size_class(b->n_h[m]) == c) {
-          order.push_back(m);
-          b->cls_count[c]++;
-          b->cls_nmax[c] = std::max(b->cls_nmax[c], b->n_h[m]);
-        }
+    upv(b->pdiag, pdiag.data(), sizeof(double) * tn);
+    upv(b->st0, b->init_state.data(), sizeof(BatchState) * nmol);
     upv(b->cls_list, order.data(), sizeof(int) * nmol);
-    plan_eig_classes(b);
-    MHIP_CHECK(hipStreamSynchronize(s));
+    const std::vector<int> big(order.begin() + b->cls_count[0] + b->cls_count[1], order.end());
+    if (!big.empty()) b->bj = bj_create(bm, big);
+    MHIP_CHECK(hipStreamSynchronize(s));  // the host vectors go out of scope
     *out = b;
   });
 }
@@ -1142,13 +1257,6 @@ int mhip_batch_set_tiles(mhip_batch* b, const int* tiles) {
                    "mhip_batch_set_tiles: workgroup sizes are 64, 128, 256, 512 or 1024");
       b->tile[c] = tiles[c];
     }
-    plan_eig_classes(b);
-    if (b->exec) {
-      (void)hipGraphExecDestroy(b->exec);
-      (void)hipGraphDestroy(b->graph);
-      b->exec = nullptr;
-      b->graph = nullptr;
-    }
   });
 }
 
@@ -1156,26 +1264,15 @@ int mhip_batch_set_eig_lds(mhip_batch* b, int lds) {
   return bguard([&] {
     MHIP_REQUIRE(b, "mhip_batch_set_eig_lds: bad arguments");
     b->force_global_eig = lds == 0;
-    plan_eig_classes(b);
-    if (b->exec) {
-      (void)hipGraphExecDestroy(b->exec);
-      (void)hipGraphDestroy(b->graph);
-      b->exec = nullptr;
-      b->graph = nullptr;
-    }
   });
 }
 
 // the per-molecule state and the starting densities, before a run
 static void reset_batch(mhip_batch* b) {
-  hipStream_t s = b->s;
-  MHIP_CHECK(hipMemcpyAsync(b->st.ptr, b->init_state.data(), sizeof(BatchState) * b->nmol,
-                            hipMemcpyHostToDevice, s));
-  MHIP_CHECK(hipMemcpyAsync(b->p.ptr, b->p0.data(), sizeof(double) * b->p0.size(), hipMemcpyHostToDevice, s));
-  MHIP_CHECK(hipMemcpyAsync(b->pa.ptr, b->pa0.data(), sizeof(double) * b->pa0.size(), hipMemcpyHostToDevice, s));
-  MHIP_CHECK(hipMemcpyAsync(b->pold.ptr, b->pa0.data(), sizeof(double) * b->pa0.size(), hipMemcpyHostToDevice, s));
-  MHIP_CHECK(hipMemcpyAsync(b->p1.ptr, b->p1h.data(), sizeof(double) * b->p1h.size(), hipMemcpyHostToDevice, s));
-  MHIP_CHECK(hipStreamSynchronize(s));
+  MHIP_CHECK(hipMemcpyAsync(b->st.ptr, b->st0.ptr, sizeof(BatchState) * b->nmol, hipMemcpyDeviceToDevice, b->s));
+  hipLaunchKernelGGL(k_binit, dim3(b->nmol), dim3(256), 0, b->s, b->mols.as<BatchMol>(), b->pdiag.as<double>(),
+                     b->orboff.as<long long>(), b->act.as<int>(), b->doeig.as<int>());
+  MHIP_LAUNCH_CHECK();
 }
 
 int mhip_batch_eig_profile(mhip_batch* b, int iters, double* ms, double* flops, long long* rotations) {
@@ -1203,7 +1300,7 @@ int mhip_batch_eig_profile(mhip_batch* b, int iters, double* ms, double* flops, 
       }
     } off{b};
     for (int it = 0; it < iters; ++it) {
-      one_iteration(b);
+      one_iteration(b, false);
       MHIP_CHECK(hipStreamSynchronize(s));
       for (int c = 0; c < 4; ++c) {
         float t = 0.0f;
@@ -1221,35 +1318,34 @@ int mhip_batch_eig_profile(mhip_batch* b, int iters, double* ms, double* flops, 
   });
 }
 
-// Run the batched SCF from the starting densities: capture `iters`
-// iterations once into a graph, replay it until every molecule is done.
+// Run the batched SCF from the starting densities, at most iters_per_graph *
+// max_launches iterations (and recomputed Fock builds) of each molecule.
 int mhip_batch_run(mhip_batch* b, int iters_per_graph, int max_launches, double* seconds, int* n_converged) {
   return bguard([&] {
     MHIP_REQUIRE(b && iters_per_graph > 0 && max_launches > 0, "mhip_batch_run: bad arguments");
     hipStream_t s = b->s;
+    const int cap = (int)std::min<long long>((long long)iters_per_graph * max_launches, 1 << 30);
     reset_batch(b);
-    if (!b->exec || b->graph_iters != iters_per_graph) {
-      if (b->exec) {
-        (void)hipGraphExecDestroy(b->exec);
-        (void)hipGraphDestroy(b->graph);
-      }
-      MHIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      for (int it = 0; it < iters_per_graph; ++it) one_iteration(b);
-      MHIP_CHECK(hipStreamEndCapture(s, &b->graph));
-      MHIP_CHECK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-      b->graph_iters = iters_per_graph;
-    }
+    MHIP_CHECK(hipStreamSynchronize(s));
     const auto t0 = std::chrono::steady_clock::now();
-    std::vector<BatchState> hs(b->nmol);
-    int done = 0;
-    for (int l = 0; l < max_launches; ++l) {
-      MHIP_CHECK(hipGraphLaunch(b->exec, s));
-      MHIP_CHECK(hipMemcpyAsync(hs.data(), b->st.ptr, sizeof(BatchState) * b->nmol, hipMemcpyDeviceToHost, s));
-      MHIP_CHECK(hipStreamSynchronize(s));
-      done = 0;
-      for (const auto& z : hs) done += z.done ? 1 : 0;
-      if (done == b->nmol) break;
+    MHIP_CHECK(hipEventRecord(b->ev[4], s));
+    // small molecules: each class on a stream of its own, a workgroup for
+    // every molecule from start to end; beside them the block-Jacobi classes,
+    // an iteration at a time
+    const int one_wg = b->force_global_eig ? 4 : 2;
+    for (int c = 0, off = 0; c < one_wg; off += b->cls_count[c++]) {
+      if (b->cls_count[c] == 0) continue;
+      MHIP_CHECK(hipStreamWaitEvent(b->cs[c], b->ev[4], 0));
+      launch_scf_class(b, b->cs[c], c, off, cap);
+      MHIP_CHECK(hipEventRecord(b->ev[c], b->cs[c]));
     }
+    if (b->bj && one_wg == 2)
+      for (int it = 0; it < cap && one_iteration(b, true) > 0; ++it) {}
+    for (int c = 0; c < one_wg; ++c)
+      if (b->cls_count[c]) MHIP_CHECK(hipStreamWaitEvent(s, b->ev[c], 0));
+    std::vector<BatchState> hs(b->nmol);
+    MHIP_CHECK(hipMemcpyAsync(hs.data(), b->st.ptr, sizeof(BatchState) * b->nmol, hipMemcpyDeviceToHost, s));
+    MHIP_CHECK(hipStreamSynchronize(s));
     const auto t1 = std::chrono::steady_clock::now();
     if (seconds) *seconds = std::chrono::duration<double>(t1 - t0).count();
     if (n_converged) {
@@ -1285,13 +1381,14 @@ int mhip_batch_density(mhip_batch* b, int m, double* p) {
 void mhip_batch_destroy(mhip_batch* b) {
   if (!b) return;
   (void)hipStreamSynchronize(b->s);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+  bj_destroy(b->bj);
+  for (auto c : b->cs) (void)hipStreamDestroy(c);
+  for (auto e : b->ev) (void)hipEventDestroy(e);
   for (DevBuf* x : {&b->w, &b->h, &b->f, &b->p, &b->pa, &b->pold, &b->p1, &b->C, &b->A, &b->T, &b->eig, &b->jrow,
                     &b->jcol, &b->nf0, &b->norb, &b->woff, &b->wcum, &b->w1off, &b->ccol, &b->heavy, &b->light,
                     &b->nhb, &b->nlb, &b->args, &b->mols, &b->cnv, &b->st, &b->act, &b->doeig, &b->mode, &b->niter,
                     &b->shift, &b->ee, &b->partial, &b->scal, &b->orboff, &b->atom_mol, &b->atom_idx,
-                    &b->row_mol, &b->row_idx, &b->cls_list})
+                    &b->row_mol, &b->row_idx, &b->cls_list, &b->pdiag, &b->st0})
     x->release();
   (void)hipStreamDestroy(b->s);
   delete b;

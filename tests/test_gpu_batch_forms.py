@@ -1,0 +1,86 @@
+"""The batched SCF's two forms at the edges of their ranges: one workgroup for
+a molecule up to 64 orbitals, block-Jacobi steps over several above (padded
+sizes 128, 192 and 256), and the single-molecule SCF that shares the first."""
+import numpy as np
+import pytest
+
+from mopac_gpu_amd import batch as B
+from mopac_gpu_amd import geometry, hamiltonian
+from mopac_gpu_amd.scf import Context
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+# 6 to 254 orbitals, on both sides of and at 32, 64, 128 and 192
+MOLS = [("water", 1), ("alkane", 1), ("water", 5), ("alkane", 5), ("water", 6), ("alkane", 10), ("helix", 3),
+        ("water", 11), ("alkane", 20), ("alkane", 21), ("water", 22), ("alkane", 31), ("water", 32), ("water", 33),
+        ("alkane", 42)]
+MAKE = {"water": geometry.water_cluster, "alkane": geometry.alkane, "helix": geometry.glycine_helix}
+
+
+@pytest.fixture(scope="module")
+def systems():
+    return [hamiltonian.build(*MAKE[kind](size, 17)) for kind, size in MOLS]
+
+
+@pytest.fixture(scope="module")
+def edge_batch(systems):
+    b = B.Batch(systems, scfcrt=1e-6)
+    yield b
+    b.close()
+
+
+def test_every_size_matches_the_oracle(systems, edge_batch):
+    edge_batch.run()
+    escf, niter, conv = edge_batch.results()
+    assert conv.all()
+    for m, s in enumerate(systems):
+        o = oracle.iterate(s, scfcrt=1e-6)
+        assert int(niter[m]) == o["niter"], (MOLS[m], niter[m], o["niter"])
+        assert abs(escf[m] - o["escf"]) < 1e-6 * max(1.0, abs(o["escf"])), MOLS[m]
+        assert np.max(np.abs(edge_batch.density(m) - o["p"])) < 1e-6, MOLS[m]
+
+
+def test_iteration_limit_stops_both_forms(systems, edge_batch):
+    """Three iterations are the same three in either eigensolver form, and a
+    second run starts over."""
+    edge_batch.run(iters_per_graph=3, max_launches=1)
+    e1, n1, c1 = edge_batch.results()
+    edge_batch.set_eig_lds(False)
+    edge_batch.run(iters_per_graph=1, max_launches=3)
+    e2, n2, c2 = edge_batch.results()
+    edge_batch.set_eig_lds(True)
+    assert not c1.any() and not c2.any()
+    assert (n1 == n2).all() and (n1 <= 3).all()
+    assert np.max(np.abs(e1 - e2) / np.maximum(1.0, np.abs(e1))) < 1e-9
+    edge_batch.run()
+    assert edge_batch.results()[2].all()
+
+
+@pytest.mark.parametrize("m", range(7))
+def test_single_molecule_in_one_workgroup_matches_the_general_path(systems, m):
+    s = systems[m]
+    assert s.norbs <= 64
+    kw = dict(scfcrt=1e-6, want=("p", "f", "c", "eig"))
+    out = []
+    for inner in (0, 16):  # a chosen inner sweep count takes the general path
+        ctx = Context(0)
+        ctx.lib.mhip_set_tuning(ctx.h, -1, inner, -1.0)
+        ctx.upload(s)
+        out.append((ctx.iter(**kw), ctx.iter(itrmax=4, **kw)))
+        ctx.close()
+    (a, few), (b, few_b) = out
+    assert a["converged"] and b["converged"] and a["niter"] == b["niter"]
+    assert few["niter"] == few_b["niter"] and few["converged"] == few_b["converged"]
+    assert abs(a["escf"] - b["escf"]) < 1e-7 * max(1.0, abs(b["escf"]))
+    # the in-loop eigensolves stop at residuals of 1e-10, which the densities'
+    # differences carry over gaps of tenths of eV and the iterations left
+    for k in ("p", "f", "eig"):
+        assert np.max(np.abs(a[k] - b[k])) < 1e-7, k
+    # the eigenvectors of the exit diagonalization: orthonormal, and F's own
+    n = s.norbs
+    f = np.zeros((n, n))
+    f[np.tril_indices(n)] = a["f"]
+    f = f + np.tril(f, -1).T
+    assert np.max(np.abs(a["c"].T @ a["c"] - np.eye(n))) < 1e-11
+    assert np.max(np.abs(f @ a["c"] - a["c"] * a["eig"])) < 1e-8  # F(i,i) + i*1e-10 is what is diagonalized
