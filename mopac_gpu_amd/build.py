@@ -28,6 +28,7 @@ SOURCES = [
     "k_batch.hip",
     "k_batch_eig.hip",
     "k_guess.hip",
+    "pitched.hip",
     "mozyme_scf.hip",
     "k_mozyme.hip",
     "scf_driver.hip",

@@ -11,6 +11,7 @@
 #include "k_guess.h"
 #include "k_occvirt.h"
 #include "k_pseudo.h"
+#include "pitched.h"
 
 namespace mhip {
 struct MzFock;  // MOZYME sparse Fock build state (mozyme_scf.hip)
@@ -45,6 +46,7 @@ struct mhip_ctx {
   double* hscal = nullptr;  // pinned host scalars
   void* hstage = nullptr;   // pinned staging for result downloads (grow-only)
   size_t hstage_bytes = 0;
+  mhip::PitchedCopy pitched;  // eigenvectors to and from the caller
   // pseudo-diagonalization workspace
   mhip::PseudoWork pseudo;
   mhip::OccVirtWork ov;

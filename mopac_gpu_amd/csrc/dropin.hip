@@ -9,6 +9,7 @@
 #include "common.h"
 #include "k_eigen.h"
 #include "k_pseudo.h"
+#include "pitched.h"
 
 namespace mhip {
 namespace {
@@ -23,6 +24,7 @@ struct Implicit {
   DevBuf scal;
 };
 Implicit g_imp;
+PitchedCopy g_pitched;        // held with g_mu
 std::mutex g_mu;
 int g_selected_device = 0;    // set by mhip_setDevice
 int g_pair[2] = {0, 1};       // mhip_set_mozyme_gpu_pair (recorded; one GPU is used)
@@ -35,6 +37,7 @@ void release_implicit() {
                     &g_imp.scal})
     b->release();
   g_imp.plan.release();
+  g_pitched.release();
   release_split_scratch(g_imp.s);
   release_splitk_scratch(g_imp.s);
   if (g_imp.hs) (void)hipHostFree(g_imp.hs);
@@ -61,8 +64,7 @@ Implicit& imp() {
 
 void h2d2(DevBuf& b, const double* src, int rows, int cols, int ld, int ldd, hipStream_t s) {
   b.ensure(sizeof(double) * (size_t)ldd * cols + 8);
-  MHIP_CHECK(hipMemcpy2DAsync(b.ptr, sizeof(double) * ldd, src, sizeof(double) * ld,
-                              sizeof(double) * rows, cols, hipMemcpyHostToDevice, s));
+  g_pitched.up(b.ptr, sizeof(double) * ldd, src, sizeof(double) * ld, sizeof(double) * rows, cols, s);
 }
 
 void report(const HipError& e) {
@@ -96,9 +98,7 @@ static void call_gemm_impl(bool split, char tra, char trb, int m, int n, int k, 
     else
       gemm(I.s, tra, trb, m, n, k, alpha, I.a.as<double>(), ar, I.b.as<double>(), br, beta,
            I.c.as<double>(), m);
-    MHIP_CHECK(hipMemcpy2DAsync(c, sizeof(double) * ldc, I.c.ptr, sizeof(double) * m,
-                                sizeof(double) * m, n, hipMemcpyDeviceToHost, I.s));
-    MHIP_CHECK(hipStreamSynchronize(I.s));
+    g_pitched.down(c, sizeof(double) * ldc, I.c.ptr, sizeof(double) * m, sizeof(double) * m, n, I.s);
   } catch (const HipError& e) {
     report(e);
   }
@@ -171,8 +171,7 @@ void mhip_dsyevd(int n, double* a, int lda, double* w, int* info) {
     if (jacobi_sweeps(I.s, I.plan, A, A2, I.c.as<double>(), 1.0e-12, 60, I.hs, I.scal.as<double>(), &sweeps) != 0)
       *info = 1;
     jacobi_sort(I.s, I.plan, A, I.c.as<double>(), I.d.as<double>(), I.b.as<double>());
-    MHIP_CHECK(hipMemcpy2DAsync(a, sizeof(double) * lda, I.d.ptr, sizeof(double) * np,
-                                sizeof(double) * n, n, hipMemcpyDeviceToHost, I.s));
+    g_pitched.down(a, sizeof(double) * lda, I.d.ptr, sizeof(double) * np, sizeof(double) * n, n, I.s);
     MHIP_CHECK(hipMemcpyAsync(w, I.b.ptr, sizeof(double) * n, hipMemcpyDeviceToHost, I.s));
     MHIP_CHECK(hipStreamSynchronize(I.s));
   } catch (const HipError& e) {

@@ -241,6 +241,16 @@ static void download(mhip_ctx* c, void* dst, const void* src, size_t bytes) {
   for (auto& th : pool) th.join();
 }
 
+// The eigenvectors: n columns of n in the caller's array, npad apart here.
+static void upload_c(mhip_ctx* c, const double* src) {
+  const size_t col = sizeof(double) * c->norbs;
+  c->pitched.up(c->C.ptr, sizeof(double) * c->npad, src, col, col, c->norbs, c->stream);
+}
+static void download_c(mhip_ctx* c, double* dst) {
+  const size_t col = sizeof(double) * c->norbs;
+  c->pitched.down(dst, col, c->C.ptr, sizeof(double) * c->npad, col, c->norbs, c->stream);
+}
+
 // eigenvectors_LAPACK on the device copy of a packed matrix: adds i*1e-10 to
 // the diagonal in place, then solves; ctx C/eig hold the result (sorted).
 static void eigen_packed(mhip_ctx* c, double* fpacked, bool perturb, double tol = 1.0e-12,
@@ -788,9 +798,7 @@ void run_scf(mhip_ctx* c, const mhip_scf_opts* o, mhip_scf_result* r, double* p_
   if (p_out) download(c, p_out, P, sizeof(double) * mp);
   if (f_out) download(c, f_out, c->f.ptr, sizeof(double) * mp);
   if (eig_out) download(c, eig_out, c->eig.ptr, sizeof(double) * n);
-  if (c_out)
-    MHIP_CHECK(hipMemcpy2D(c_out, sizeof(double) * n, c->C.ptr, sizeof(double) * c->npad,
-                           sizeof(double) * n, n, hipMemcpyDeviceToHost));
+  if (c_out) download_c(c, c_out);
 }
 
 }  // namespace mhip
@@ -843,6 +851,7 @@ int mhip_finalize(mhip_ctx* c) {
     c->ov.release();
     if (c->hscal) (void)hipHostFree(c->hscal);
     if (c->hstage) (void)hipHostFree(c->hstage);
+    c->pitched.release();
     if (c->hone) (void)hipHostFree(c->hone);
     c->one.release();
     mhip::release_split_scratch(c->stream);
@@ -881,8 +890,7 @@ int mhip_density(mhip_ctx* c, const double* cvec, int ndubl, double occ, double*
     MHIP_REQUIRE(ndubl >= 0 && ndubl <= c->norbs, "mhip_density: ndubl out of range");
     const int n = c->norbs;
     if (cvec) {
-      MHIP_CHECK(hipMemcpy2DAsync(c->C.ptr, sizeof(double) * c->npad, cvec, sizeof(double) * n,
-                                  sizeof(double) * n, n, hipMemcpyHostToDevice, c->stream));
+      upload_c(c, cvec);
       c->have_c = false;
     }
     syrk_packed(c->stream, n, ndubl, occ, c->C.as<double>(), c->npad, c->p.as<double>());
@@ -953,9 +961,7 @@ int mhip_eigen(mhip_ctx* c, double* cvec, double* fpacked, double* eig, int ndim
     // the reference perturbs its argument in place
     MHIP_CHECK(hipMemcpyAsync(fpacked, c->fcopy.ptr, b, hipMemcpyDeviceToHost, s));
     MHIP_CHECK(hipMemcpyAsync(eig, c->eig.ptr, sizeof(double) * ndim, hipMemcpyDeviceToHost, s));
-    MHIP_CHECK(hipMemcpy2DAsync(cvec, sizeof(double) * ndim, c->C.ptr, sizeof(double) * c->npad,
-                                sizeof(double) * ndim, ndim, hipMemcpyDeviceToHost, s));
-    MHIP_CHECK(hipStreamSynchronize(s));
+    download_c(c, cvec);
   });
 }
 
@@ -967,15 +973,12 @@ int mhip_pseudo_diag(mhip_ctx* c, const double* fao, double* vector, int nocc, c
     MHIP_REQUIRE(nocc > 0 && nocc < n, "mhip_pseudo_diag: nocc out of range");
     hipStream_t s = c->stream;
     MHIP_CHECK(hipMemcpyAsync(c->fcopy.ptr, fao, sizeof(double) * c->mpack, hipMemcpyHostToDevice, s));
-    MHIP_CHECK(hipMemcpy2DAsync(c->C.ptr, sizeof(double) * c->npad, vector, sizeof(double) * n,
-                                sizeof(double) * n, n, hipMemcpyHostToDevice, s));
+    upload_c(c, vector);
     MHIP_CHECK(hipMemcpyAsync(c->eig.ptr, eig, sizeof(double) * n, hipMemcpyHostToDevice, s));
     long long nr = 0;
     pseudo_diag_device(s, c->pseudo, n, c->npad, c->fcopy.as<double>(), c->C.as<double>(), nocc,
                        c->eig.as<double>(), &nr);
-    MHIP_CHECK(hipMemcpy2DAsync(vector, sizeof(double) * n, c->C.ptr, sizeof(double) * c->npad,
-                                sizeof(double) * n, n, hipMemcpyDeviceToHost, s));
-    MHIP_CHECK(hipStreamSynchronize(s));
+    download_c(c, vector);
     if (nrot) *nrot = nr;
     c->have_c = false;
   });
