@@ -5,7 +5,7 @@
 namespace mhip {
 
 struct PseudoWork {
-  DevBuf fd, wv, fmo, flag, ab, cols, rot, counts, offs, part;
+  DevBuf fd, wv, fmo, ab, part;
   void ensure(int n, int nocc, int ld);
   void release();
 };

@@ -4,18 +4,17 @@
 //   tiny = 0.05 max|FMO|,
 //   for every (virtual i, occupied j) in that order whose |FMO| >= tiny and
 //   |FMO/(e_j - e_i)| >= 1.5e-7, rotate columns j and i of C.
-// FMO is not updated during the rotations, so every rotation angle is known
-// up front: one kernel computes all of them, a scan compacts the accepted
-// ones in order, and the rotation kernel keeps a slab of rows of C in LDS and
-// applies the whole ordered list to it (rows are independent, so this is
-// exactly the sequential result).
+// FMO is not updated during the rotations, so every angle is known up front,
+// and the rows of C are independent.  Within a row, rotation (i, j) needs the
+// results of (i, j - 1) and (i - 1, j) only: the rotations pass through a
+// chain of lanes, one per virtual, in the order of every element's updates.
+#include <algorithm>
+
 #include "common.h"
 #include "k_pseudo.h"
 
 namespace mhip {
 namespace {
-
-constexpr int SCAN_BLOCK = 1024;
 
 __global__ __launch_bounds__(256) void k_absmax_partial(long long len, const double* __restrict__ x,
                                                         double* __restrict__ part) {
@@ -33,7 +32,8 @@ __global__ __launch_bounds__(256) void k_absmax_partial(long long len, const dou
 }
 
 __global__ __launch_bounds__(256) void k_absmax_final(int nb, const double* __restrict__ part,
-                                                      double* __restrict__ out) {
+                                                      double* __restrict__ out,
+                                                      unsigned long long* __restrict__ count) {
   double m = 0.0;
   for (int i = threadIdx.x; i < nb; i += 256) m = fmax(m, part[i]);
   __shared__ double red[256];
@@ -43,100 +43,132 @@ __global__ __launch_bounds__(256) void k_absmax_final(int nb, const double* __re
     if (threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = 0.05 * red[0];
+  if (threadIdx.x == 0) {
+    out[0] = 0.05 * red[0];
+    *count = 0;
+  }
 }
 
-// Rotation parameters for every (virtual, occupied) pair, linear index
-// ij = v * nocc + j, exactly as diag.F90:130-153 computes them.
-__global__ void k_rot_params(int nocc, int nvirt, const double* __restrict__ fmo,
-                             const double* __restrict__ eig, const double* __restrict__ tiny_dev,
-                             double bigeps, int* __restrict__ flag, double2* __restrict__ ab) {
-  const long long len = (long long)nocc * nvirt;
+// Rotation parameters for every (virtual, occupied) pair, exactly as
+// diag.F90:130-153 computes them, in the order k_rotate reads them: entry
+// [b][t][l] is virtual 64 b + l with occupied t - l, kSkip where the pair is
+// not rotated or there is none.
+constexpr int kStep = 16;        // steps that k_rotate loads at once
+constexpr int kFront = 64;       // room before a row in LDS
+constexpr double kSkip = 2.0;    // no cosine
+__global__ __launch_bounds__(256) void k_rot_params(int nocc, int nvirt, int steps, const double* __restrict__ fmo,
+                                                    const double* __restrict__ eig,
+                                                    const double* __restrict__ tiny_dev, double bigeps,
+                                                    double2* __restrict__ ab,
+                                                    unsigned long long* __restrict__ count) {
+  const long long len = (long long)((nvirt + 63) / 64) * steps * 64;
   const double tiny = tiny_dev[0];
-  for (long long ij = blockIdx.x * (long long)blockDim.x + threadIdx.x; ij < len;
-       ij += (long long)gridDim.x * blockDim.x) {
-    const int v = (int)(ij / nocc), j = (int)(ij % nocc);
-    const double c = fmo[ij];
-    int ok = 0;
-    double alpha = 1.0, beta = 0.0;
-    if (!(fabs(c) < tiny)) {
-      const double a = eig[j], b = eig[nocc + v];
-      const double d = a - b;
-      if (!(fabs(c / d) < bigeps)) {
-        const double e = (d >= 0.0 ? 1.0 : -1.0) * sqrt(4.0 * c * c + d * d);
-        alpha = sqrt(0.5 * (1.0 + d / e));
-        beta = -(c >= 0.0 ? 1.0 : -1.0) * sqrt(1.0 - alpha * alpha);
-        ok = 1;
+  int rotated = 0;
+  for (long long q = blockIdx.x * 256LL + threadIdx.x; q < len; q += (long long)gridDim.x * 256) {
+    const int l = (int)(q & 63);
+    const long long bt = q >> 6;
+    const int v = (int)(bt / steps) * 64 + l, j = (int)(bt % steps) - l;
+    double alpha = kSkip, beta = 0.0;
+    if (v < nvirt && j >= 0 && j < nocc) {
+      const double c = fmo[(long long)v * nocc + j];
+      if (!(fabs(c) < tiny)) {
+        const double d = eig[j] - eig[nocc + v];
+        if (!(fabs(c / d) < bigeps)) {
+          const double e = (d >= 0.0 ? 1.0 : -1.0) * sqrt(4.0 * c * c + d * d);
+          alpha = sqrt(0.5 * (1.0 + d / e));
+          beta = -(c >= 0.0 ? 1.0 : -1.0) * sqrt(1.0 - alpha * alpha);
+          ++rotated;
+        }
       }
     }
-    flag[ij] = ok;
-    ab[ij] = make_double2(alpha, beta);
+    ab[q] = make_double2(alpha, beta);
   }
-}
-
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_counts(long long len, const int* __restrict__ flag,
-                                                            int* __restrict__ counts) {
-  const long long i = blockIdx.x * (long long)SCAN_BLOCK + threadIdx.x;
-  __shared__ int red[SCAN_BLOCK];
-  red[threadIdx.x] = (i < len) ? flag[i] : 0;
+  for (int off = 32; off > 0; off >>= 1) rotated += __shfl_xor(rotated, off);
+  __shared__ int part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = rotated;
   __syncthreads();
-  for (int w = SCAN_BLOCK / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    const int all = part[0] + part[1] + part[2] + part[3];
+    if (all) atomicAdd(count, (unsigned long long)all);
   }
-  if (threadIdx.x == 0) counts[blockIdx.x] = red[0];
 }
 
-// exclusive scan of the per-block counts (single workgroup), total in offs[nb]
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_offsets(int nb, const int* __restrict__ counts,
-                                                             long long* __restrict__ offs) {
-  __shared__ long long buf[SCAN_BLOCK];
-  long long carry = 0;
-  for (int base = 0; base < nb; base += SCAN_BLOCK) {
-    const int i = base + threadIdx.x;
-    const long long v = (i < nb) ? counts[i] : 0;
-    buf[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < SCAN_BLOCK; off <<= 1) {
-      const long long t = (threadIdx.x >= off) ? buf[threadIdx.x - off] : 0;
-      __syncthreads();
-      buf[threadIdx.x] += t;
-      __syncthreads();
+// lane l gets lane l - 1's value, lane 0 gets `first`
+__device__ __forceinline__ double from_lane_below(double x, double first) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(x), 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(x), 0x138, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// All rotations of a row of C, a row per wave.  64 virtuals at a time, one in
+// each lane's register; at step t lane l rotates its virtual with occupied
+// t - l, which comes from lane l - 1 as that left it, so the occupied
+// coefficients stream from the row in LDS through the lanes and back.  The
+// row has kStep-rounded room around it there: what enters lane 0 after the
+// last occupied and leaves lane 63 before the first is not rotated.
+// A step issues two lane shifts, four FP64 operations and the selects; its
+// angles are one coalesced load, kStep steps ahead.  Several rows a wave
+// would issue as much per row, on fewer of the chip's SIMDs.  The ordered
+// list, a lane per row and one rotation after another with an LDS read and
+// write each, took 434 us at 384 orbitals (256 occupied); this takes 37.
+__global__ __launch_bounds__(256) void k_rotate(int n, int ldc, double* __restrict__ C, int nocc, int nvirt,
+                                                int steps, const double2* __restrict__ ab) {
+  extern __shared__ double slab[];  // a row of kFront + steps per wave
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rows = blockDim.x >> 6, len = kFront + steps;  // 1, 2 or 4 rows
+  const int row0 = blockIdx.x * rows, row = row0 + wave;
+  for (int e = tid; e < rows * nocc; e += blockDim.x) {
+    const int r = e & (rows - 1), c = e / rows;
+    slab[r * len + kFront + c] = row0 + r < n ? C[(size_t)(row0 + r) + (size_t)c * ldc] : 0.0;
+  }
+  __syncthreads();
+  double* S = slab + wave * len;
+  for (int v0 = 0; v0 < nvirt; v0 += 64) {
+    double* col = C + (size_t)row + (size_t)(nocc + v0 + lane) * ldc;
+    const bool have = v0 + lane < nvirt && row < n;
+    double a = 0.0, b = have ? *col : 0.0;
+    const double2* q = ab + (size_t)(v0 >> 6) * steps * 64 + lane;
+    double2 next[kStep];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) next[u] = q[(size_t)u * 64];
+    for (int t0 = 0; t0 < steps; t0 += kStep) {
+      double2 rot[kStep];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) rot[u] = next[u];
+      if (t0 + kStep < steps) {
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) next[u] = q[(size_t)(t0 + kStep + u) * 64];
+      }
+      double x[kStep];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) x[u] = S[kFront + t0 + u];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) {
+        const bool skip = rot[u].x == kSkip;
+        a = from_lane_below(a, x[u]);
+        const double na = rot[u].x * a + rot[u].y * b;
+        const double nb = rot[u].x * b - rot[u].y * a;
+        a = skip ? a : na;
+        b = skip ? b : nb;
+        x[u] = a;
+      }
+      // lane 63 is 63 steps behind lane 0, and behind this wave's reads
+      if (lane == 63) {
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) S[kFront - 63 + t0 + u] = x[u];
+      }
     }
-    if (i < nb) offs[i] = carry + buf[threadIdx.x] - v;
-    const long long tot = buf[SCAN_BLOCK - 1];
-    __syncthreads();
-    carry += tot;
+    if (have) *col = b;
   }
-  if (threadIdx.x == 0) offs[nb] = carry;
-}
-
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_scatter(long long len, int nocc,
-                                                             const int* __restrict__ flag,
-                                                             const double2* __restrict__ ab,
-                                                             const long long* __restrict__ offs,
-                                                             int2* __restrict__ cols,
-                                                             double2* __restrict__ rot) {
-  const long long i = blockIdx.x * (long long)SCAN_BLOCK + threadIdx.x;
-  __shared__ int buf[SCAN_BLOCK];
-  const int v = (i < len) ? flag[i] : 0;
-  buf[threadIdx.x] = v;
   __syncthreads();
-  for (int off = 1; off < SCAN_BLOCK; off <<= 1) {
-    const int t = (threadIdx.x >= off) ? buf[threadIdx.x - off] : 0;
-    __syncthreads();
-    buf[threadIdx.x] += t;
-    __syncthreads();
-  }
-  if (v) {
-    const long long dst = offs[blockIdx.x] + buf[threadIdx.x] - 1;
-    const int vv = (int)(i / nocc), j = (int)(i % nocc);
-    cols[dst] = make_int2(j, nocc + vv);
-    rot[dst] = ab[i];
+  for (int e = tid; e < rows * nocc; e += blockDim.x) {
+    const int r = e & (rows - 1), c = e / rows;
+    if (row0 + r < n) C[(size_t)(row0 + r) + (size_t)c * ldc] = slab[r * len + kFront + c];
   }
 }
 
-// Apply the ordered rotation list to `rows` consecutive rows of C held in LDS.
+// Apply an ordered list of rotations of any two columns to `rows` consecutive
+// rows of C held in LDS.
 __global__ __launch_bounds__(64) void k_apply_rotations(int n, int ldc, double* __restrict__ C,
                                                         int rows, const long long* __restrict__ total,
                                                         const int2* __restrict__ cols,
@@ -169,24 +201,22 @@ __global__ __launch_bounds__(64) void k_apply_rotations(int n, int ldc, double* 
 
 }  // namespace
 
+// the first occupied enters lane 0 at step 0, the last leaves lane 63 at step
+// nocc + 62
+static int rot_steps(int nocc) { return (nocc + 63 + kStep - 1) / kStep * kStep; }
+
 void PseudoWork::ensure(int n, int nocc, int ld) {
   const long long nvirt = n - nocc;
   const long long len = (long long)nocc * nvirt;
   fd.ensure(sizeof(double) * (size_t)ld * ld);
   wv.ensure(sizeof(double) * (size_t)ld * std::max<long long>(nvirt, 1));
   fmo.ensure(sizeof(double) * std::max<long long>(len, 1));
-  flag.ensure(sizeof(int) * std::max<long long>(len, 1));
-  ab.ensure(sizeof(double2) * std::max<long long>(len, 1));
-  cols.ensure(sizeof(int2) * std::max<long long>(len, 1));
-  rot.ensure(sizeof(double2) * std::max<long long>(len, 1));
-  const long long nblk = (len + SCAN_BLOCK - 1) / SCAN_BLOCK + 1;
-  counts.ensure(sizeof(int) * nblk);
-  offs.ensure(sizeof(long long) * (nblk + 1));
-  part.ensure(sizeof(double) * 1024);
+  ab.ensure(sizeof(double2) * ((nvirt + 63) / 64) * 64 * rot_steps(nocc));
+  part.ensure(sizeof(double) * 1032);
 }
 
 void PseudoWork::release() {
-  for (DevBuf* b : {&fd, &wv, &fmo, &flag, &ab, &cols, &rot, &counts, &offs, &part}) b->release();
+  for (DevBuf* b : {&fd, &wv, &fmo, &ab, &part}) b->release();
 }
 
 void pseudo_diag_device(hipStream_t s, PseudoWork& w, int n, int ld, const double* fpacked,
@@ -207,38 +237,26 @@ void pseudo_diag_device(hipStream_t s, PseudoWork& w, int n, int ld, const doubl
   hipLaunchKernelGGL(k_absmax_partial, dim3(nb), dim3(256), 0, s, len, w.fmo.as<double>(),
                      w.part.as<double>());
   MHIP_LAUNCH_CHECK();
+  unsigned long long* count = reinterpret_cast<unsigned long long*>(w.part.as<double>() + 1024);
   hipLaunchKernelGGL(k_absmax_final, dim3(1), dim3(256), 0, s, nb, w.part.as<double>(),
-                     w.part.as<double>() + 1023);
+                     w.part.as<double>() + 1023, count);
   MHIP_LAUNCH_CHECK();
-  const int pb = (int)std::min<long long>(8192, (len + 255) / 256);
-  hipLaunchKernelGGL(k_rot_params, dim3(pb), dim3(256), 0, s, nocc, nvirt, w.fmo.as<double>(), eig,
-                     w.part.as<double>() + 1023, 1.5e-7, w.flag.as<int>(), w.ab.as<double2>());
+  const int steps = rot_steps(nocc);
+  const long long entries = (long long)((nvirt + 63) / 64) * 64 * steps;
+  hipLaunchKernelGGL(k_rot_params, dim3((int)std::min<long long>(512, (entries + 255) / 256)), dim3(256), 0, s, nocc,
+                     nvirt, steps, w.fmo.as<double>(), eig, w.part.as<double>() + 1023, 1.5e-7, w.ab.as<double2>(),
+                     count);
   MHIP_LAUNCH_CHECK();
-  const int nblk = (int)((len + SCAN_BLOCK - 1) / SCAN_BLOCK);
-  hipLaunchKernelGGL(k_scan_counts, dim3(nblk), dim3(SCAN_BLOCK), 0, s, len, w.flag.as<int>(),
-                     w.counts.as<int>());
-  MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(SCAN_BLOCK), 0, s, nblk, w.counts.as<int>(),
-                     w.offs.as<long long>());
-  MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_scan_scatter, dim3(nblk), dim3(SCAN_BLOCK), 0, s, len, nocc,
-                     w.flag.as<int>(), w.ab.as<double2>(), w.offs.as<long long>(),
-                     w.cols.as<int2>(), w.rot.as<double2>());
-  MHIP_LAUNCH_CHECK();
-  const int rows = std::max(1, std::min(64, 19456 / n));
-  const size_t lds = sizeof(double) * (size_t)rows * n;
-  static bool attr_set = false;
-  if (!attr_set) {
-    MHIP_CHECK(hipFuncSetAttribute((const void*)k_apply_rotations,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    attr_set = true;
-  }
-  hipLaunchKernelGGL(k_apply_rotations, dim3((n + rows - 1) / rows), dim3(64), lds, s, n, ld, C,
-                     rows, w.offs.as<long long>() + nblk, w.cols.as<int2>(), w.rot.as<double2>());
+  // up to four rows a workgroup, as they fit the LDS
+  const size_t max_lds = 160 * 1024, row = sizeof(double) * (kFront + steps);
+  int rows = 4;
+  while (rows > 1 && rows * row > max_lds) rows >>= 1;
+  MHIP_CHECK(hipFuncSetAttribute((const void*)k_rotate, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds));
+  hipLaunchKernelGGL(k_rotate, dim3((n + rows - 1) / rows), dim3(64 * rows), rows * row, s, n, ld, C, nocc, nvirt,
+                     steps, w.ab.as<double2>());
   MHIP_LAUNCH_CHECK();
   if (nrot_out) {
-    MHIP_CHECK(hipMemcpyAsync(nrot_out, w.offs.as<long long>() + nblk, sizeof(long long),
-                              hipMemcpyDeviceToHost, s));
+    MHIP_CHECK(hipMemcpyAsync(nrot_out, count, sizeof(long long), hipMemcpyDeviceToHost, s));
     MHIP_CHECK(hipStreamSynchronize(s));
   }
 }
