@@ -112,8 +112,6 @@ __device__ __forceinline__ void cross_setup(CrossRegs& v, int k, int g) {
   const int k2 = k ^ v.d;
   v.own_rot = k * 16;
   v.mate_rot = k2 * 16;
-  v.lr = (k * SB + 32 + k2) * 8;
-  v.rl = (k2 * SB + 32 + k) * 8;
   v.own_q = (32 + k) * 8;
 }
 
@@ -212,11 +210,12 @@ __device__ __forceinline__ void cross_rounds(std::integer_sequence<int, R...>, d
 // intra[pair] is set, the levels that rotate the pairs inside the blocks: 16
 // cross rounds between the 16-wide halves of both blocks at once, then 8, 4,
 // 2 and 1 between ever smaller halves.  A level inside the blocks is the
-// cross level of S with two index bits exchanged (the bit that tells the
-// halves becomes the one that tells the blocks).  The sweep schedule sets
-// intra once per sweep of the block's group, so every index pair of the
-// matrix is rotated once per sweep, in about half the sequential rounds of a
-// full 64-index inner sweep.
+// cross level with two index bits exchanged (the bit that tells the halves
+// becomes the one that tells the blocks): S is addressed that way, where
+// moving it there and back took 1.5 us more a level.  The sweep schedule sets intra
+// once per sweep of the block's group, so every index pair of the matrix is
+// rotated once per sweep, in about half the sequential rounds of a full
+// 64-index inner sweep.
 //
 // A cross round needs one barrier: the element that rotation k of the next
 // round acts on is in a block of this round, whose thread computes the next
@@ -255,25 +254,8 @@ struct JacSolve {
   int max_inner;
 };
 
-// S and Q's columns with index bits 5 and j exchanged; all threads have passed
-// a barrier since the last access to S, and do again.
-__device__ __forceinline__ void exchange_bits(double (*S)[SB], CrossRegs& v, int k, int g, int j) {
-  auto to = [&](int i) {
-    const int x = ((i >> 5) ^ (i >> j)) & 1;
-    return i ^ (x << 5) ^ (x << j);
-  };
-  double t[SB * SB / CROSS_THREADS];
-#pragma unroll
-  for (int it = 0; it < SB * SB / CROSS_THREADS; ++it) {
-    const int e = (32 * g + k) + CROSS_THREADS * it;
-    t[it] = S[to(e / SB)][to(e % SB)];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < SB * SB / CROSS_THREADS; ++it) {
-    const int e = (32 * g + k) + CROSS_THREADS * it;
-    S[e / SB][e % SB] = t[it];
-  }
+// Q's columns with index bits 5 and j exchanged.
+__device__ __forceinline__ void exchange_q(CrossRegs& v, int k, int j) {
   const bool up = (k >> j) & 1;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -281,11 +263,11 @@ __device__ __forceinline__ void exchange_bits(double (*S)[SB], CrossRegs& v, int
     if (up) v.ql[i] = x;
     else v.qr[i] = x;
   }
-  __syncthreads();
 }
 
 // Diagonalizes the problem in lds.s(): the upper right quadrant and the two
-// diagonal ones, and the lower left one where do_intra asks for it.  Returns the inner sweeps it took (0: nothing rotated); with p.q null, Q is left in
+// diagonal ones, and the lower left one where do_intra asks for it.  Returns
+// the inner sweeps it took (0: nothing rotated); with p.q null, Q is left in
 // lds.q() and S in lds.s().
 __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_intra, const JacSolve& p) {
   double(*S)[SB] = lds.s();
@@ -301,6 +283,13 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
     v.qr[j] = (4 * g + j == 32 + k) ? 1.0 : 0.0;
   }
   int sweeps = 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a round ends with the angles of the next, which wave 7 computes in three
+  // of four rounds, 6, 5 or 0 in the others, while two waves share each SIMD:
+  // 5% of an SCF at 24 to 1020 orbitals.  Update workgroups come after.
+  if (wave == 7) __builtin_amdgcn_s_setprio(3);
+  else if (wave >= 5) __builtin_amdgcn_s_setprio(2);
+  else __builtin_amdgcn_s_setprio(1);
   for (int sw = 0; sw < p.max_inner; ++sw) {
     v.ll = S[k][k2];
     v.rr = S[32 + k][32 + k2];
@@ -328,16 +317,26 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
       // nothing to rotate between a real index and the padding (a matrix that
       // is one pair problem)
       if (p.nreal <= (1 << lv)) continue;
-      if (lv < 5) exchange_bits(S, v, k, g, lv);
+      // index i of the level is pi(i) of S, bits 5 and lv exchanged: a level
+      // inside the blocks only has other addresses, and Q's columns move.
+      // pi(a ^ b) = pi(a) ^ pi(b), and the sigmas stay below bit lv.
+      auto pi = [lv](int i) {
+        const int x = ((i >> 5) ^ (i >> lv)) & 1;
+        return i ^ (x << 5) ^ (x << lv);
+      };
+      const int up = 1 << lv, rk = pi(k), rd = pi(v.d), rg = pi(g), rq = rk ^ up, rk2 = rk ^ rd, rq2 = rq ^ rd;
+      if (lv < 5) exchange_q(v, k, lv);
       const int nr = 1 << lv;
-      v.ll = S[k][k2];
-      v.rr = S[32 + k][32 + k2];
+      v.lr = (rk * SB + rq2) * 8;
+      v.rl = (rk2 * SB + rq) * 8;
+      v.ll = S[rk][rk2];
+      v.rr = S[rq][rq2];
       // angles of round 0 and the diagonals after it
       if (tid < 32) {
-        const double app = S[tid][tid], aqq = S[32 + tid][32 + tid], apq = S[tid][32 + tid];
+        const double app = S[rk][rk], aqq = S[rq][rq], apq = S[rk][rq];
         double c, sn, t;
         rotation_of(app, aqq, apq, c, sn, t);
-        S[tid][32 + tid] = 0.0;
+        S[rk][rq] = 0.0;
         lds.rot[0][tid] = make_double2(c, sn);
         lds.dgl[0][tid] = app - t * apq;
         lds.dgl[0][32 + tid] = aqq + t * apq;
@@ -351,21 +350,25 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
       for (int j = 0; j < 4; ++j) v.qr[j] = __shfl(v.qr[j], (tid & 32) | (k ^ SL), 64);
       // S whole again: the diagonal blocks here, the upper right one is there
       // and gives the lower left one
-      const int last = 32 + (k ^ SL), last2 = 32 + (k2 ^ SL);
+      const int last = rq ^ SL, last2 = rq2 ^ SL;
       if (lv < 5 || do_intra) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const int q = 32 + (k ^ (g + 16 * j));
-          S[q][k] = S[k][q];
+          const int q = rq ^ rg ^ (j ? pi(16) : 0);
+          S[q][rk] = S[rk][q];
         }
       }
-      S[k][k2] = S[k2][k] = v.ll;
+      S[rk][rk2] = S[rk2][rk] = v.ll;
       S[last][last2] = S[last2][last] = v.rr;
-      if (tid < SB) S[tid][tid] = lds.dgl[(nr - 1) & 1][tid];
+      if (tid < SB) {
+        const int r = pi(tid);
+        S[r][r] = lds.dgl[(nr - 1) & 1][tid];
+      }
       __syncthreads();
-      if (lv < 5) exchange_bits(S, v, k, g, lv);
+      if (lv < 5) exchange_q(v, k, lv);
     }
   }
+  __builtin_amdgcn_s_setprio(0);
   if (p.di) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
