@@ -308,9 +308,8 @@ __global__ __launch_bounds__(256) void k_jac_apply_c(double* __restrict__ C, int
 // Solving in a launch of its own left the chip to npairs workgroups for 22
 // of a step's 37 us at 1020 orbitals (with the A update behind it, and the C
 // update on a second stream, ordered by two events per step); this launch
-// takes 24 us, of which the solve's 32 rounds are 12 (each a chain of about
-// 940 cycles: LDS, the block, the next angle, a barrier) and putting its
-// problem together 4.  At 3072 orbitals the updates set it (48 us).
+// takes 22 us, of which the solve's 32 rounds are 12 and putting its problem
+// together 4.  At 3072 orbitals the updates set it (48 us).
 __global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int base) {
   static_assert(UPD_NT == CROSS_THREADS, "one workgroup size for every role");
   __shared__ JacLds lds;
@@ -598,6 +597,13 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
     // the first step's solve of a later sweep ran in the last launch of the
     // sweep before
     if (ahead && sw == 0) solve(0, skip_abs);
+    // A solve shares its CU with an update workgroup where two fit, and takes
+    // longer for it.  While the updates need no more than about three rounds
+    // of the chip one to a CU, they still end before the solves: LDS that is
+    // not used keeps every workgroup alone.  SCFs at 1020 orbitals (408
+    // workgroups) 53.3 -> 49.4 ms, 1200 (570) 71.2 -> 66.4, 1500 (900) equal,
+    // 1800 (1305) 133 -> 160.
+    const size_t alone = npairs + ntiles + nctiles <= 3 * 256 ? 16384 : 0;
     for (int step = 0; step < nsteps; ++step) {
       if (!ahead) {
         mark(step, 0);
@@ -616,7 +622,7 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
                         dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
                         inner};
         auto launch = [&](int from, int to) {
-          hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), 0, s, a, from);
+          hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from);
           MHIP_LAUNCH_CHECK();
         };
         if (!timing) {
