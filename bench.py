@@ -208,14 +208,16 @@ def main():
     lib.mhip_kernel_timing(ctx.h, 0, *jrefs)
     solve_ms, n_solve, apply_ms, n_apply, applyc_ms, n_applyc, tiles, pairs, rotations = [v.value for v in jv]
     npad = ((n + 63) // 64) * 64
+    c_rows = (s.nclose ** 2 + (npad - s.nclose) ** 2) / npad  # mean over the pairs
     # block-Jacobi algorithmic work: A-update = two 64^3 products per processed
-    # tile; C-update = one n x 64 x 64 product per processed pair; solve = the
+    # tile; C-update = one m x 64 x 64 product per processed pair, m the size of
+    # its group (the exit diagonalization's occupied or virtual one); solve = the
     # rotations the library counted (32 x 32 cross rounds per pair, plus 2 x 496
     # inside the blocks once per sweep) x (64 + 64 + 64 element pairs) x 6 flops
     entries = [
         ("k_jac_solve", "mfma", solve_ms, n_solve, rotations * 3.0 * 64 * 6, 0.0),
         ("k_jac_apply_a_mfma", "mfma", apply_ms, n_apply, tiles * 2.0 * 2.0 * 64 ** 3, 0.0),
-        ("k_jac_apply_c_mfma", "mfma", applyc_ms, n_applyc, pairs * 2.0 * npad * 64 * 64, 0.0),
+        ("k_jac_apply_c_mfma", "mfma", applyc_ms, n_applyc, pairs * 2.0 * c_rows * 64 * 64, 0.0),
     ]
     for i in range(nk):
         name = lib.mhip_kernel_class_name(i).decode()

@@ -48,9 +48,10 @@ extern int g_jacobi_schedule;
 void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc);
 // Sweeps until max|offdiag| <= tol * max(1, max|diag|).  A2 is scratch of A's
 // size; the steps go from one to the other, and A names the one that holds
-// the result on return.  Returns 0 when converged, 1 when max_sweeps ran out.
+// the result on return.  With c_blocks (a grouped plan) C is two diagonal
+// blocks, the rest of it zero and left alone.  Returns 0 when converged, 1 when max_sweeps ran out.
 int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
-                  double* host_scal, double* dev_scal, int* sweeps_done);
+                  double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks = false);
 // eig_dev[k] = k-th smallest diagonal entry, Cout[:,k] = C[:,perm[k]].
 void jacobi_sort(hipStream_t s, JacobiPlan& plan, const double* A, const double* C, double* Cout,
                  double* eig_dev);

@@ -319,8 +319,10 @@ __global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int ba
   } else if (b < a.npairs + a.ntiles) {
     step_tile_a(lds.m, a, b - a.npairs);
   } else {
-    const int c = b - a.npairs - a.ntiles, nrow = a.lda / SB;
-    step_tile_c(lds.m, a, (c % nrow) * SB, c / nrow);
+    // tiles of C; of two diagonal blocks only theirs
+    const int c = b - a.npairs - a.ntiles, nrow = a.lda / SB, rows0 = a.crows ? a.crows : nrow, n0 = a.npo * rows0;
+    if (c < n0) step_tile_c(lds.m, a, (c % rows0) * SB, c / rows0);
+    else step_tile_c(lds.m, a, (rows0 + (c - n0) % (nrow - rows0)) * SB, a.npo + (c - n0) / (nrow - rows0));
   }
 }
 
@@ -537,7 +539,7 @@ void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc) {
 }
 
 int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
-                  double* host_scal, double* dev_scal, int* sweeps_done) {
+                  double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks) {
   const int lda = plan.npad;
   int done = 0;
   // Inner sweeps per step.  Cross schedule: one; a second saves up to a fifth
@@ -550,7 +552,9 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
   // every step's solves ride in the launch of the step before
   const bool ahead = cross && g_kernel_variant == 1 && plan.npairs > 1;
   const int npairs = plan.npairs, npv = npairs - plan.npo, nsteps = plan.nsteps;
-  const int ntiles = plan.npo * (plan.npo + 1) / 2 + npv * (npv + 1) / 2, nctiles = npairs * (plan.npad / SB);
+  const int ntiles = plan.npo * (plan.npo + 1) / 2 + npv * (npv + 1) / 2, nrow = plan.npad / SB;
+  const int crows = c_blocks ? plan.split / SB : 0;
+  const int nctiles = crows ? plan.npo * crows + npv * (nrow - crows) : npairs * nrow;
   int slot = 0;  // of the step at hand in the two-step buffers
   auto qslot = [&](int k) { return plan.qbuf.as<double>() + (size_t)k * npairs * SB * SB; };
   auto aslot = [&](int k) { return plan.active.as<int>() + (size_t)k * npairs; };
@@ -620,7 +624,7 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
                         pairs_of(step), qslot(slot), aslot(slot),      pairs_of(next),
                         intra_of(next), plan.where.as<int>() + (size_t)step * plan.nb, qslot(slot ^ 1), aslot(slot ^ 1),
                         dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
-                        inner};
+                        inner,      crows};
         auto launch = [&](int from, int to) {
           hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from);
           MHIP_LAUNCH_CHECK();

@@ -454,6 +454,7 @@ struct JacStep {
   double* diag_n;     // and after the next one
   double tol, skip_abs;
   int max_inner;
+  int crows = 0;      // > 0: C is two diagonal blocks, the first of crows 64-row tiles and npo pairs
 };
 
 // Tile (P1 <= P2) of A: Ao(rows of P1, cols of P2) = Q1^T A Q2, and its
