@@ -19,6 +19,8 @@ struct JacobiPlan {
   long long active_rotations = 0;                 // 2x2 rotations of the timed solves
   std::vector<int> intra_host;                    // host copy of intra
   std::vector<hipEvent_t> ev;
+  hipEvent_t tested = nullptr;                    // behind the last stopping test
+  void ensure_test_event(hipStream_t s);
   DevBuf pairs;  // nsteps x npairs x 2 block indices
   DevBuf qbuf;   // two steps x npairs x 64 x 64 rotations
   DevBuf diag;   // two steps x nb x 32 x 32 diagonal blocks as the solves left them
@@ -37,6 +39,8 @@ struct JacobiPlan {
     for (DevBuf* b : {&pairs, &qbuf, &diag, &where, &part, &perm, &active, &intra, &counts}) b->release();
     for (auto e : ev) (void)hipEventDestroy(e);
     ev.clear();
+    if (tested) (void)hipEventDestroy(tested);
+    tested = nullptr;
   }
 };
 
@@ -49,7 +53,8 @@ void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc);
 // Sweeps until max|offdiag| <= tol * max(1, max|diag|).  A2 is scratch of A's
 // size; the steps go from one to the other, and A names the one that holds
 // the result on return.  With c_blocks (a grouped plan) C is two diagonal
-// blocks, the rest of it zero and left alone.  Returns 0 when converged, 1 when max_sweeps ran out.
+// blocks, the rest of it zero and left alone.  host_scal: two doubles in
+// pinned memory.  Returns 0 when converged, 1 when max_sweeps ran out.
 int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
                   double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks = false);
 // eig_dev[k] = k-th smallest diagonal entry, Cout[:,k] = C[:,perm[k]].

@@ -159,8 +159,9 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_jac_solve(
 __global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_solve_x(
     const double* __restrict__ A, int lda, int nreal, const int* __restrict__ pairs,
     const int* __restrict__ intra, double* __restrict__ Qbuf, int* __restrict__ active, double* __restrict__ diag,
-    double tol, double skip_abs, int max_inner) {
+    double tol, double skip_abs, int max_inner, SweepTest test) {
   __shared__ JacLds lds;
+  if (test.done(skip_abs)) return;
   const int pidx = blockIdx.x;
   const int I = pairs[2 * pidx], J = pairs[2 * pidx + 1];
   solve_from_memory(lds, A, lda, I, J, intra[pidx] != 0,
@@ -310,9 +311,10 @@ __global__ __launch_bounds__(256) void k_jac_apply_c(double* __restrict__ C, int
 // update on a second stream, ordered by two events per step); this launch
 // takes 22 us, of which the solve's 32 rounds are 12 and putting its problem
 // together 4.  At 3072 orbitals the updates set it (48 us).
-__global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int base) {
+__global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int base, SweepTest test) {
   static_assert(UPD_NT == CROSS_THREADS, "one workgroup size for every role");
   __shared__ JacLds lds;
+  if (test.done(a.skip_abs)) return;
   const int b = (int)blockIdx.x + base;
   if (b < a.npairs) {
     step_solve(lds, a, b);
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(256) void k_offmax_partial(int n, const double* __r
 }
 
 __global__ __launch_bounds__(1024) void k_offmax_final(int n, const double* __restrict__ part,
-                                                       double* __restrict__ out) {
+                                                       double* __restrict__ out, double* __restrict__ host) {
   double off = 0.0, dg = 0.0;
   for (int j = threadIdx.x; j < n; j += 1024) {
     off = fmax(off, part[2 * j]);
@@ -374,8 +376,8 @@ __global__ __launch_bounds__(1024) void k_offmax_final(int n, const double* __re
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[0] = r1[0];
-    out[1] = r2[0];
+    out[0] = host[0] = r1[0];
+    out[1] = host[1] = r2[0];
   }
 }
 
@@ -533,6 +535,18 @@ void JacobiPlan::build(int n_in, int split) {
   counts.ensure((size_t)2 * nsteps * sizeof(int));
 }
 
+void JacobiPlan::ensure_test_event(hipStream_t s) {
+  if (tested) return;
+  // an event belongs to the device that is current, a stream to its own
+  int device = 0, of_stream = 0;
+  MHIP_CHECK(hipGetDevice(&device));
+  MHIP_CHECK(hipStreamGetDevice(s, &of_stream));
+  if (device != of_stream) MHIP_CHECK(hipSetDevice(of_stream));
+  const hipError_t r = hipEventCreateWithFlags(&tested, hipEventDisableTiming);
+  if (device != of_stream) (void)hipSetDevice(device);
+  MHIP_CHECK(r);
+}
+
 void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc) {
   hipLaunchKernelGGL(k_set_identity, dim3((npad + 255) / 256, npad), dim3(256), 0, s, npad, C, ldc);
   MHIP_LAUNCH_CHECK();
@@ -561,25 +575,54 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
   auto dslot = [&](int k) { return plan.diag.as<double>() + (size_t)k * plan.nb * BS * BS; };
   auto pairs_of = [&](int step) { return plan.pairs.as<int>() + (size_t)step * npairs * 2; };
   auto intra_of = [&](int step) { return plan.intra.as<int>() + (size_t)step * npairs; };
-  auto solve = [&](int step, double skip_abs) {
+  auto solve = [&](int step, double skip_abs, SweepTest test = {}) {
     if (cross)
       hipLaunchKernelGGL(k_jac_solve_x, dim3(npairs), dim3(CROSS_THREADS), 0, s, A, lda, plan.n, pairs_of(step),
                          intra_of(step), qslot(slot), aslot(slot), ahead ? dslot(slot) : nullptr, inner_tol, skip_abs,
-                         inner);
+                         inner, test);
     else
       hipLaunchKernelGGL(k_jac_solve, dim3(npairs), dim3(SOLVE_THREADS), 0, s, A, lda, plan.n, pairs_of(step),
                          qslot(slot), aslot(slot), 1.0e-14, skip_abs, inner);
     MHIP_LAUNCH_CHECK();
   };
+  // A solve shares its CU with an update workgroup where two fit, and takes
+  // longer for it.  While the updates need no more than about three rounds of
+  // the chip one to a CU, they still end before the solves: LDS that is not
+  // used keeps every workgroup alone.  SCFs at 1020 orbitals (408 workgroups)
+  // 53.3 -> 49.4 ms, 1200 (570) 71.2 -> 66.4, 1500 (900) equal, 1800 (1305)
+  // 133 -> 160.
+  const size_t alone = npairs + ntiles + nctiles <= 3 * 256 ? 16384 : 0;
+  auto launch_step = [&](int step, double skip_abs, int from, int to, SweepTest test) {
+    const int next = (step + 1) % nsteps;
+    const JacStep a{A,          ahead ? A2 : A,  C,                lda,
+                    plan.n,     npairs,          plan.npo,         ntiles,
+                    pairs_of(step), qslot(slot), aslot(slot),      pairs_of(next),
+                    intra_of(next), plan.where.as<int>() + (size_t)step * plan.nb, qslot(slot ^ 1), aslot(slot ^ 1),
+                    dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
+                    inner,      crows};
+    hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from, test);
+    MHIP_LAUNCH_CHECK();
+  };
+  const int total = npairs + ntiles + nctiles;
+  plan.ensure_test_event(s);
   for (int sw = 0; sw <= max_sweeps; ++sw) {
     hipLaunchKernelGGL(k_offmax_partial, dim3(plan.n), dim3(256), 0, s, plan.n, A, lda,
                        plan.grouped ? plan.split : 0, plan.part.as<double>());
     MHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_offmax_final, dim3(1), dim3(1024), 0, s, plan.n, plan.part.as<double>(),
-                       dev_scal);
+    hipLaunchKernelGGL(k_offmax_final, dim3(1), dim3(1024), 0, s, plan.n, plan.part.as<double>(), dev_scal,
+                       host_scal);
     MHIP_LAUNCH_CHECK();
-    MHIP_CHECK(hipMemcpyAsync(host_scal, dev_scal, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-    MHIP_CHECK(hipStreamSynchronize(s));
+    MHIP_CHECK(hipEventRecord(plan.tested, s));
+    const bool timing = plan.timing && g_kernel_variant == 1;
+    // The sweep's first launch waits on the device for the test's outcome, not
+    // for the host's: it runs while the host learns it, or does nothing.
+    const bool early = ahead && !timing && sw < max_sweeps;
+    if (early) {
+      const SweepTest test{dev_scal, tol};
+      if (sw == 0) solve(0, 0.0, test);
+      else launch_step(0, 0.0, 0, total, test);
+    }
+    MHIP_CHECK(hipEventSynchronize(plan.tested));
     const double thr = tol * std::max(1.0, host_scal[1]);
     if (host_scal[0] <= thr) break;
     // pairs whose whole 64x64 block is already this diagonal are left alone
@@ -593,21 +636,13 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
       plan.ev.assign(6 * nsteps, nullptr);
       for (auto& e : plan.ev) MHIP_CHECK(hipEventCreate(&e));
     }
-    const bool timing = plan.timing && g_kernel_variant == 1;
     // part k of the step's launch between events 2 k and 2 k + 1
     auto mark = [&](int step, int k) {
       if (timing) MHIP_CHECK(hipEventRecord(plan.ev[6 * step + k], s));
     };
     // the first step's solve of a later sweep ran in the last launch of the
     // sweep before
-    if (ahead && sw == 0) solve(0, skip_abs);
-    // A solve shares its CU with an update workgroup where two fit, and takes
-    // longer for it.  While the updates need no more than about three rounds
-    // of the chip one to a CU, they still end before the solves: LDS that is
-    // not used keeps every workgroup alone.  SCFs at 1020 orbitals (408
-    // workgroups) 53.3 -> 49.4 ms, 1200 (570) 71.2 -> 66.4, 1500 (900) equal,
-    // 1800 (1305) 133 -> 160.
-    const size_t alone = npairs + ntiles + nctiles <= 3 * 256 ? 16384 : 0;
+    if (ahead && sw == 0 && !early) solve(0, skip_abs);
     for (int step = 0; step < nsteps; ++step) {
       if (!ahead) {
         mark(step, 0);
@@ -618,31 +653,20 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
         hipLaunchKernelGGL(k_count_active, dim3(1), dim3(64), 0, s, npairs, plan.npo, aslot(slot),
                            plan.counts.as<int>() + 2 * step);
       if (g_kernel_variant == 1) {
-        const int next = (step + 1) % nsteps, first = ahead ? 0 : npairs, total = npairs + ntiles + nctiles;
-        const JacStep a{A,          ahead ? A2 : A,  C,                lda,
-                        plan.n,     npairs,          plan.npo,         ntiles,
-                        pairs_of(step), qslot(slot), aslot(slot),      pairs_of(next),
-                        intra_of(next), plan.where.as<int>() + (size_t)step * plan.nb, qslot(slot ^ 1), aslot(slot ^ 1),
-                        dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
-                        inner,      crows};
-        auto launch = [&](int from, int to) {
-          hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from);
-          MHIP_LAUNCH_CHECK();
-        };
         if (!timing) {
-          launch(first, total);
+          if (!early || sw == 0 || step > 0) launch_step(step, skip_abs, ahead ? 0 : npairs, total, {});
         } else {
           // the same work in a launch per part, for the parts' times
           if (ahead) {
             mark(step, 0);
-            launch(0, npairs);
+            launch_step(step, skip_abs, 0, npairs, {});
             mark(step, 1);
           }
           mark(step, 2);
-          launch(npairs, npairs + ntiles);
+          launch_step(step, skip_abs, npairs, npairs + ntiles, {});
           mark(step, 3);
           mark(step, 4);
-          launch(npairs + ntiles, total);
+          launch_step(step, skip_abs, npairs + ntiles, total, {});
           mark(step, 5);
         }
         if (ahead) {

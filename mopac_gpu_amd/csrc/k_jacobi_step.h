@@ -435,6 +435,20 @@ __device__ __forceinline__ void stage_q(double (&v)[SB * SB / UPD_NT], const dou
   }
 }
 
+// The outcome of a sweep's stopping test, for a launch that does not wait for
+// the host: max |off-diagonal| and max |diagonal| (stat, null where the host
+// has decided) against tol.  done() also sets what a pair is left alone below.
+struct SweepTest {
+  const double* stat = nullptr;
+  double tol = 0.0;
+  __device__ bool done(double& skip_abs) const {
+    if (!stat) return false;
+    const double thr = tol * fmax(1.0, stat[1]);
+    skip_abs = 0.1 * thr;
+    return stat[0] <= thr;
+  }
+};
+
 // One launch of the cross schedule: step s applied to A and C, and step
 // s + 1's pair problems solved.
 struct JacStep {
