@@ -503,37 +503,83 @@ __global__ __launch_bounds__(GB_NT) void k_syrk_big(int n, int k, double occ, co
       }
 }
 
-__global__ __launch_bounds__(NT) void k_syrk_packed_mfma(int n, int k, double occ, const double* a,
-                                                         int lda, double* p) {
-  __shared__ double As[TK][TB + 1];
-  __shared__ double Bs[TK][TB + 1];
+// Any n and k, lda and alignment: 64 x 64 tiles of the lower triangle, each a
+// workgroup of two groups of four waves that take the halves of every chunk of
+// 32 k and add up at the end (the tiles of 1020 orbitals, 136, leave half the
+// CUs without one as it is).  The next chunk's loads are in flight over a
+// chunk's products, with one barrier between them; four waves, a chunk of 16 k
+// at a time and its loads waited for took 109 us at 1020 orbitals (680
+// occupied) and 56 at 462, this takes 38 and 18.
+constexpr int SY_NT = 512, SY_K = 32;
+__global__ __launch_bounds__(SY_NT) void k_syrk_packed_mfma(int n, int k, double occ, const double* a,
+                                                            int lda, double* p) {
+  constexpr int S = TB + 16;  // the four k of an MFMA operand on different banks
+  __shared__ double As[2][SY_K][S];
+  __shared__ double Bs[2][SY_K][S];
   const int t = blockIdx.x;
   int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
   while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
   while (bi * (bi + 1) / 2 > t) --bi;
   const int bj = t - bi * (bi + 1) / 2;
   const int row0 = bi * TB, col0 = bj * TB;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const int half = w >> 2, qr = 32 * ((w >> 1) & 1), qc = 32 * (w & 1);
+  constexpr int NL = SY_K * TB / SY_NT;
+  double ra[NL], rb[NL];
+  auto gload = [&](int k0) {
+#pragma unroll
+    for (int r = 0; r < NL; ++r) {
+      const int e = tid + r * SY_NT, mm = e % TB, kk = e / TB;
+      ra[r] = ld_a<false>(a, lda, row0 + mm, k0 + kk, n, k);
+      rb[r] = ld_a<false>(a, lda, col0 + mm, k0 + kk, n, k);
+    }
+  };
+  auto lstore = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < NL; ++r) {
+      const int e = tid + r * SY_NT, mm = e % TB, kk = e / TB;
+      As[buf][kk][mm] = ra[r];
+      Bs[buf][kk][mm] = rb[r];
+    }
+  };
   d4_t acc[4];
   for (int i = 0; i < 4; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 0; k0 < k; k0 += TK) {
+  gload(0);
+  lstore(0);
+  __syncthreads();
+  for (int k0 = 0, cur = 0; k0 < k; k0 += SY_K, cur ^= 1) {
+    if (k0 + SY_K < k) gload(k0 + SY_K);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = tid + r * NT;
-      const int mm = e & 63, kk = e >> 6;
-      As[kk][mm] = ld_a<false>(a, lda, row0 + mm, k0 + kk, n, k);
-      Bs[kk][mm] = ld_a<false>(a, lda, col0 + mm, k0 + kk, n, k);
+    for (int ks = 0; ks < SY_K / 2; ks += 4) {
+      const int kk = half * (SY_K / 2) + ks + lk;
+      const double a0 = As[cur][kk][qr + li], a1 = As[cur][kk][qr + 16 + li];
+      const double b0 = Bs[cur][kk][qc + li], b1 = Bs[cur][kk][qc + 16 + li];
+      acc[0] = mfma16x16x4(a0, b0, acc[0]);
+      acc[1] = mfma16x16x4(a0, b1, acc[1]);
+      acc[2] = mfma16x16x4(a1, b0, acc[2]);
+      acc[3] = mfma16x16x4(a1, b1, acc[3]);
     }
-    __syncthreads();
-    mfma_tile64([&](int r, int kk) { return As[kk][r]; }, [&](int kk, int cc) { return Bs[kk][cc]; },
-                TK, acc);
+    if (k0 + SY_K < k) lstore(cur ^ 1);
     __syncthreads();
   }
-  mfma_tile64_store(acc, [&](int r, int cc, double v) {
-    const long long gr = row0 + r, gc = col0 + cc;
-    if (gr >= n || gc > gr) return;
-    p[gr * (gr + 1) / 2 + gc] = occ * v;
-  });
+  static_assert(sizeof(As) >= sizeof(double) * 4 * 16 * 64, "room for one half's sums");
+  double* part = &As[0][0][0] + (w & 3) * 16 * 64 + lane;
+  if (half == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) part[(4 * i + q) * 64] = acc[i][q];
+  }
+  __syncthreads();
+  if (half == 1) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long gr = row0 + qr + 16 * (i >> 1) + lk + 4 * q, gc = col0 + qc + 16 * (i & 1) + li;
+      if (gr < n && gc <= gr) p[gr * (gr + 1) / 2 + gc] = occ * (acc[i][q] + part[(4 * i + q) * 64]);
+    }
 }
 
 inline int cdiv(long long a, long long b) { return (int)((a + b - 1) / b); }
@@ -781,7 +827,7 @@ static void syrk_launch(hipStream_t s, int n, int k, double occ, const double* a
   }
   const int nt = cdiv(n, TB);
   if (g_kernel_variant == 1)
-    hipLaunchKernelGGL(k_syrk_packed_mfma, dim3(nt * (nt + 1) / 2), dim3(NT), 0, s, n, k, occ, a, lda, p);
+    hipLaunchKernelGGL(k_syrk_packed_mfma, dim3(nt * (nt + 1) / 2), dim3(SY_NT), 0, s, n, k, occ, a, lda, p);
   else
     hipLaunchKernelGGL(k_syrk_packed, dim3(nt * (nt + 1) / 2), dim3(NT), 0, s, n, k, occ, a, lda, p);
   MHIP_LAUNCH_CHECK();
