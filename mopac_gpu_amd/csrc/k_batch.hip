@@ -490,8 +490,8 @@ __global__ void k_bctl_post(int nmol, const int* __restrict__ list, const BatchM
 // one-centre terms), a thread per element between two atoms (its exchange
 // sum of at most 16 terms).  No partial sums go through memory, and no wave
 // is left with an atom's three or four partners: the row and column passes
-// of k_fock.hip, a wave per atom, took 95 of 105 thousand cycles beside the
-// eigensolve at 26 orbitals, this takes TODO.
+// of k_fock.hip, a wave per atom, took 95 thousand cycles at 26 orbitals,
+// this takes 20 thousand.
 template <int NT>
 __device__ void fock_small(const FockArgs& a, const int* atom_of, double* ps) {
   const int n = a.sys.norbs, tid = threadIdx.x, mp = tri(n), numat = a.sys.numat;

@@ -368,6 +368,7 @@ struct BatchJacobi {
   BjGroup g[kGroups] = {};
   DevBuf mols, st, dense, q, act, diag, counts;
   int* host = nullptr;  // pinned copy of counts
+  hipEvent_t tested = nullptr;
   int n = 0;
 };
 
@@ -436,6 +437,7 @@ BatchJacobi* bj_create(const std::vector<BatchMol>& mol, const std::vector<int>&
   j->st.ensure(sizeof(BjState) * std::max<size_t>(t.size(), 1));
   j->counts.ensure(sizeof(int) * (kMaxSweeps + 2));
   MHIP_CHECK(hipHostMalloc((void**)&j->host, sizeof(int) * (kMaxSweeps + 2), hipHostMallocDefault));
+  MHIP_CHECK(hipEventCreateWithFlags(&j->tested, hipEventDisableTiming));
   if (!t.empty()) MHIP_CHECK(hipMemcpy(j->mols.ptr, t.data(), sizeof(BjMol) * t.size(), hipMemcpyHostToDevice));
   return j;
 }
@@ -445,6 +447,7 @@ void bj_destroy(BatchJacobi* j) {
   for (auto& p : j->plan) p.release();
   for (DevBuf* b : {&j->mols, &j->st, &j->dense, &j->q, &j->act, &j->diag, &j->counts}) b->release();
   if (j->host) (void)hipHostFree(j->host);
+  if (j->tested) (void)hipEventDestroy(j->tested);
   delete j;
 }
 
@@ -488,20 +491,33 @@ int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, 
     hipLaunchKernelGGL(k_bj_test, dim3(nmol), dim3(1024), 0, s, a, sw == kMaxSweeps ? 1 : 0, counts + 1 + sw);
     MHIP_LAUNCH_CHECK();
     MHIP_CHECK(hipMemcpyAsync(j->host, counts, sizeof(int) * (kMaxSweeps + 2), hipMemcpyDeviceToHost, s));
-    MHIP_CHECK(hipStreamSynchronize(s));
-    open = j->host[0];
-    if (j->host[1 + sw] == 0) break;
-    if (sw == 0) {
-      hipLaunchKernelGGL(k_bj_first, dim3(total([](const BjGroup& g) { return g.npairs; })), dim3(CROSS_THREADS), 0, s,
-                         a);
-      MHIP_LAUNCH_CHECK();
-    }
+    MHIP_CHECK(hipEventRecord(j->tested, s));
+    // the sweep's first launches find on the device which molecules go on, and
+    // run while the host learns whether any does
     const BjLaunch whole = a;
-    for (a.step = 0; a.step < nsteps; ++a.step) {
+    auto step = [&] {
       for (int g = 0; g < kGroups; ++g) a.on[g] = whole.on[g] && a.step < a.g[g].nsteps;
       const int wgs = total([](const BjGroup& g) { return g.npairs + g.ntiles + g.nctiles; });
       hipLaunchKernelGGL(k_bj_step, dim3(wgs), dim3(CROSS_THREADS), 0, s, a);
       MHIP_LAUNCH_CHECK();
+    };
+    a.step = 0;
+    if (sw < kMaxSweeps) {
+      if (sw == 0) {
+        hipLaunchKernelGGL(k_bj_first, dim3(total([](const BjGroup& g) { return g.npairs; })), dim3(CROSS_THREADS), 0,
+                           s, a);
+        MHIP_LAUNCH_CHECK();
+      }
+      step();
+    }
+    MHIP_CHECK(hipEventSynchronize(j->tested));
+    open = j->host[0];
+    if (j->host[1 + sw] == 0) {
+      a = whole;
+      break;
+    }
+    for (; a.step < nsteps; ++a.step) {
+      if (a.step > 0) step();
       for (int g = 0; g < kGroups; ++g)
         if (a.on[g]) a.par[g] ^= 1;
     }
