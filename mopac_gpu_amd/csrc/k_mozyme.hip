@@ -82,12 +82,12 @@ __global__ void k_mz_fill_u64(long long n, unsigned long long* __restrict__ x) {
 }
 
 // bit i of bits[a * nw + i / 64]: occupied LMO i holds atom a
-__global__ void k_mz_atom_bits(LmoDev L, int nw, unsigned long long* __restrict__ bits) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.nocc) return;
+__global__ __launch_bounds__(64) void k_mz_atom_bits(LmoDev L, int nw, unsigned long long* __restrict__ bits) {
+  const int i = blockIdx.x;
   const int b0 = L.nncf[i], n = L.ncf[i];
   const unsigned long long bit = 1ull << (i & 63);
-  for (int k = 0; k < n; ++k) atomicOr(bits + (size_t)(L.icocc[b0 + k] - 1) * nw + (i >> 6), bit);
+  for (int k = threadIdx.x; k < n; k += 64)
+    atomicOr(bits + (size_t)(L.icocc[b0 + k] - 1) * nw + (i >> 6), bit);
 }
 
 // per atom: LMOs before each 64-LMO word (cum) and in all (cnt)
@@ -128,23 +128,39 @@ __global__ __launch_bounds__(1024) void k_mz_scan_counts(int n, const int* __res
   if (threadIdx.x == 0) off[n] = carry;
 }
 
+// Sums over the wave's lanes before this one, and over all of them.
+__device__ __forceinline__ int mz_wave_before(int v, int lane, int& all) {
+  int incl = v;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(incl, o);
+    if (lane >= o) incl += u;
+  }
+  all = __shfl(incl, 63);
+  return incl - v;
+}
+
 // each (LMO, atom) entry straight to its place in the atom's list, in LMO
-// order: the rank of LMO i among the atom's LMOs
-__global__ void k_mz_atom_fill(LmoDev L, int nw, const unsigned long long* __restrict__ bits,
-                               const int* __restrict__ cum, const int* __restrict__ off,
-                               int* __restrict__ ent_lmo, int* __restrict__ ent_coff) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.nocc) return;
+// order: the rank of LMO i among the atom's LMOs.  A wave per LMO, a lane per
+// atom; a thread per LMO took 43 us at 60 residues, this takes 5.
+__global__ __launch_bounds__(64) void k_mz_atom_fill(LmoDev L, int nw, const unsigned long long* __restrict__ bits,
+                                                     const int* __restrict__ cum, const int* __restrict__ off,
+                                                     int* __restrict__ ent_lmo, int* __restrict__ ent_coff) {
+  const int i = blockIdx.x, lane = threadIdx.x;
   const int b0 = L.nncf[i], n = L.ncf[i];
   const unsigned long long below = (1ull << (i & 63)) - 1ull;
   int coff = L.ncocc[i];
-  for (int k = 0; k < n; ++k) {
-    const int a = L.icocc[b0 + k] - 1;
-    const size_t wa = (size_t)a * nw + (i >> 6);
-    const int slot = off[a] + cum[wa] + __popcll(bits[wa] & below);
-    ent_lmo[slot] = i;
-    ent_coff[slot] = coff;
-    coff += L.iorbs[a];
+  for (int k0 = 0; k0 < n; k0 += 64) {
+    const bool in = k0 + lane < n;
+    const int a = in ? L.icocc[b0 + k0 + lane] - 1 : 0;
+    int all;
+    const int at = coff + mz_wave_before(in ? L.iorbs[a] : 0, lane, all);
+    if (in) {
+      const size_t wa = (size_t)a * nw + (i >> 6);
+      const int slot = off[a] + cum[wa] + __popcll(bits[wa] & below);
+      ent_lmo[slot] = i;
+      ent_coff[slot] = at;
+    }
+    coff += all;
   }
 }
 
@@ -385,18 +401,22 @@ __device__ int occ_virt_element(const LmoDev& L, const VirtLds& V, const double*
   return (lij && fabs(sum) > P.oldlim) ? 2 : 1;
 }
 
-// aocc[kk]: squared weight of the kk-th atom slot of the occupied LMOs
-__global__ void k_mz_aocc(LmoDev L, double* __restrict__ aocc) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= L.nocc) return;
-  const int loopj = L.ncocc[j];
-  int kl = 0;
-  for (int kk = L.nncf[j]; kk < L.nncf[j] + L.ncf[j]; ++kk) {
-    const int no = L.iorbs[L.icocc[kk] - 1];
+// aocc[kk]: squared weight of the kk-th atom slot of the occupied LMOs, a wave
+// per LMO and a lane per atom (a thread per LMO: 61 to 115 us at 60 residues;
+// 4 now)
+__global__ __launch_bounds__(64) void k_mz_aocc(LmoDev L, double* __restrict__ aocc) {
+  const int j = blockIdx.x, lane = threadIdx.x;
+  const int b0 = L.nncf[j], n = L.ncf[j];
+  int kl = L.ncocc[j];
+  for (int k0 = 0; k0 < n; k0 += 64) {
+    const bool in = k0 + lane < n;
+    const int no = in ? L.iorbs[L.icocc[b0 + k0 + lane] - 1] : 0;
+    int all;
+    const int at = kl + mz_wave_before(no, lane, all);
     double s = 0.0;
-    for (int x = 0; x < no; ++x) s += L.cocc[loopj + kl + x] * L.cocc[loopj + kl + x];
-    aocc[kk] = s;
-    kl += no;
+    for (int x = 0; x < no; ++x) s += L.cocc[at + x] * L.cocc[at + x];
+    if (in) aocc[b0 + k0 + lane] = s;
+    kl += all;
   }
 }
 
@@ -1596,17 +1616,6 @@ __global__ void k_mz_damp(int norbs, const int* __restrict__ idiag, const double
 
 
 // ---------------------------------------------------------------- tidy, check, eimp
-// Sums over the wave's lanes before this one, and over all of them.
-__device__ __forceinline__ int mz_wave_before(int v, int lane, int& all) {
-  int incl = v;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(incl, o);
-    if (lane >= o) incl += u;
-  }
-  all = __shfl(incl, 63);
-  return incl - v;
-}
-
 // tidy (src/MOZYME/tidy.F90:16-244), first pass, a wave per LMO and a lane per
 // atom: an atom stays when the squared sum of its coefficients, in order,
 // exceeds thresh; its flag, and the LMO's kept atom and coefficient counts.
@@ -1967,14 +1976,14 @@ void mz_density_dev(hipStream_t s, long long mpack, int nocc, int mode, const do
   hipLaunchKernelGGL(k_mz_fill_u64, dim3((int)std::min<long long>(4096, cdiv(nbits, 256))), dim3(256), 0, s, nbits,
                      bits);
   MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_mz_atom_bits, dim3(cdiv(nocc, 256)), dim3(256), 0, s, B.dev, nw, bits);
+  hipLaunchKernelGGL(k_mz_atom_bits, dim3(nocc), dim3(64), 0, s, B.dev, nw, bits);
   MHIP_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_mz_atom_cum, dim3(cdiv(numat, 256)), dim3(256), 0, s, numat, nw, bits, W.dcum.as<int>(),
                      W.dacnt.as<int>());
   MHIP_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_mz_scan_counts, dim3(1), dim3(1024), 0, s, numat, W.dacnt.as<int>(), W.daoff.as<int>());
   MHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_mz_atom_fill, dim3(cdiv(nocc, 256)), dim3(256), 0, s, B.dev, nw, bits, W.dcum.as<int>(),
+  hipLaunchKernelGGL(k_mz_atom_fill, dim3(nocc), dim3(64), 0, s, B.dev, nw, bits, W.dcum.as<int>(),
                      W.daoff.as<int>(), W.dalmo.as<int>(), W.dacoff.as<int>());
   MHIP_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_mz_density_gather, dim3(cdiv(W.nspairs, 128)), dim3(128), 0, s, B.dev, W.nspairs,
@@ -2064,7 +2073,7 @@ void mz_diagg1_dev(hipStream_t s, const mhip_lmo_set* L, const double* fao_d, co
     dfmo.ensure(sizeof(double) * fmo_dim);
     difmo.ensure(sizeof(int) * 2 * fmo_dim);
     if (L->nocc > 0) {
-      hipLaunchKernelGGL(k_mz_aocc, dim3(cdiv(L->nocc, 128)), dim3(128), 0, s, B.dev, daocc.as<double>());
+      hipLaunchKernelGGL(k_mz_aocc, dim3(L->nocc), dim3(64), 0, s, B.dev, daocc.as<double>());
       MHIP_LAUNCH_CHECK();
     }
     std::vector<int> offs(nv, 0), counts(nv, 0);

@@ -62,3 +62,31 @@ def test_tidy_keeps_and_check_scales(gpu_ctx, grown, occupied, thresh):
         scale = 1.0 / math.sqrt(total)
         assert gc[gno[k]:gno[k] + len(coefs)].tolist() == [v * scale for v in coefs]
     assert error == expected
+
+
+def test_density_from_per_atom_lists(gpu_ctx, grown):
+    """The stored blocks of 2 C C^T from the atoms' lists of LMOs."""
+    s = grown
+    c = np.zeros((s.norbs, s.nocc))
+    first = np.concatenate([[0], np.cumsum(s.iorbs)])
+    for k in range(s.nocc):
+        m = s.ncocc[k]
+        for a in s.icocc[s.nncf[k]:s.nncf[k] + s.ncf[k]]:
+            no = s.iorbs[a - 1]
+            c[first[a - 1]:first[a - 1] + no, k] = s.cocc[m:m + no]
+            m += no
+    p = 2.0 * c @ c.T
+    got = mozyme.GpuMozyme(gpu_ctx, s).density()
+    nij = np.asarray(s.nijbo)
+    seen = 0
+    for a in range(s.numat):
+        for b in range(a + 1):
+            if nij[a, b] < 0:
+                continue
+            block = p[first[a]:first[a + 1], first[b]:first[b + 1]]
+            want = block[np.tril_indices(len(block))] if a == b else block.ravel()
+            have = got[nij[a, b]:nij[a, b] + want.size]
+            # at most nocc products of numbers below 1 a sum
+            assert np.max(np.abs(have - want)) < 1e-15 * s.nocc
+            seen += want.size
+    assert seen > 1000
