@@ -502,7 +502,7 @@ def run_batch(args):
     classes = []
     for c, name in enumerate(["n<=32", "n<=64", "n<=128", "n<=256"]):
         if eig_ms[c] > 0:
-            classes.append({"class": name, "workgroup": b.tiles[c], "ms": round(float(eig_ms[c]), 2),
+            classes.append({"class": name, "ms": round(float(eig_ms[c]), 2),
                             "gflop": round(float(eig_fl[c]) / 1e9, 2), "rotations": int(eig_rot[c]),
                             "tflops": round(float(eig_fl[c]) / (eig_ms[c] * 1e-3) / 1e12, 3)})
     ach = float(eig_fl.sum()) / (float(eig_ms.sum()) * 1e-3) / 1e12
