@@ -11,8 +11,8 @@
 // In one workgroup per molecule, A packed in its LDS, a 180-orbital
 // eigensolve took 5 ms (179 rounds a sweep, each two barriers over all of A,
 // and C turned from a log of the rotations), so 50 such molecules took as
-// long as 250 would have; here a step of all molecules of a padded size is a
-// launch of 61 us on average at 150 of them (a sweep is 3, 5 or 7 steps).
+// long as 250 would have; here a step of all molecules is a launch, 55 us on
+// average with 150 of them (a sweep is 3, 5 or 7 steps).
 #include <algorithm>
 #include <vector>
 

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(256) void k_jac_apply_c(double* __restrict__ C, int
 // of a step's 37 us at 1020 orbitals (with the A update behind it, and the C
 // update on a second stream, ordered by two events per step); this launch
 // takes 22 us, of which the solve's 32 rounds are 12 and putting its problem
-// together 4.  At 3072 orbitals the updates set it (48 us).
+// together 4.  At 3072 orbitals the updates set it: 54 us, 40 in two groups.
 __global__ __launch_bounds__(CROSS_THREADS, 4) void k_jac_step(JacStep a, int base, SweepTest test) {
   static_assert(UPD_NT == CROSS_THREADS, "one workgroup size for every role");
   __shared__ JacLds lds;
