@@ -31,7 +31,7 @@ class PitchedCopy {
   static constexpr int kSlots = 2;
   static constexpr size_t kMinSlot = size_t(64) << 10, kMaxSlot = size_t(4) << 20;
   bool direct(const void* host, size_t width) const;
-  void ensure(size_t bytes, hipStream_t s);
+  void ensure(size_t width, size_t rows, hipStream_t s);
   void wait(int i);
   char* pin_ = nullptr;
   size_t slot_ = 0;

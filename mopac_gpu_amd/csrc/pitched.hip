@@ -28,11 +28,13 @@ void PitchedCopy::wait(int i) {
   busy_[i] = false;
 }
 
-// Slots of a third of `bytes` or a little less: a matrix passes in a few
-// pieces, the host's part of one beside the DMA of another.
-void PitchedCopy::ensure(size_t bytes, hipStream_t s) {
+// Slots of a third to two thirds of the matrix (within kMinSlot and kMaxSlot),
+// which then passes in a few pieces, the host's part of one beside the DMA of
+// another; and of one row at least, which `direct` keeps below kMaxSlot.
+void PitchedCopy::ensure(size_t width, size_t rows, hipStream_t s) {
   size_t want = kMinSlot;
-  while (want < kMaxSlot && 3 * want < bytes) want *= 2;
+  while (want < kMaxSlot && (want < width || 3 * want < width * rows)) want *= 2;
+  MHIP_REQUIRE(want >= width, "copy through pinned slots: row longer than a slot");
   if (want <= slot_) return;
   release();
   MHIP_CHECK(hipHostMalloc((void**)&pin_, want * kSlots, hipHostMallocDefault));
@@ -62,10 +64,10 @@ void PitchedCopy::up(void* dst, size_t dpitch, const void* src, size_t spitch, s
     MHIP_CHECK(hipMemcpy2DAsync(dst, dpitch, src, spitch, width, rows, hipMemcpyHostToDevice, s));
     return;
   }
-  ensure(width * rows, s);
+  ensure(width, rows, s);
   wait(0);
   wait(1);
-  const size_t per = std::max<size_t>(1, slot_ / width);
+  const size_t per = slot_ / width;
   int i = 0;
   for (size_t r = 0; r < rows; r += per, i ^= 1) {
     const size_t n = std::min(per, rows - r);
@@ -93,10 +95,10 @@ void PitchedCopy::down(void* dst, size_t dpitch, const void* src, size_t spitch,
     MHIP_CHECK(hipStreamSynchronize(s));
     return;
   }
-  ensure(width * rows, s);
+  ensure(width, rows, s);
   wait(0);
   wait(1);
-  const size_t per = std::max<size_t>(1, slot_ / width);
+  const size_t per = slot_ / width;
   auto issue = [&](size_t r, int i) {
     MHIP_CHECK(hipMemcpy2DAsync(pin_ + i * slot_, width, static_cast<const char*>(src) + r * spitch, spitch, width,
                                 std::min(per, rows - r), hipMemcpyDeviceToHost, s));

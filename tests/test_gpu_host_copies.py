@@ -9,12 +9,17 @@ pytestmark = pytest.mark.gpu
 
 
 # one value; columns without gaps; ragged ones in one and in several pieces;
-# 13 and 27 MB (slots at their largest); one column longer than a slot
+# 13 and 27 MB (slots at their largest); one and two columns of 64 KB to 4 MB,
+# each as long as a slot or longer than a third of the matrix; columns longer
+# than the largest slot
 @pytest.mark.parametrize("m,n,pad", [(1, 1, 0), (1, 40, 3), (7, 301, 2), (300, 77, 0), (123, 701, 5),
-                                     (1237, 1301, 5), (1901, 1777, 1), (600001, 2, 3)])
+                                     (1237, 1301, 5), (1901, 1777, 1), (8193, 2, 3),
+                                     (9000, 2, 3), (12000, 2, 3), (20000, 1, 3), (24000, 1, 3), (40000, 2, 1),
+                                     (524288, 2, 3), (600001, 2, 3)])
 def test_pitched_copies_touch_only_their_rows(gpu_ctx, m, n, pad):
     rng = np.random.default_rng(m + n)
     lib, ld = L.load(), m + pad
+    lib.mhip_destroy_resources()  # slots only grow: these are this matrix's own
     a = np.asfortranarray(rng.integers(-8, 9, (ld, 1)).astype(float))
     b = np.asfortranarray(rng.integers(-8, 9, (1, n)).astype(float))
     c = np.asfortranarray(rng.integers(-8, 9, (ld, n)).astype(float))
