@@ -6,6 +6,7 @@
 #include <utility>
 
 #include "common.h"
+#include "jacobi_rotation.h"
 #include "mfma.h"
 
 namespace mhip {
@@ -23,39 +24,6 @@ __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   return v;
-}
-
-// Rotation by the smaller of the angles that zero apq in [[app, apq], [apq,
-// aqq]]: with d = aqq - app, h = 2 apq and r = sqrt(d^2 + h^2), c^2 = (1 +
-// |d| / r) / 2 and s = sign(d) h / (2 r c); t = s / c, and the diagonal after
-// it is app - t apq, aqq + t apq.  c and s start in FP32 (a reciprocal square
-// root is one instruction there), an FP64 step turns them by what they leave
-// of apq (angle good to about 1e-14), and they are scaled to c^2 + s^2 = 1 in
-// FP64 to the last bit.  Every round of a pair solve waits for this chain of
-// 17 dependent operations; FP64 division and square roots take 100.  With
-// apq and d both below 1e-15, far under any stopping threshold (they are
-// absolute), nothing is turned.
-__device__ __forceinline__ void rotation_of(double app, double aqq, double apq, double& c, double& sn,
-                                            double& t) {
-  const double d = aqq - app;
-  const float df = (float)d, ad = fabsf(df), hh = (float)apq;
-  const float r2 = fmaf(4.0f * hh, hh, ad * ad);
-  const float rinv = __builtin_amdgcn_rsqf(r2);
-  const float c2 = fmaf(0.5f * ad, rinv, 0.5f);
-  const float cinv = __builtin_amdgcn_rsqf(c2);
-  const bool none = r2 < 1.0e-30f;
-  const float cf = none ? 1.0f : c2 * cinv, sf = none ? 0.0f : copysignf(1.0f, df) * hh * rinv * cinv;
-  double c0 = (double)cf, s0 = (double)sf;
-  // the off-diagonal element after the rotation, over sign(d) r
-  const double left = fma(fma(c0, c0, -s0 * s0), apq, -(c0 * s0) * d);
-  const double turn = left * (double)(none ? 0.0f : copysignf(rinv, df));
-  const double c1 = fma(-turn, s0, c0), s1 = fma(turn, c0, s0);
-  const double e = fma(-c1, c1, fma(-s1, s1, 1.0));
-  const double corr = fma(e, fma(e, 0.375, 0.5), 1.0);
-  c = c1 * corr;
-  sn = s1 * corr;
-  const double ci = none ? 1.0 : (double)cinv;
-  t = sn * (ci * fma(-c, ci, 2.0));  // s / c, 1 / c by a Newton step from FP32's
 }
 
 // The value of lane (lane ^ MASK) for the masks the cross rounds step by:
