@@ -309,13 +309,14 @@ __global__ __launch_bounds__(512) void k_bj_order(BjLaunch a, BatchState* __rest
   const BjMol& M = a.mol[m];
   const int np = M.npad, tid = threadIdx.x;
   const double* A = M.A[s.cur];
-  if (tid < np) d[tid] = A[(size_t)tid + (size_t)tid * np];
+  const double level = tid < np ? A[(size_t)tid + (size_t)tid * np] : 0.0, key = sort_key(level);
+  if (tid < np) d[tid] = key;
   __syncthreads();
   if (tid < np) {
     int rank = 0;
-    for (int j = 0; j < np; ++j) rank += (d[j] < d[tid]) || (d[j] == d[tid] && j < tid);
+    for (int j = 0; j < np; ++j) rank += (d[j] < key) || (d[j] == key && j < tid);
     from[rank] = tid;
-    if (rank < M.n) M.eig[rank] = d[tid];
+    if (rank < M.n) M.eig[rank] = level;
   }
   __syncthreads();
   for (int e = tid; e < np * np; e += 512) M.Cs[e] = M.C[(size_t)(e % np) + (size_t)from[e / np] * np];

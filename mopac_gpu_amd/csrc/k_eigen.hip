@@ -405,11 +405,12 @@ __global__ __launch_bounds__(64 * SORT_WAVES) void k_sort_diag(int npad, const d
   __shared__ int below[SORT_WAVES][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
-  const double di = (i < npad) ? A[(size_t)i + (size_t)i * lda] : 0.0;
+  const double level = (i < npad) ? A[(size_t)i + (size_t)i * lda] : 0.0, di = sort_key(level);
   int rank = 0;
   for (int j0 = 0; j0 < npad; j0 += SORT_CHUNK) {
     const int nj = min(SORT_CHUNK, npad - j0);
-    for (int j = threadIdx.x; j < nj; j += 64 * SORT_WAVES) d[j] = A[(size_t)(j0 + j) + (size_t)(j0 + j) * lda];
+    for (int j = threadIdx.x; j < nj; j += 64 * SORT_WAVES)
+      d[j] = sort_key(A[(size_t)(j0 + j) + (size_t)(j0 + j) * lda]);
     __syncthreads();
 #pragma unroll 8
     for (int j = w; j < nj; j += SORT_WAVES) {
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(64 * SORT_WAVES) void k_sort_diag(int npad, const d
   if (w == 0 && i < npad) {
     for (int v = 1; v < SORT_WAVES; ++v) rank += below[v][lane];
     perm[rank] = i;
-    eig[rank] = di;
+    eig[rank] = level;
   }
 }
 

@@ -20,6 +20,10 @@ __device__ __forceinline__ int gidx_dev(int pairI, int pairJ, int local) {
   return (local < BS) ? pairI * BS + local : pairJ * BS + (local - BS);
 }
 
+// What levels are ordered by: a NaN is above all others, so that every level
+// has a place of its own whatever a matrix holds.
+__device__ __forceinline__ double sort_key(double level) { return level == level ? level : __builtin_huge_val(); }
+
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));

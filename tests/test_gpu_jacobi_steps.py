@@ -51,3 +51,17 @@ def test_eigenpairs(n, kind):
     assert np.abs(a @ v - v * w).max() <= (1.0e-12 * np.sqrt(n) + rot) * top
     assert np.abs(w - np.linalg.eigvalsh(a)).max() <= (1.0e-12 * np.sqrt(n) + rot) * max(top, scale)
     assert np.all(np.diff(w) >= 0.0)
+
+
+@pytest.mark.parametrize("n", (33, 64, 130))
+def test_nan_has_a_place_in_the_order(n):
+    """A NaN spreads over the levels and vectors; each keeps a place of its own
+    (their order is an index), and the next matrix is not touched by it."""
+    a = _matrix("dense", n)
+    a[0, n - 1] = a[n - 1, 0] = np.nan
+    v = np.array(a, order="F")
+    w = np.zeros(n)
+    info = ctypes.c_int(-9)
+    L.load().mhip_dsyevd(n, L.ptr(v), n, L.ptr(w), ctypes.byref(info))
+    assert info.value != 0 or np.isnan(v).any()
+    test_eigenpairs(n, "dense")
