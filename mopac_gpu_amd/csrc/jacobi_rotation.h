@@ -10,11 +10,12 @@ namespace {
 // it is app - t apq, aqq + t apq.  c and s start in FP32 (a reciprocal square
 // root is one instruction there), an FP64 step turns them by what they leave
 // of apq, and they are scaled to c^2 + s^2 = 1 in FP64.  The turn is what is
-// left over (c0^2 + s0^2) r, with both factors to FP64's second order: an
-// FP32 1 / r alone, good to 3e-7, left 1e-13 r of the element that is then
-// taken for zero.  Over 10^6 pairs it is 1.6e-16 r at most, and 2.0e-16 with
-// FP64 division and square roots throughout; c^2 + s^2 is 1 to 4e-16.
-// Every round of a pair solve waits for this chain of 19 dependent operations;
+// left over the levels' distance, whose reciprocal is FP32's 1 / r after a
+// Newton step: with that 1 / r itself, good to 3e-7, 1e-13 r was left of an
+// element that is then taken for zero.  Over 10^6 pairs 1.6e-16 r is left at
+// most, 2.0e-16 with FP64 division and square roots throughout, and c^2 + s^2
+// is 1 to 4e-16.
+// Every round of a pair solve waits for this chain of 18 dependent operations;
 // FP64 division and square roots take 100.  With apq and d both below 1e-15,
 // far under any stopping threshold (they are absolute), nothing is turned.
 __device__ __forceinline__ void rotation_of(double app, double aqq, double apq, double& c, double& sn,
@@ -28,13 +29,12 @@ __device__ __forceinline__ void rotation_of(double app, double aqq, double apq, 
   const bool none = r2 < 1.0e-30f;
   const float cf = none ? 1.0f : c2 * cinv, sf = none ? 0.0f : copysignf(1.0f, df) * hh * rinv * cinv;
   const double c0 = (double)cf, s0 = (double)sf;
-  // 1 / ((c0^2 + s0^2) r) is rinv (1 + more): a Newton step for r, the first
-  // order for the length
-  const double ri = (double)(none ? 0.0f : rinv), s02 = s0 * s0;
-  const double more = fma(-0.5, fma(d, d, 4.0 * apq * apq) * (ri * ri), 1.5) - fma(c0, c0, s02);
-  // the off-diagonal element after the rotation, over sign(d) r
-  const double left = fma(fma(c0, c0, -s02), apq, -(c0 * s0) * d);
-  const double turn1 = left * copysign(ri, d), turn = fma(turn1, more, turn1);
+  const double p = fma(c0, c0, -s0 * s0), q = c0 * s0;
+  // the off-diagonal element and the levels' distance after that rotation
+  const double left = fma(p, apq, -q * d), dist = fma(p, d, q * (4.0 * apq));
+  // left / dist, 1 / dist by a Newton step from FP32's 1 / r
+  const double ri = (double)(none ? 0.0f : copysignf(rinv, df));
+  const double turn = left * ri * fma(-dist, ri, 2.0);
   const double c1 = fma(-turn, s0, c0), s1 = fma(turn, c0, s0);
   const double e = fma(-c1, c1, fma(-s1, s1, 1.0));
   const double corr = fma(e, fma(e, 0.375, 0.5), 1.0);
