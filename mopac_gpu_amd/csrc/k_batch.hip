@@ -389,7 +389,7 @@ __device__ __noinline__ EigCount beig_lds(JacLds& lds, const BatchMol& M, double
     }
   }
   __syncthreads();
-  const int sweeps = pair_solve(lds, 0, 1, true, JacSolve{n, nullptr, nullptr, nullptr, nullptr, tol, 0.0, kEigSweeps});
+  const int sweeps = pair_solve<true>(lds, 0, 1, true, JacSolve{n, nullptr, nullptr, nullptr, nullptr, tol, 0.0, kEigSweeps});
   // ascending order, ties by index; the padding stays where it is
   if (tid < SB) {
     const double d = S[tid][tid];

@@ -46,6 +46,7 @@ struct BjState {
   int did;         // this call diagonalizes the molecule
   int cur;         // which A holds the result
   int sweeps;
+  int scale;       // A is the matrix times 2^-scale
   double skip;     // pairs this diagonal are left alone
   unsigned long long rot;
 };
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(256) void k_bj_begin(const BjMol* __restrict__ mols
   if (go)
     for (int k = threadIdx.x; k < M.n; k += 256) M.f[(size_t)k * (k + 1) / 2 + k] += (double)(k + 1) * 1.0e-10;
   if (threadIdx.x == 0) {
-    st[i] = BjState{go ? 1 : 0, go ? 1 : 0, 0, 0, 0.0, 0ull};
+    st[i] = BjState{go ? 1 : 0, go ? 1 : 0, 0, 0, 0, 0.0, 0ull};
     if (!bst[M.mol].done) atomicAdd(counts, 1);
   }
 }
@@ -207,13 +208,15 @@ __global__ __launch_bounds__(UPD_NT) void k_bj_ctf(BjLaunch a, const BatchState*
 }
 
 // max|offdiag| <= tol max(1, max|diag|) over the molecule's n x n block: stop,
-// or go on with the pairs that are not yet a tenth of that
-__global__ __launch_bounds__(1024) void k_bj_test(BjLaunch a, int last, int* __restrict__ count) {
+// or go on with the pairs that are not yet a tenth of that.  A matrix out of
+// the angles' range is scaled before its first sweep, its largest element to
+// 2^10.
+__global__ __launch_bounds__(1024) void k_bj_test(BjLaunch a, int sweep, int last, int* __restrict__ count) {
   int b = blockIdx.x, g, m;
   if (!locate(a, b, g, m, [](const BjGroup&) { return 1; })) return;
   if (!a.st[m].run) return;
   const BjMol& M = a.mol[m];
-  const double* A = M.A[a.par[g]];
+  double* A = M.A[a.par[g]];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   double off = 0.0, dg = 0.0;
   for (int c = w; c < M.n; c += 16)
@@ -230,12 +233,19 @@ __global__ __launch_bounds__(1024) void k_bj_test(BjLaunch a, int last, int* __r
     rd[w] = dg;
   }
   __syncthreads();
-  if (tid != 0) return;
-  for (int i = 1; i < 16; ++i) {
+  for (int i = 0; i < 16; ++i) {
     off = fmax(off, ro[i]);
     dg = fmax(dg, rd[i]);
   }
   BjState& s = a.st[m];
+  if (const double top = fmax(off, dg); sweep == 0 && out_of_range(top)) {
+    const int e = ilogb(top) - 10;
+    for (int i = tid; i < M.npad * M.npad; i += 1024) A[i] = ldexp(A[i], -e);
+    off = ldexp(off, -e);
+    dg = ldexp(dg, -e);
+    if (tid == 0) s.scale = e;
+  }
+  if (tid != 0) return;
   const double thr = a.tol * fmax(1.0, dg);
   s.cur = a.par[g];
   if (off <= thr || last) {
@@ -309,7 +319,7 @@ __global__ __launch_bounds__(512) void k_bj_order(BjLaunch a, BatchState* __rest
   const BjMol& M = a.mol[m];
   const int np = M.npad, tid = threadIdx.x;
   const double* A = M.A[s.cur];
-  const double level = tid < np ? A[(size_t)tid + (size_t)tid * np] : 0.0, key = sort_key(level);
+  const double level = tid < np ? ldexp(A[(size_t)tid + (size_t)tid * np], s.scale) : 0.0, key = sort_key(level);
   if (tid < np) d[tid] = key;
   __syncthreads();
   if (tid < np) {
@@ -489,7 +499,8 @@ int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, 
   MHIP_LAUNCH_CHECK();
   int open = 0;
   for (int sw = 0; sw <= kMaxSweeps; ++sw) {
-    hipLaunchKernelGGL(k_bj_test, dim3(nmol), dim3(1024), 0, s, a, sw == kMaxSweeps ? 1 : 0, counts + 1 + sw);
+    hipLaunchKernelGGL(k_bj_test, dim3(nmol), dim3(1024), 0, s, a, sw, sw == kMaxSweeps ? 1 : 0,
+                       counts + 1 + sw);
     MHIP_LAUNCH_CHECK();
     MHIP_CHECK(hipMemcpyAsync(j->host, counts, sizeof(int) * (kMaxSweeps + 2), hipMemcpyDeviceToHost, s));
     MHIP_CHECK(hipEventRecord(j->tested, s));

@@ -10,6 +10,9 @@
 // In the SCF the solver starts from the previous eigenvectors (A = C^T F C is
 // then nearly diagonal and one to three sweeps converge it); the first call
 // starts from C = I.  Stopping test: max |A_ij| (i != j) <= tol * max|A_ii|.
+#include <algorithm>
+#include <cmath>
+
 #include "common.h"
 #include "k_eigen.h"
 #include "k_jacobi_step.h"
@@ -381,6 +384,12 @@ __global__ __launch_bounds__(1024) void k_offmax_final(int n, const double* __re
   }
 }
 
+// A by 2^e
+__global__ __launch_bounds__(256) void k_scale_by_power(long long len, double* __restrict__ A, int e) {
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < len; i += (long long)gridDim.x * 256)
+    A[i] = ldexp(A[i], e);
+}
+
 // active pairs of the step in each group: out[0] over [0, npo), out[1] over [npo, npairs)
 __global__ void k_count_active(int npairs, int npo, const int* __restrict__ active, int* __restrict__ out) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
@@ -561,8 +570,11 @@ void jacobi_set_identity(hipStream_t s, int npad, double* C, int ldc) {
   MHIP_LAUNCH_CHECK();
 }
 
-int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
-                  double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks) {
+// jacobi_sweeps on a matrix whose elements end at kAngleRange in the cross
+// schedule; one with larger ones is left alone, and returns 2 with the test's
+// two values in host_scal.
+static int sweeps_in_range(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol,
+                           int max_sweeps, double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks) {
   const int lda = plan.npad;
   int done = 0;
   // Inner sweeps per step.  Cross schedule: one; a second saves up to a fifth
@@ -627,13 +639,15 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
     // for the host's: it runs while the host learns it, or does nothing.
     const bool early = ahead && !timing && sw < max_sweeps;
     if (early) {
-      const SweepTest test{dev_scal, tol};
+      const SweepTest test{dev_scal, tol, sw == 0};
       if (sw == 0) solve(0, 0.0, test);
       else launch_step(0, 0.0, 0, total, test);
     }
     MHIP_CHECK(hipEventSynchronize(plan.tested));
     const double thr = tol * std::max(1.0, host_scal[1]);
     if (host_scal[0] <= thr) break;
+    const double top = std::max(host_scal[0], host_scal[1]);
+    if (cross && sw == 0 && top > kAngleRange && std::isfinite(top)) return 2;
     // pairs whose whole 64x64 block is already this diagonal are left alone
     const double skip_abs = 0.1 * thr;
     if (sw == max_sweeps) {
@@ -724,6 +738,25 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
   }
   if (sweeps_done) *sweeps_done = done;
   return 0;
+}
+
+int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, double* C, double tol, int max_sweeps,
+                  double* host_scal, double* dev_scal, int* sweeps_done, bool c_blocks) {
+  int rc = sweeps_in_range(s, plan, A, A2, C, tol, max_sweeps, host_scal, dev_scal, sweeps_done, c_blocks);
+  if (rc != 2) return rc;
+  // the largest element to 2^10, above the 1 that the stopping test takes for
+  // the diagonal of a smaller one
+  const int e = std::ilogb(std::max(host_scal[0], host_scal[1])) - 10;
+  const long long len = (long long)plan.npad * plan.npad;
+  auto scale = [&](int by) {
+    hipLaunchKernelGGL(k_scale_by_power, dim3((int)std::min<long long>(4096, (len + 255) / 256)), dim3(256), 0, s, len,
+                       A, by);
+    MHIP_LAUNCH_CHECK();
+  };
+  scale(-e);
+  rc = sweeps_in_range(s, plan, A, A2, C, tol, max_sweeps, host_scal, dev_scal, sweeps_done, c_blocks);
+  scale(e);
+  return rc;
 }
 
 void jacobi_sort(hipStream_t s, JacobiPlan& plan, const double* A, const double* C, double* Cout,

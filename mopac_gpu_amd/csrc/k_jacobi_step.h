@@ -20,6 +20,14 @@ __device__ __forceinline__ int gidx_dev(int pairI, int pairJ, int local) {
   return (local < BS) ? pairI * BS + local : pairJ * BS + (local - BS);
 }
 
+// The angles start in FP32: a problem with elements above this is solved as a
+// power of two times one with elements up to 1, which has the same rotations.
+// r^2 of a pair is at most (2 x 64 x 2^50)^2 in a 64 x 64 problem.
+constexpr double kAngleRange = 0x1p50;
+__device__ __forceinline__ bool out_of_range(double top) {
+  return top > kAngleRange && top < __builtin_huge_val();
+}
+
 // What levels are ordered by: a NaN is above all others, so that every level
 // has a place of its own whatever a matrix holds.
 __device__ __forceinline__ double sort_key(double level) { return level == level ? level : __builtin_huge_val(); }
@@ -237,10 +245,18 @@ __device__ __forceinline__ void exchange_q(CrossRegs& v, int k, int j) {
   }
 }
 
+// S by 2^e
+__device__ __noinline__ void scale_problem(double (*S)[SB], int e) {
+  for (int i = threadIdx.x; i < SB * SB; i += CROSS_THREADS) S[i / SB][i % SB] = ldexp(S[i / SB][i % SB], e);
+  __syncthreads();
+}
+
 // Diagonalizes the problem in lds.s(): the upper right quadrant and the two
 // diagonal ones, and the lower left one where do_intra asks for it.  Returns
 // the inner sweeps it took (0: nothing rotated); with p.q null, Q is left in
-// lds.q() and S in lds.s().
+// lds.q() and S in lds.s().  ANY: of any size; elsewhere the matrix is in the
+// angles' range (a test here costs a step of the solver 0.7%).
+template <bool ANY = false>
 __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_intra, const JacSolve& p) {
   double(*S)[SB] = lds.s();
   double(*Q)[LDSW] = lds.q();
@@ -254,7 +270,7 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
     v.ql[j] = (4 * g + j == k) ? 1.0 : 0.0;
     v.qr[j] = (4 * g + j == 32 + k) ? 1.0 : 0.0;
   }
-  int sweeps = 0;
+  int sweeps = 0, scale = 0;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // a round ends with the angles of the next, which wave 7 computes in three
   // of four rounds, 6, 5 or 0 in the others, while two waves share each SIMD:
@@ -283,7 +299,14 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
       dg = fmax(dg, lds.red_dg[w]);
     }
     __syncthreads();
-    if ((sw == 0 && off <= p.skip_abs) || off <= p.tol * fmax(dg, 1.0)) break;
+    if ((sw == 0 && off <= p.skip_abs) || off <= p.tol * fmax(dg, ANY ? ldexp(1.0, -scale) : 1.0)) break;
+    if constexpr (ANY) {
+      const double top = fmax(off, dg);
+      if (sw == 0 && out_of_range(top)) {
+        scale = __builtin_amdgcn_readfirstlane(ilogb(top) + 1);
+        scale_problem(S, -scale);
+      }
+    }
     ++sweeps;
     for (int lv = do_intra ? 0 : 5; lv < 6; ++lv) {
       // nothing to rotate between a real index and the padding (a matrix that
@@ -341,6 +364,7 @@ __device__ __forceinline__ int pair_solve(JacLds& lds, int I, int J, bool do_int
     }
   }
   __builtin_amdgcn_s_setprio(0);
+  if (ANY && scale) scale_problem(S, scale);
   if (p.di) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -413,11 +437,12 @@ __device__ __forceinline__ void stage_q(double (&v)[SB * SB / UPD_NT], const dou
 struct SweepTest {
   const double* stat = nullptr;
   double tol = 0.0;
+  bool first = false;  // of the sweeps: nothing is done out of the angles' range
   __device__ bool done(double& skip_abs) const {
     if (!stat) return false;
     const double thr = tol * fmax(1.0, stat[1]);
     skip_abs = 0.1 * thr;
-    return stat[0] <= thr;
+    return stat[0] <= thr || (first && out_of_range(fmax(stat[0], stat[1])));
   }
 };
 

@@ -1,6 +1,8 @@
 """The batched SCF's two forms at the edges of their ranges: one workgroup for
 a molecule up to 64 orbitals, block-Jacobi steps over several above (padded
 sizes 128, 192 and 256), and the single-molecule SCF that shares the first."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,25 @@ def test_single_molecule_in_one_workgroup_matches_the_general_path(systems, m):
     f = f + np.tril(f, -1).T
     assert np.max(np.abs(a["c"].T @ a["c"] - np.eye(n))) < 1e-11
     assert np.max(np.abs(f @ a["c"] - a["c"] * a["eig"])) < 1e-8  # F(i,i) + i*1e-10 is what is diagonalized
+
+
+@pytest.mark.parametrize("scale", (1.0, 1e20, 1e40))
+@pytest.mark.parametrize("mol", [("water", 5)])
+def test_levels_of_any_size(mol, scale):
+    """One iteration on an H whose levels are evenly spread over -scale to
+    scale: the density is that of H's own lower levels."""
+    s = hamiltonian.build(*MAKE[mol[0]](mol[1], 17))
+    n = s.norbs
+    rng = np.random.default_rng(n)
+    v = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    h = (v * (scale * np.linspace(-1.0, 1.0, n))) @ v.T
+    # no integrals: F is H, and a level shift of the starting diagonal
+    s = dataclasses.replace(s, h=h[np.tril_indices(n)], w=np.zeros_like(s.w), pdiag=np.full(n, 2.0 * s.nclose / n))
+    b = B.Batch([s], scfcrt=1e-6)
+    b.run(iters_per_graph=1, max_launches=1)
+    p = b.density(0)
+    b.close()
+    want = 2.0 * v[:, :s.nclose] @ v[:, :s.nclose].T
+    # residuals of 1e-10 of the largest level over the gap of 2 / (n - 1), on up
+    # to n elements
+    assert np.max(np.abs(p - want[np.tril_indices(n)])) < 1e-10 * n * n

@@ -65,3 +65,21 @@ def test_nan_has_a_place_in_the_order(n):
     L.load().mhip_dsyevd(n, L.ptr(v), n, L.ptr(w), ctypes.byref(info))
     assert info.value != 0 or np.isnan(v).any()
     test_eigenpairs(n, "dense")
+
+
+@pytest.mark.parametrize("scale", (1e18, 1e20, 1e40, 1e150))
+@pytest.mark.parametrize("n", (64, 128, 192))
+def test_eigenpairs_of_huge_matrices(n, scale):
+    """The rotations' angles start in FP32, whose squares end at 3e38; without
+    padding the matrix may have any size.  Same bounds as above."""
+    a = _matrix("dense", n)
+    v = np.array(scale * a, order="F")
+    w = np.zeros(n)
+    info = ctypes.c_int(-9)
+    L.load().mhip_dsyevd(n, L.ptr(v), n, L.ptr(w), ctypes.byref(info))
+    assert info.value == 0
+    rot = 12 * 4 * n * EPS
+    top = np.abs(np.linalg.eigvalsh(a)).max()
+    assert np.abs(v.T @ v - np.eye(n)).max() <= rot
+    assert np.abs(a @ v - v * (w / scale)).max() <= (1.0e-12 * np.sqrt(n) + rot) * top
+    assert np.abs(w / scale - np.linalg.eigvalsh(a)).max() <= (1.0e-12 * np.sqrt(n) + rot) * top
