@@ -319,7 +319,8 @@ __global__ __launch_bounds__(512) void k_bj_order(BjLaunch a, BatchState* __rest
   const BjMol& M = a.mol[m];
   const int np = M.npad, tid = threadIdx.x;
   const double* A = M.A[s.cur];
-  const double level = tid < np ? ldexp(A[(size_t)tid + (size_t)tid * np], s.scale) : 0.0, key = sort_key(level);
+  const double level = tid < np ? ldexp(A[(size_t)tid + (size_t)tid * np], s.scale) : 0.0;
+  const double key = sort_key(level, tid, M.n);
   if (tid < np) d[tid] = key;
   __syncthreads();
   if (tid < np) {

@@ -408,18 +408,18 @@ __global__ void k_count_active(int npairs, int npo, const int* __restrict__ acti
 // through LDS in chunks.  A thread per entry compared with all of them, in
 // four workgroups at 1020 orbitals, took 74 us; this takes 12.
 constexpr int SORT_CHUNK = 2048, SORT_WAVES = 8;
-__global__ __launch_bounds__(64 * SORT_WAVES) void k_sort_diag(int npad, const double* __restrict__ A, int lda,
+__global__ __launch_bounds__(64 * SORT_WAVES) void k_sort_diag(int n, int npad, const double* __restrict__ A, int lda,
                                                                int* __restrict__ perm, double* __restrict__ eig) {
   __shared__ double d[SORT_CHUNK];
   __shared__ int below[SORT_WAVES][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
-  const double level = (i < npad) ? A[(size_t)i + (size_t)i * lda] : 0.0, di = sort_key(level);
+  const double level = (i < npad) ? A[(size_t)i + (size_t)i * lda] : 0.0, di = sort_key(level, i, n);
   int rank = 0;
   for (int j0 = 0; j0 < npad; j0 += SORT_CHUNK) {
     const int nj = min(SORT_CHUNK, npad - j0);
     for (int j = threadIdx.x; j < nj; j += 64 * SORT_WAVES)
-      d[j] = sort_key(A[(size_t)(j0 + j) + (size_t)(j0 + j) * lda]);
+      d[j] = sort_key(A[(size_t)(j0 + j) + (size_t)(j0 + j) * lda], j0 + j, n);
     __syncthreads();
 #pragma unroll 8
     for (int j = w; j < nj; j += SORT_WAVES) {
@@ -762,7 +762,7 @@ int jacobi_sweeps(hipStream_t s, JacobiPlan& plan, double*& A, double*& A2, doub
 void jacobi_sort(hipStream_t s, JacobiPlan& plan, const double* A, const double* C, double* Cout,
                  double* eig_dev) {
   const int npad = plan.npad;
-  hipLaunchKernelGGL(k_sort_diag, dim3((npad + 63) / 64), dim3(64 * SORT_WAVES), 0, s, npad, A, npad,
+  hipLaunchKernelGGL(k_sort_diag, dim3((npad + 63) / 64), dim3(64 * SORT_WAVES), 0, s, plan.n, npad, A, npad,
                      plan.perm.as<int>(), eig_dev);
   MHIP_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_permute_cols, dim3((npad + 255) / 256, npad), dim3(256), 0, s, npad, npad, C,

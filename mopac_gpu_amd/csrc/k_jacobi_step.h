@@ -28,9 +28,12 @@ __device__ __forceinline__ bool out_of_range(double top) {
   return top > kAngleRange && top < __builtin_huge_val();
 }
 
-// What levels are ordered by: a NaN is above all others, so that every level
-// has a place of its own whatever a matrix holds.
-__device__ __forceinline__ double sort_key(double level) { return level == level ? level : __builtin_huge_val(); }
+// What the levels of n orbitals are ordered by: a NaN is above all others, so
+// that every level has a place of its own whatever a matrix holds, and the
+// padding after them, whatever they are (ties go by index).
+__device__ __forceinline__ double sort_key(double level, int i, int n) {
+  return i < n && level == level ? level : __builtin_huge_val();
+}
 
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll

@@ -88,8 +88,8 @@ def test_single_molecule_in_one_workgroup_matches_the_general_path(systems, m):
     assert np.max(np.abs(f @ a["c"] - a["c"] * a["eig"])) < 1e-8  # F(i,i) + i*1e-10 is what is diagonalized
 
 
-@pytest.mark.parametrize("scale", (1.0, 1e20, 1e40))
-@pytest.mark.parametrize("mol", [("water", 5)])
+@pytest.mark.parametrize("scale", (1.0, 1e6, 1e20, 1e40))
+@pytest.mark.parametrize("mol", [("water", 5), ("water", 11), ("water", 22), ("water", 32), ("water", 33)])
 def test_levels_of_any_size(mol, scale):
     """One iteration on an H whose levels are evenly spread over -scale to
     scale: the density is that of H's own lower levels."""

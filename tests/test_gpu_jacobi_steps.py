@@ -67,11 +67,11 @@ def test_nan_has_a_place_in_the_order(n):
     test_eigenpairs(n, "dense")
 
 
-@pytest.mark.parametrize("scale", (1e18, 1e20, 1e40, 1e150))
-@pytest.mark.parametrize("n", (64, 128, 192))
+@pytest.mark.parametrize("scale", (1e5, 1e18, 1e20, 1e40, 1e150))
+@pytest.mark.parametrize("n", (33, 64, 128, 130, 192))
 def test_eigenpairs_of_huge_matrices(n, scale):
-    """The rotations' angles start in FP32, whose squares end at 3e38; without
-    padding the matrix may have any size.  Same bounds as above."""
+    """The rotations' angles start in FP32, whose squares end at 3e38, and the
+    padding's entries are about 1e4.  Same bounds as above."""
     a = _matrix("dense", n)
     v = np.array(scale * a, order="F")
     w = np.zeros(n)
