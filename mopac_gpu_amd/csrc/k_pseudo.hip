@@ -159,6 +159,11 @@ __global__ __launch_bounds__(256) void k_rotate(int n, int ldc, double* __restri
       }
     }
     if (have) *col = b;
+    // every lane reads what lane 63 stored: not before this point, and not
+    // from before it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __syncthreads();
   for (int e = tid; e < rows * nocc; e += blockDim.x) {
