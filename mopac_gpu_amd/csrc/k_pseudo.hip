@@ -51,12 +51,13 @@ __global__ __launch_bounds__(256) void k_absmax_final(int nb, const double* __re
 
 // Rotation parameters for every (virtual, occupied) pair, exactly as
 // diag.F90:130-153 computes them, in the order k_rotate reads them: entry
-// [b][t][l] is virtual 64 b + l with occupied t - l, kSkip where the pair is
-// not rotated or there is none.
+// [b][t][l] is virtual 64 b + l with occupied j0 + t - l of the nj from j0 on,
+// kSkip where the pair is not rotated or there is none.
 constexpr int kStep = 16;        // steps that k_rotate loads at once
 constexpr int kFront = 64;       // room before a row in LDS
 constexpr double kSkip = 2.0;    // no cosine
-__global__ __launch_bounds__(256) void k_rot_params(int nocc, int nvirt, int steps, const double* __restrict__ fmo,
+__global__ __launch_bounds__(256) void k_rot_params(int nocc, int j0, int nj, int nvirt, int steps,
+                                                    const double* __restrict__ fmo,
                                                     const double* __restrict__ eig,
                                                     const double* __restrict__ tiny_dev, double bigeps,
                                                     double2* __restrict__ ab,
@@ -69,10 +70,10 @@ __global__ __launch_bounds__(256) void k_rot_params(int nocc, int nvirt, int ste
     const long long bt = q >> 6;
     const int v = (int)(bt / steps) * 64 + l, j = (int)(bt % steps) - l;
     double alpha = kSkip, beta = 0.0;
-    if (v < nvirt && j >= 0 && j < nocc) {
-      const double c = fmo[(long long)v * nocc + j];
+    if (v < nvirt && j >= 0 && j < nj) {
+      const double c = fmo[(long long)v * nocc + j0 + j];
       if (!(fabs(c) < tiny)) {
-        const double d = eig[j] - eig[nocc + v];
+        const double d = eig[j0 + j] - eig[nocc + v];
         if (!(fabs(c / d) < bigeps)) {
           const double e = (d >= 0.0 ? 1.0 : -1.0) * sqrt(4.0 * c * c + d * d);
           alpha = sqrt(0.5 * (1.0 + d / e));
@@ -100,7 +101,8 @@ __device__ __forceinline__ double from_lane_below(double x, double first) {
   return __hiloint2double(hi, lo);
 }
 
-// All rotations of a row of C, a row per wave.  64 virtuals at a time, one in
+// All rotations of a row of C with the nocc occupied from column Co on, a row
+// per wave.  64 virtuals at a time, one in
 // each lane's register; at step t lane l rotates its virtual with occupied
 // t - l, which comes from lane l - 1 as that left it, so the occupied
 // coefficients stream from the row in LDS through the lanes and back.  The
@@ -111,20 +113,22 @@ __device__ __forceinline__ double from_lane_below(double x, double first) {
 // would issue as much per row, on fewer of the chip's SIMDs.  The ordered
 // list, a lane per row and one rotation after another with an LDS read and
 // write each, took 434 us at 384 orbitals (256 occupied); this takes 37.
-__global__ __launch_bounds__(256) void k_rotate(int n, int ldc, double* __restrict__ C, int nocc, int nvirt,
-                                                int steps, const double2* __restrict__ ab) {
+constexpr int kRotRows = 4;  // a workgroup's
+__global__ __launch_bounds__(64 * kRotRows) void k_rotate(int n, int ldc, double* __restrict__ Co,
+                                                          double* __restrict__ Cv, int nocc, int nvirt, int steps,
+                                                          const double2* __restrict__ ab) {
   extern __shared__ double slab[];  // a row of kFront + steps per wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rows = blockDim.x >> 6, len = kFront + steps;  // 1, 2 or 4 rows
-  const int row0 = blockIdx.x * rows, row = row0 + wave;
-  for (int e = tid; e < rows * nocc; e += blockDim.x) {
-    const int r = e & (rows - 1), c = e / rows;
-    slab[r * len + kFront + c] = row0 + r < n ? C[(size_t)(row0 + r) + (size_t)c * ldc] : 0.0;
+  const int len = kFront + steps;
+  const int row0 = blockIdx.x * kRotRows, row = row0 + wave;
+  for (int e = tid; e < kRotRows * nocc; e += 64 * kRotRows) {
+    const int r = e % kRotRows, c = e / kRotRows;
+    slab[r * len + kFront + c] = row0 + r < n ? Co[(size_t)(row0 + r) + (size_t)c * ldc] : 0.0;
   }
   __syncthreads();
   double* S = slab + wave * len;
   for (int v0 = 0; v0 < nvirt; v0 += 64) {
-    double* col = C + (size_t)row + (size_t)(nocc + v0 + lane) * ldc;
+    double* col = Cv + (size_t)row + (size_t)(v0 + lane) * ldc;
     const bool have = v0 + lane < nvirt && row < n;
     double a = 0.0, b = have ? *col : 0.0;
     const double2* q = ab + (size_t)(v0 >> 6) * steps * 64 + lane;
@@ -166,9 +170,9 @@ __global__ __launch_bounds__(256) void k_rotate(int n, int ldc, double* __restri
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __syncthreads();
-  for (int e = tid; e < rows * nocc; e += blockDim.x) {
-    const int r = e & (rows - 1), c = e / rows;
-    if (row0 + r < n) C[(size_t)(row0 + r) + (size_t)c * ldc] = slab[r * len + kFront + c];
+  for (int e = tid; e < kRotRows * nocc; e += 64 * kRotRows) {
+    const int r = e % kRotRows, c = e / kRotRows;
+    if (row0 + r < n) Co[(size_t)(row0 + r) + (size_t)c * ldc] = slab[r * len + kFront + c];
   }
 }
 
@@ -209,6 +213,15 @@ __global__ __launch_bounds__(64) void k_apply_rotations(int n, int ldc, double* 
 // the first occupied enters lane 0 at step 0, the last leaves lane 63 at step
 // nocc + 62
 static int rot_steps(int nocc) { return (nocc + 63 + kStep - 1) / kStep * kStep; }
+// The occupied levels go through in equal parts whose rows fit the LDS, each
+// part past every virtual before the next: a virtual still meets them in
+// order, and so does an occupied the virtuals.
+constexpr int kMaxLds = 160 * 1024;
+constexpr int kMaxPart = kMaxLds / (int)sizeof(double) / kRotRows - kFront - 63 - kStep;
+static int rot_part(int nocc) {
+  const int parts = (nocc + kMaxPart - 1) / kMaxPart;
+  return (nocc + parts - 1) / parts;
+}
 
 void PseudoWork::ensure(int n, int nocc, int ld) {
   const long long nvirt = n - nocc;
@@ -216,7 +229,7 @@ void PseudoWork::ensure(int n, int nocc, int ld) {
   fd.ensure(sizeof(double) * (size_t)ld * ld);
   wv.ensure(sizeof(double) * (size_t)ld * std::max<long long>(nvirt, 1));
   fmo.ensure(sizeof(double) * std::max<long long>(len, 1));
-  ab.ensure(sizeof(double2) * ((nvirt + 63) / 64) * 64 * rot_steps(nocc));
+  ab.ensure(sizeof(double2) * ((nvirt + 63) / 64) * 64 * rot_steps(rot_part(nocc)));
   part.ensure(sizeof(double) * 1032);
 }
 
@@ -246,20 +259,20 @@ void pseudo_diag_device(hipStream_t s, PseudoWork& w, int n, int ld, const doubl
   hipLaunchKernelGGL(k_absmax_final, dim3(1), dim3(256), 0, s, nb, w.part.as<double>(),
                      w.part.as<double>() + 1023, count);
   MHIP_LAUNCH_CHECK();
-  const int steps = rot_steps(nocc);
-  const long long entries = (long long)((nvirt + 63) / 64) * 64 * steps;
-  hipLaunchKernelGGL(k_rot_params, dim3((int)std::min<long long>(512, (entries + 255) / 256)), dim3(256), 0, s, nocc,
-                     nvirt, steps, w.fmo.as<double>(), eig, w.part.as<double>() + 1023, 1.5e-7, w.ab.as<double2>(),
-                     count);
-  MHIP_LAUNCH_CHECK();
-  // up to four rows a workgroup, as they fit the LDS
-  const size_t max_lds = 160 * 1024, row = sizeof(double) * (kFront + steps);
-  int rows = 4;
-  while (rows > 1 && rows * row > max_lds) rows >>= 1;
-  MHIP_CHECK(hipFuncSetAttribute((const void*)k_rotate, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds));
-  hipLaunchKernelGGL(k_rotate, dim3((n + rows - 1) / rows), dim3(64 * rows), rows * row, s, n, ld, C, nocc, nvirt,
-                     steps, w.ab.as<double2>());
-  MHIP_LAUNCH_CHECK();
+  MHIP_CHECK(hipFuncSetAttribute((const void*)k_rotate, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+  const int part = rot_part(nocc);
+  for (int j0 = 0; j0 < nocc; j0 += part) {
+    const int nj = std::min(part, nocc - j0), steps = rot_steps(nj);
+    const long long entries = (long long)((nvirt + 63) / 64) * 64 * steps;
+    hipLaunchKernelGGL(k_rot_params, dim3((int)std::min<long long>(512, (entries + 255) / 256)), dim3(256), 0, s, nocc,
+                       j0, nj, nvirt, steps, w.fmo.as<double>(), eig, w.part.as<double>() + 1023, 1.5e-7,
+                       w.ab.as<double2>(), count);
+    MHIP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_rotate, dim3((n + kRotRows - 1) / kRotRows), dim3(64 * kRotRows),
+                       sizeof(double) * kRotRows * (kFront + steps), s, n, ld, C + (size_t)j0 * ld,
+                       C + (size_t)nocc * ld, nj, nvirt, steps, w.ab.as<double2>());
+    MHIP_LAUNCH_CHECK();
+  }
   if (nrot_out) {
     MHIP_CHECK(hipMemcpyAsync(nrot_out, count, sizeof(long long), hipMemcpyDeviceToHost, s));
     MHIP_CHECK(hipStreamSynchronize(s));

@@ -32,7 +32,9 @@ def test_rotations_match_oracle(gpu_ctx, waters, occupied):
         _check(gpu_ctx, s, nocc)
 
 
-def test_rows_that_fill_the_lds(gpu_ctx):
-    """Over 5 000 occupied levels a workgroup holds fewer rows."""
-    s = hamiltonian.build(*geometry.water_cluster(870, 5))
-    _check(gpu_ctx, s, 5190)
+@pytest.mark.parametrize("occupied", (4977, 4978, 5190))
+def test_rows_that_fill_the_lds(gpu_ctx, occupied):
+    """Over 4 977 occupied levels a row goes through the LDS in parts; one and
+    several blocks of 64 virtuals."""
+    s = hamiltonian.build(*geometry.water_cluster(870 if occupied == 5190 else 841, 5))
+    _check(gpu_ctx, s, occupied)
