@@ -507,17 +507,18 @@ static int setup_fragments(mhip_ctx* c, const mhip_scf_opts* o) {
 // The plain SCF of a molecule that one workgroup diagonalizes in its LDS runs
 // there from start to exit, in one launch: iteration by iteration from the
 // host, 26 orbitals took 24 launches and 4 waits an iteration, 3.1 ms in all
-// against 1.3 here.  The general path keeps what differs from it: PULAY, the
-// pseudo-diagonalizations, the eigensolver's other settings and its timing.
+// against 1.0 here.  The general path keeps what differs from it: PULAY, the
+// pseudo-diagonalizations, the split-BF16 form (whose density is a product of
+// its own), the eigensolver's other settings and its timing.
 struct OneMol {
   FockArgs args;
   BatchMol mol;
   BatchState st;
 };
 static bool one_workgroup_scf(const mhip_ctx* c, const mhip_scf_opts* o) {
-  return c->norbs <= kMaxLdsN && !o->pulay && !o->pseudo_diag && o->nclose > 0 && o->nclose < c->norbs &&
-         g_kernel_variant == 1 && g_jacobi_schedule == 1 && c->plan.max_inner == 0 && !c->plan.timing &&
-         !g_ktimer.on;
+  return c->norbs <= kMaxLdsN && !o->pulay && !o->pseudo_diag && o->precision != 1 && o->nclose > 0 &&
+         o->nclose < c->norbs && g_kernel_variant == 1 && g_jacobi_schedule == 1 && c->plan.max_inner == 0 &&
+         !c->plan.timing && !g_ktimer.on;
 }
 static const BatchState& run_one_workgroup(mhip_ctx* c, const mhip_scf_opts* o) {
   hipStream_t s = c->stream;

@@ -88,6 +88,15 @@ def test_single_molecule_in_one_workgroup_matches_the_general_path(systems, m):
     assert np.max(np.abs(f @ a["c"] - a["c"] * a["eig"])) < 1e-8  # F(i,i) + i*1e-10 is what is diagonalized
 
 
+def test_split_precision_of_a_small_molecule(gpu_ctx, systems):
+    """precision = 1 is the split-BF16 form at any size."""
+    gpu_ctx.upload(systems[2])
+    plain = gpu_ctx.iter(scfcrt=1e-6)
+    split = gpu_ctx.iter(scfcrt=1e-6, precision=1)
+    assert split["n_split_iter"] > 0 and plain["n_split_iter"] == 0
+    assert abs(split["escf"] - plain["escf"]) < 1e-6
+
+
 @pytest.mark.parametrize("scale", (1.0, 1e6, 1e20, 1e40))
 @pytest.mark.parametrize("mol", [("water", 5), ("water", 11), ("water", 22), ("water", 32), ("water", 33)])
 def test_levels_of_any_size(mol, scale):
