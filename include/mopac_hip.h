@@ -191,6 +191,9 @@ int mhip_batch_set_tiles(mhip_batch* b, const int* tiles);
  * one workgroup with cyclic Jacobi on matrices in global memory (for
  * comparison). */
 int mhip_batch_set_eig_lds(mhip_batch* b, int lds);
+/* Sweeps after which an eigensolve is given up (1 to 60, the default): its
+ * molecule then does not count as converged. */
+int mhip_batch_set_eig_sweeps(mhip_batch* b, int max_sweeps);
 /* Eigensolver profile: `iters` iterations of the batch from its starting
  * densities, launched one by one (no graph) with HIP events around the
  * eigensolver launch of each size class (n <= 32, 64, 128, 256).  ms[4]: the

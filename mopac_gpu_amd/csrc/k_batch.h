@@ -24,7 +24,8 @@ struct BatchState {
   int niter, iredy, ready, done, converged, newdg, oknewd, recompute, have_c, do_eig, mode, itrmax;
   int adaptive;   // loosen the eigensolver's tolerance while PL is large
   int sweeps, ndiag, last_sweeps;  // Jacobi sweeps and diagonalizations so far
-  int stuck;      // an eigensolve ran out of sweeps
+  int stuck;      // an eigensolve ran out of sweeps: the molecule does not count as converged
+  int max_sweeps;
   double ten, shift, shfmax, shfto, shftbo, shiftb, pl, eold, diff, sellim, escf, ee;
   double eig_homo, eig_lumo, enuclr, atheat, selcon, pltest;
   // eigensolver work of this molecule since the batch was reset: applied
@@ -39,7 +40,7 @@ struct BatchState {
 constexpr int kMaxBatchN = 256;
 constexpr int kMaxLdsN = 64;
 
-constexpr int kEigSweeps = 60;  // the sweep limit of an eigensolve
+constexpr int kEigSweeps = 60;  // the sweep limit of an eigensolve, at most
 
 // The starting control state of one molecule (iter.F90:91-251).
 BatchState batch_start(double enuclr, double atheat, double scfcrt, int itrmax);
@@ -59,6 +60,7 @@ void bj_destroy(BatchJacobi* j);
 // Diagonalizes the molecules with do_eig set whose padded size is in [lo, hi]:
 // levels, eigenvectors (the next call's warm start) and the packed density.
 // Waits for the device once a sweep; returns how many of them are not done.
-int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, double tol, int lo, int hi);
+int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, double tol, int max_sweeps, int lo,
+             int hi);
 
 }  // namespace mhip

@@ -168,7 +168,7 @@ __device__ __forceinline__ void eig_done(const BatchMol& M, BatchState& s, EigCo
   s.eig_flops += beig_flops(M.n, M.nocc, c.nrot, warm);
   s.sweeps += c.sweeps;
   s.last_sweeps = c.sweeps;
-  s.stuck |= c.sweeps >= kEigSweeps;
+  s.stuck |= c.sweeps >= s.max_sweeps;
   s.ndiag += 1;
   s.have_c = 1;
 }
@@ -177,7 +177,7 @@ __device__ __forceinline__ void eig_done(const BatchMol& M, BatchState& s, EigCo
 // M.eig, and, with nocc > 0, the packed density into M.p.  Matrices in global
 // memory.
 template <int NT>
-__device__ EigCount beig_global(const BatchMol& M, double* f, bool warm, double tol, bool density) {
+__device__ EigCount beig_global(const BatchMol& M, double* f, bool warm, double tol, int max_sweeps, bool density) {
   const int n = M.n, tid = threadIdx.x;
   __shared__ double red[NT];
   __shared__ double cs[kMaxBatchN / 2], sn[kMaxBatchN / 2];
@@ -221,7 +221,7 @@ __device__ EigCount beig_global(const BatchMol& M, double* f, bool warm, double 
   __syncthreads();
   const int np = (n + 1) & ~1;
   const int npair = np / 2;
-  for (int sweep = 0; sweep < kEigSweeps; ++sweep) {
+  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     double off = 0.0, dg = 0.0;
     for (int e = tid; e < n * n; e += NT) {
       const int r = e % n, c = e / n;
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(NT) void k_beig(const BatchMol* __restrict__ mols, 
   const int m = list[blockIdx.x];
   if (!do_eig[m]) return;
   const bool warm = st[m].have_c != 0;
-  eig_done(mols[m], st[m], beig_global<NT>(mols[m], mols[m].f, warm, tol, true), warm);
+  eig_done(mols[m], st[m], beig_global<NT>(mols[m], mols[m].f, warm, tol, st[m].max_sweeps, true), warm);
 }
 
 __device__ __forceinline__ int tri(int i) { return (i * (i + 1)) >> 1; }
@@ -347,7 +347,8 @@ __device__ __forceinline__ int tri_row(int e) {
 static_assert(kMaxLdsN == SB, "one pair problem");
 constexpr int kLdsThreads = CROSS_THREADS;
 
-__device__ __noinline__ EigCount beig_lds(JacLds& lds, const BatchMol& M, double* f, bool warm, double tol, bool density) {
+__device__ __noinline__ EigCount beig_lds(JacLds& lds, const BatchMol& M, double* f, bool warm, double tol,
+                                          int max_sweeps, bool density) {
   const int n = M.n, tid = threadIdx.x;
   __shared__ int rank[SB];
   double(*S)[SB] = lds.s();
@@ -389,7 +390,8 @@ __device__ __noinline__ EigCount beig_lds(JacLds& lds, const BatchMol& M, double
     }
   }
   __syncthreads();
-  const int sweeps = pair_solve<true>(lds, 0, 1, true, JacSolve{n, nullptr, nullptr, nullptr, nullptr, tol, 0.0, kEigSweeps});
+  const int sweeps =
+      pair_solve<true>(lds, 0, 1, true, JacSolve{n, nullptr, nullptr, nullptr, nullptr, tol, 0.0, max_sweeps});
   // ascending order, ties by index; the padding stays where it is
   if (tid < SB) {
     const double d = S[tid][tid];
@@ -455,7 +457,7 @@ __global__ __launch_bounds__(kLdsThreads, 4) void k_beig_lds(const BatchMol* __r
   const int m = list[blockIdx.x];
   if (!do_eig[m]) return;
   const bool warm = st[m].have_c != 0;
-  eig_done(mols[m], st[m], beig_lds(lds, mols[m], mols[m].f, warm, tol, true), warm);
+  eig_done(mols[m], st[m], beig_lds(lds, mols[m], mols[m].f, warm, tol, st[m].max_sweeps, true), warm);
 }
 
 // ---- control, part 3: PL, frontier levels, newdg (iter.F90:1030-1041) -------
@@ -719,8 +721,8 @@ __device__ __forceinline__ void scf_body(JacLds* lds, const FockArgs* __restrict
   FockArgs a = args[m];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = M.n;
   auto eig = [&](double* f, bool warm, double t, bool density) {
-    if constexpr (LDS) return beig_lds(*lds, M, f, warm, t, density);
-    else return beig_global<NT>(M, f, warm, t, density);
+    if constexpr (LDS) return beig_lds(*lds, M, f, warm, t, s.max_sweeps, density);
+    else return beig_global<NT>(M, f, warm, t, s.max_sweeps, density);
   };
   if (tid == 0) s = st[m];
   __shared__ int atom_of[kMaxLdsN];
@@ -893,6 +895,7 @@ struct mhip_batch {
   DevBuf cls_list;
   int tile[4] = {64, 128, 256, 256};   // workgroup size per class (n <= 32, 64, 128, 256)
   double tol = 1.0e-10;
+  int max_sweeps = kEigSweeps;
   std::vector<BatchState> init_state;
   // eager timing of the eigensolver launches per size class
   hipEvent_t eig_ev[4][2] = {};
@@ -977,8 +980,8 @@ int one_iteration(mhip_batch* b, bool big_only) {
     if (c < 2 || b->force_global_eig) launch_eig_class(b, c, off, b->cls_count[c]);
     else if (b->bj && (!big_only || c == 2))
       // by itself only for its own time
-      open += bj_solve(b->bj, s, b->st.as<BatchState>(), b->doeig.as<int>(), b->tol, big_only || c == 2 ? 128 : 192,
-                       !big_only && c == 2 ? 128 : 256);
+      open += bj_solve(b->bj, s, b->st.as<BatchState>(), b->doeig.as<int>(), b->tol, b->max_sweeps,
+                       big_only || c == 2 ? 128 : 192, !big_only && c == 2 ? 128 : 256);
     if (b->eig_timing) MHIP_CHECK(hipEventRecord(b->eig_ev[c][1], s));
     off += b->cls_count[c];
   }
@@ -1012,6 +1015,7 @@ namespace mhip {
 BatchState batch_start(double enuclr, double atheat, double scfcrt, int itrmax) {
   BatchState z{};
   z.itrmax = itrmax > 0 ? itrmax : 2000;
+  z.max_sweeps = kEigSweeps;
   z.ten = -80.0;
   z.shift = 1.0;
   z.shfmax = 20.0;
@@ -1267,6 +1271,18 @@ int mhip_batch_set_eig_lds(mhip_batch* b, int lds) {
   });
 }
 
+int mhip_batch_set_eig_sweeps(mhip_batch* b, int max_sweeps) {
+  return bguard([&] {
+    MHIP_REQUIRE(b && max_sweeps > 0 && max_sweeps <= kEigSweeps, "mhip_batch_set_eig_sweeps: 1 to 60 sweeps");
+    b->max_sweeps = max_sweeps;
+    for (auto& z : b->init_state) z.max_sweeps = max_sweeps;
+    MHIP_CHECK(hipMemcpy(b->st0.ptr, b->init_state.data(), sizeof(BatchState) * b->nmol, hipMemcpyHostToDevice));
+  });
+}
+
+// self-consistent, by levels that every eigensolve on the way converged to
+static bool converged(const BatchState& z) { return z.converged && !z.stuck; }
+
 // the per-molecule state and the starting densities, before a run
 static void reset_batch(mhip_batch* b) {
   MHIP_CHECK(hipMemcpyAsync(b->st.ptr, b->st0.ptr, sizeof(BatchState) * b->nmol, hipMemcpyDeviceToDevice, b->s));
@@ -1350,20 +1366,20 @@ int mhip_batch_run(mhip_batch* b, int iters_per_graph, int max_launches, double*
     if (seconds) *seconds = std::chrono::duration<double>(t1 - t0).count();
     if (n_converged) {
       int c = 0;
-      for (const auto& z : hs) c += z.converged ? 1 : 0;
+      for (const auto& z : hs) c += converged(z) ? 1 : 0;
       *n_converged = c;
     }
   });
 }
 
-int mhip_batch_results(mhip_batch* b, double* escf, int* niter, int* converged) {
+int mhip_batch_results(mhip_batch* b, double* escf, int* niter, int* conv) {
   return bguard([&] {
     std::vector<BatchState> hs(b->nmol);
     MHIP_CHECK(hipMemcpy(hs.data(), b->st.ptr, sizeof(BatchState) * b->nmol, hipMemcpyDeviceToHost));
     for (int m = 0; m < b->nmol; ++m) {
       if (escf) escf[m] = hs[m].escf;
       if (niter) niter[m] = hs[m].niter;
-      if (converged) converged[m] = hs[m].converged;
+      if (conv) conv[m] = converged(hs[m]) ? 1 : 0;
     }
   });
 }

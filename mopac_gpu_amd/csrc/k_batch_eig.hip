@@ -26,7 +26,7 @@ namespace mhip {
 namespace {
 
 constexpr int kGroups = 3;    // padded sizes 128, 192, 256
-constexpr int kMaxSweeps = 60;
+constexpr int kMaxSweeps = kEigSweeps;
 
 struct BjMol {
   int mol;         // index in the batch
@@ -46,6 +46,7 @@ struct BjState {
   int did;         // this call diagonalizes the molecule
   int cur;         // which A holds the result
   int sweeps;
+  int stuck;       // out of sweeps
   int scale;       // A is the matrix times 2^-scale
   double skip;     // pairs this diagonal are left alone
   unsigned long long rot;
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(256) void k_bj_begin(const BjMol* __restrict__ mols
   if (go)
     for (int k = threadIdx.x; k < M.n; k += 256) M.f[(size_t)k * (k + 1) / 2 + k] += (double)(k + 1) * 1.0e-10;
   if (threadIdx.x == 0) {
-    st[i] = BjState{go ? 1 : 0, go ? 1 : 0, 0, 0, 0, 0.0, 0ull};
+    st[i] = BjState{go ? 1 : 0, go ? 1 : 0, 0, 0, 0, 0, 0.0, 0ull};
     if (!bst[M.mol].done) atomicAdd(counts, 1);
   }
 }
@@ -250,6 +251,7 @@ __global__ __launch_bounds__(1024) void k_bj_test(BjLaunch a, int sweep, int las
   s.cur = a.par[g];
   if (off <= thr || last) {
     s.run = 0;
+    s.stuck = !(off <= thr);
   } else {
     s.skip = 0.1 * thr;
     s.sweeps += 1;
@@ -337,6 +339,8 @@ __global__ __launch_bounds__(512) void k_bj_order(BjLaunch a, BatchState* __rest
     t.eig_rot += (long long)s.rot;
     t.eig_flops += 12.0 * dn * (double)s.rot + (t.have_c ? 2.0 * dn * dn * dn + 2.0 * dn * tn : 0.0) + 2.0 * tn * M.nocc;
     t.sweeps += s.sweeps;
+    t.last_sweeps = s.sweeps;
+    t.stuck |= s.stuck;
     t.ndiag += 1;
     t.have_c = 1;
   }
@@ -463,7 +467,8 @@ void bj_destroy(BatchJacobi* j) {
   delete j;
 }
 
-int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, double tol, int lo, int hi) {
+int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, double tol, int max_sweeps, int lo,
+             int hi) {
   BjLaunch a{};
   a.mol = j->mols.as<BjMol>();
   a.st = j->st.as<BjState>();
@@ -499,8 +504,8 @@ int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, 
   hipLaunchKernelGGL(k_bj_ctf, dim3(total(tiles)), dim3(UPD_NT), 0, s, a, bst);
   MHIP_LAUNCH_CHECK();
   int open = 0;
-  for (int sw = 0; sw <= kMaxSweeps; ++sw) {
-    hipLaunchKernelGGL(k_bj_test, dim3(nmol), dim3(1024), 0, s, a, sw, sw == kMaxSweeps ? 1 : 0,
+  for (int sw = 0; sw <= max_sweeps; ++sw) {
+    hipLaunchKernelGGL(k_bj_test, dim3(nmol), dim3(1024), 0, s, a, sw, sw == max_sweeps ? 1 : 0,
                        counts + 1 + sw);
     MHIP_LAUNCH_CHECK();
     MHIP_CHECK(hipMemcpyAsync(j->host, counts, sizeof(int) * (kMaxSweeps + 2), hipMemcpyDeviceToHost, s));
@@ -515,7 +520,7 @@ int bj_solve(BatchJacobi* j, hipStream_t s, BatchState* bst, const int* do_eig, 
       MHIP_LAUNCH_CHECK();
     };
     a.step = 0;
-    if (sw < kMaxSweeps) {
+    if (sw < max_sweeps) {
       if (sw == 0) {
         hipLaunchKernelGGL(k_bj_first, dim3(total([](const BjGroup& g) { return g.npairs; })), dim3(CROSS_THREADS), 0,
                            s, a);

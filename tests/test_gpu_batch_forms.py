@@ -88,6 +88,21 @@ def test_single_molecule_in_one_workgroup_matches_the_general_path(systems, m):
     assert np.max(np.abs(f @ a["c"] - a["c"] * a["eig"])) < 1e-8  # F(i,i) + i*1e-10 is what is diagonalized
 
 
+def test_eigensolves_out_of_sweeps_do_not_count(systems, edge_batch):
+    """Two sweeps do not converge the first diagonalization; the SCF may still
+    settle, on levels that are not F's."""
+    b = edge_batch
+    for lds in (True, False):
+        b.set_eig_lds(lds)
+        b.lib.mhip_batch_set_eig_sweeps(b.h, 2)
+        _, n = b.run()
+        assert n == 0 and not b.results()[2].any()
+        b.lib.mhip_batch_set_eig_sweeps(b.h, 60)
+        _, n = b.run()
+        assert n == len(systems) and b.results()[2].all()
+    b.set_eig_lds(True)
+
+
 def test_split_precision_of_a_small_molecule(gpu_ctx, systems):
     """precision = 1 is the split-BF16 form at any size."""
     gpu_ctx.upload(systems[2])
