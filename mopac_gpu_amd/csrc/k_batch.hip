@@ -879,7 +879,9 @@ struct mhip_batch {
   hipStream_t s = nullptr;
   std::vector<int> n_h, nocc_h, numat_h;
   // device storage
-  DevBuf w, h, f, p, pa, pold, p1, C, A, T, eig, jrow, jcol;
+  DevBuf w, h, f, p, pa, pold, p1, C, eig, jrow, jcol;
+  std::vector<BatchMol> mol_h;  // as mols has them
+  DevBuf global;                // the matrices of the global-memory form, once it is asked for
   DevBuf nf0, norb, woff, wcum, w1off, ccol, heavy, light, nhb, nlb;
   DevBuf args, mols, cnv, st, act, doeig, mode, niter, shift, ee, partial, scal, orboff;
   DevBuf pdiag, st0;  // starting diagonals and control states, where every run begins
@@ -950,6 +952,27 @@ void launch_scf_class(mhip_batch* b, hipStream_t s, int cls, int offset, int cap
       hipLaunchKernelGGL(k_bscf<NT>, dim3(n), dim3(NT), 0, s, args, mols, st, list, b->tol, cap, 0);
     });
   MHIP_LAUNCH_CHECK();
+}
+
+// A and T of every molecule, and C of those that have none in the default form,
+// for the form with its matrices in memory.  They are left out until it is
+// chosen: 3 n^2 beside the 4 npad^2 that the block-Jacobi form works in.
+void ensure_global_form(mhip_batch* b) {
+  if (b->global.ptr) return;
+  size_t len = 0;
+  for (const BatchMol& q : b->mol_h) len += (size_t)q.n * q.n * (q.C ? 2 : 3);
+  b->global.ensure(sizeof(double) * len);
+  double* at = b->global.as<double>();
+  for (BatchMol& q : b->mol_h) {
+    const size_t sz = (size_t)q.n * q.n;
+    q.A = at;
+    q.T = at + sz;
+    at += 2 * sz;
+    if (q.C) continue;
+    q.C = at;
+    at += sz;
+  }
+  MHIP_CHECK(hipMemcpy(b->mols.ptr, b->mol_h.data(), sizeof(BatchMol) * b->nmol, hipMemcpyHostToDevice));
 }
 
 // One iteration of every molecule (the eigensolver profile), or of those of
@@ -1051,8 +1074,8 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     for (auto& c : b->cs) MHIP_CHECK(hipStreamCreateWithFlags(&c, hipStreamNonBlocking));
     for (auto& e : b->ev) MHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // ---- host tables, then one upload per array
-    std::vector<long long> o_w(nmol), o_mp(nmol), o_nn(nmol), o_n(nmol), o_at(nmol), o_cc(nmol), o_a(nmol);
-    long long tw = 0, tmp = 0, tnn = 0, tn = 0, tat = 0, tcc = 0, ta = 0;
+    std::vector<long long> o_w(nmol), o_mp(nmol), o_nn(nmol), o_n(nmol), o_at(nmol), o_cc(nmol);
+    long long tw = 0, tmp = 0, tnn = 0, tn = 0, tat = 0, tcc = 0;
     std::vector<int> nf0_all, norb_all, heavy_all, light_all, nhb_all, nlb_all;
     std::vector<long long> woff_all, wcum_all, w1off_all, ccol_all;
     for (int m = 0; m < nmol; ++m) {
@@ -1096,9 +1119,7 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
       MHIP_REQUIRE(nf0_all.back() + norb_all.back() == n, "mhip_batch_create: nlast(numat) != norbs");
       tw += kr;
       tmp += (long long)n * (n + 1) / 2;
-      tnn += std::max<long long>((long long)n * n, SB * SB);  // the LDS form's C is padded
-      o_a[m] = ta;
-      ta += (long long)n * n;
+      if (n <= kMaxLdsN) tnn += SB * SB;  // C, padded
       tn += n;
       tat += na;
       tcc += std::max(cc, 1LL);
@@ -1121,8 +1142,7 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     for (DevBuf* x : {&b->f, &b->p, &b->pa, &b->pold}) x->ensure(sizeof(double) * tmp);
     b->p1.ensure(sizeof(double) * tn);
     b->eig.ensure(sizeof(double) * tn);
-    for (DevBuf* x : {&b->C, &b->T}) x->ensure(sizeof(double) * tnn);
-    b->A.ensure(sizeof(double) * ta);
+    b->C.ensure(sizeof(double) * std::max(tnn, 1LL));
     b->jrow.ensure(sizeof(double) * 10 * tat);
     b->jcol.ensure(sizeof(double) * tcc);
     for (int m = 0; m < nmol; ++m) {
@@ -1164,7 +1184,8 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
                        [&](int x, int y) { return b->n_h[x] > b->n_h[y]; });
     // per-molecule argument blocks
     std::vector<FockArgs> args(nmol);
-    std::vector<BatchMol> bm(nmol);
+    std::vector<BatchMol>& bm = b->mol_h;
+    bm.resize(nmol);
     std::vector<BatchCnvg> cv(nmol);
     std::vector<long long> orboff(nmol);
     std::vector<int> atom_mol, atom_idx, row_mol, row_idx;
@@ -1204,9 +1225,7 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
       q.pa = b->pa.as<double>() + o_mp[m];
       q.pold = b->pold.as<double>() + o_mp[m];
       q.p1 = b->p1.as<double>() + o_n[m];
-      q.C = b->C.as<double>() + o_nn[m];
-      q.A = b->A.as<double>() + o_a[m];
-      q.T = b->T.as<double>() + o_nn[m];
+      q.C = n <= kMaxLdsN ? b->C.as<double>() + o_nn[m] : nullptr;
       q.eig = b->eig.as<double>() + o_n[m];
       cv[m] = BatchCnvg{n, q.p, q.pold, q.p1};
       orboff[m] = o_n[m];
@@ -1267,6 +1286,7 @@ int mhip_batch_set_tiles(mhip_batch* b, const int* tiles) {
 int mhip_batch_set_eig_lds(mhip_batch* b, int lds) {
   return bguard([&] {
     MHIP_REQUIRE(b, "mhip_batch_set_eig_lds: bad arguments");
+    if (lds == 0) ensure_global_form(b);
     b->force_global_eig = lds == 0;
   });
 }
@@ -1400,7 +1420,7 @@ void mhip_batch_destroy(mhip_batch* b) {
   bj_destroy(b->bj);
   for (auto c : b->cs) (void)hipStreamDestroy(c);
   for (auto e : b->ev) (void)hipEventDestroy(e);
-  for (DevBuf* x : {&b->w, &b->h, &b->f, &b->p, &b->pa, &b->pold, &b->p1, &b->C, &b->A, &b->T, &b->eig, &b->jrow,
+  for (DevBuf* x : {&b->w, &b->h, &b->f, &b->p, &b->pa, &b->pold, &b->p1, &b->C, &b->global, &b->eig, &b->jrow,
                     &b->jcol, &b->nf0, &b->norb, &b->woff, &b->wcum, &b->w1off, &b->ccol, &b->heavy, &b->light,
                     &b->nhb, &b->nlb, &b->args, &b->mols, &b->cnv, &b->st, &b->act, &b->doeig, &b->mode, &b->niter,
                     &b->shift, &b->ee, &b->partial, &b->scal, &b->orboff, &b->atom_mol, &b->atom_idx,

@@ -34,7 +34,7 @@ struct BjMol {
   double* A[2];    // the matrix before and after a step, in turn
   double* C;       // working eigenvectors
   double* Cs;      // ordered eigenvectors of the last solve (the warm start)
-  double* T;       // F C
+  double* T;       // F C: A[1], before the first step writes it
   double* q;       // rotations, flags and diagonal blocks of two steps
   int* act;
   double* diag;
@@ -421,7 +421,7 @@ BatchJacobi* bj_create(const std::vector<BatchMol>& mol, const std::vector<int>&
     G.pairs = p.pairs.as<int>();
     G.intra = p.intra.as<int>();
     G.where = p.where.as<int>();
-    dense += (size_t)G.count * 5 * G.npad * G.npad;
+    dense += (size_t)G.count * 4 * G.npad * G.npad;
     q += (size_t)G.count * 2 * G.npairs * SB * SB;
     act += (size_t)G.count * 2 * G.npairs;
     diag += (size_t)G.count * 2 * G.nb * BS * BS;
@@ -438,10 +438,11 @@ BatchJacobi* bj_create(const std::vector<BatchMol>& mol, const std::vector<int>&
     for (int i = j->g[g].first; i < j->g[g].first + j->g[g].count; ++i) {
       BjMol& x = t[i];
       const size_t sz = (size_t)x.npad * x.npad;
-      for (double** b : {&x.A[0], &x.A[1], &x.C, &x.Cs, &x.T}) {
+      for (double** b : {&x.A[0], &x.A[1], &x.C, &x.Cs}) {
         *b = d;
         d += sz;
       }
+      x.T = x.A[1];
       x.q = pq;
       pq += (size_t)2 * j->g[g].npairs * SB * SB;
       x.act = pa;

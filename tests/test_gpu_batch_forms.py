@@ -1,6 +1,7 @@
 """The batched SCF's two forms at the edges of their ranges: one workgroup for
 a molecule up to 64 orbitals, block-Jacobi steps over several above (padded
 sizes 128, 192 and 256), and the single-molecule SCF that shares the first."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -8,6 +9,7 @@ import pytest
 
 from mopac_gpu_amd import batch as B
 from mopac_gpu_amd import geometry, hamiltonian
+from mopac_gpu_amd import lib as L
 from mopac_gpu_amd.scf import Context
 from oracle import oracle
 
@@ -101,6 +103,34 @@ def test_eigensolves_out_of_sweeps_do_not_count(systems, edge_batch):
         _, n = b.run()
         assert n == len(systems) and b.results()[2].all()
     b.set_eig_lds(True)
+
+
+def test_device_memory_of_the_default_form(systems):
+    """Four padded matrices, the rotations and diagonal blocks of two steps and
+    the caller's arrays for a molecule above 64 orbitals; the matrices of the
+    global-memory form are there once it is chosen."""
+    s = systems[13]
+    n, npad, count = s.norbs, 256, 256
+    assert 192 < n <= npad
+    B.Batch([s], scfcrt=1e-6).close()  # the module's code is loaded
+
+    def free():  # the HIP library that this one is linked with
+        now, all_of_it = ctypes.c_size_t(), ctypes.c_size_t()
+        assert L.load().hipMemGetInfo(ctypes.byref(now), ctypes.byref(all_of_it)) == 0
+        return now.value
+
+    before = free()
+    b = B.Batch([s] * count, scfcrt=1e-6)
+    each = (before - free()) / 8 / count
+    caller = len(s.w) + 5 * s.mpack
+    # the Fock build's column partials: an atom's 1 or 10 elements by every later atom
+    limit = np.where(np.asarray(s.nlast) > np.asarray(s.nfirst), 10, 1)
+    columns = int(np.sum(limit * (s.numat - 1 - np.arange(s.numat))))
+    # rows, levels and atoms' tables are under 100 numbers an orbital
+    assert each < caller + columns + 4 * npad * npad + 192 * npad + 100 * n
+    b.set_eig_lds(False)
+    assert (before - free()) / 8 / count > each + 2.9 * n * n
+    b.close()
 
 
 def test_split_precision_of_a_small_molecule(gpu_ctx, systems):
