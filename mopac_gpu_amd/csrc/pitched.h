@@ -8,10 +8,11 @@ namespace mhip {
 
 // The runtime's 2D copy takes a pageable array row by row, with gaps between
 // the rows or without: the eigenvectors of 282 orbitals (636 KB) took 2.5 ms
-// each way.  Rows without gaps on either side are a plain copy; others pass
-// through two pinned slots, packed or unpacked by the host beside the other
-// slot's DMA, which takes rows with gaps from pinned memory at its full rate:
-// 60 us.  Memory that the runtime knows (pinned, managed, device) is left to it.
+// each way.  Rows without gaps on either side, or a single row, are a plain
+// copy; others pass through two pinned slots, packed or unpacked by the host
+// beside the other slot's DMA, which takes rows with gaps from pinned memory at
+// its full rate: 60 us.  Memory that the runtime knows (pinned, managed,
+// device) is left to it.
 //
 // One owner, one thread at a time; pins at most kSlots * kMaxSlot bytes.
 class PitchedCopy {

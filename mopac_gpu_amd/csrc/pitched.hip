@@ -56,7 +56,7 @@ void PitchedCopy::up(void* dst, size_t dpitch, const void* src, size_t spitch, s
                      hipStream_t s) {
   if (width == 0 || rows == 0) return;
   MHIP_REQUIRE(dst && src && dpitch >= width && spitch >= width, "copy to the device: invalid argument");
-  if (dpitch == width && spitch == width) {
+  if (rows == 1 || (dpitch == width && spitch == width)) {
     MHIP_CHECK(hipMemcpyAsync(dst, src, width * rows, hipMemcpyHostToDevice, s));
     return;
   }
@@ -85,7 +85,7 @@ void PitchedCopy::down(void* dst, size_t dpitch, const void* src, size_t spitch,
                        hipStream_t s) {
   if (width == 0 || rows == 0) return;
   MHIP_REQUIRE(dst && src && dpitch >= width && spitch >= width, "copy from the device: invalid argument");
-  if (dpitch == width && spitch == width) {
+  if (rows == 1 || (dpitch == width && spitch == width)) {
     MHIP_CHECK(hipMemcpyAsync(dst, src, width * rows, hipMemcpyDeviceToHost, s));
     MHIP_CHECK(hipStreamSynchronize(s));
     return;

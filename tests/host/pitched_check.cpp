@@ -97,7 +97,13 @@ hipError_t hipMemcpy2DAsync(void* dst, size_t dpitch, const void* src, size_t sp
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind k, hipStream_t s) {
-  return hipMemcpy2DAsync(dst, bytes, src, bytes, bytes, 1, k, s);
+  if (k != hipMemcpyHostToDevice || in_guarded(src)) return hipMemcpy2DAsync(dst, bytes, src, bytes, bytes, 1, k, s);
+  // pageable memory has been read on return
+  const auto* from = static_cast<const char*>(src);
+  queued.push_back([dst, staged = std::vector<char>(from, from + bytes)] {
+    std::memcpy(dst, staged.data(), staged.size());
+  });
+  return hipSuccess;
 }
 
 namespace {
