@@ -30,7 +30,7 @@ class PitchedCopy {
 
  private:
   static constexpr int kSlots = 2;
-  static constexpr size_t kMinSlot = size_t(64) << 10, kMaxSlot = size_t(4) << 20;
+  static constexpr size_t kMinSlot = size_t(256) << 10, kMaxSlot = size_t(4) << 20;
   bool direct(const void* host, size_t width) const;
   void ensure(size_t width, size_t rows, hipStream_t s);
   void wait(int i);

@@ -135,7 +135,7 @@ bool round_trip(size_t m, size_t rows, size_t pad) {
 
 int main() {
   int bad = 0, all = 0;
-  for (size_t m : {1, 77, 300, 8191, 8192, 8193, 9000, 10000, 12000, 16384, 16385, 20000, 24000, 40000, 131072, 262145,
+  for (size_t m : {1, 77, 300, 8191, 8192, 8193, 9000, 10000, 12000, 16384, 16385, 20000, 24000, 32768, 32769, 40000, 131072, 262145,
                    524287, 524288})
     for (size_t rows : {1, 2, 3, 5, 40}) {
       if (m * rows > 6000000) continue;

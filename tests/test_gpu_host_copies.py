@@ -10,8 +10,7 @@ pytestmark = pytest.mark.gpu
 
 # one value; columns without gaps; ragged ones in one and in several pieces;
 # 13 and 27 MB (slots at their largest); one and two columns of 64 KB to 4 MB,
-# each as long as a slot or longer than a third of the matrix; columns longer
-# than the largest slot
+# a slot's smallest and largest size between them; columns longer than that
 @pytest.mark.parametrize("m,n,pad", [(1, 1, 0), (1, 40, 3), (7, 301, 2), (300, 77, 0), (123, 701, 5),
                                      (1237, 1301, 5), (1901, 1777, 1), (8193, 2, 3),
                                      (9000, 2, 3), (12000, 2, 3), (20000, 1, 3), (24000, 1, 3), (40000, 2, 1),

@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 
 
 def test_every_row_has_its_slot(tmp_path):
-    """Rows on both sides of a slot's sizes (64 KB to 4 MB), one of them and
+    """Rows on both sides of a slot's sizes (256 KB to 4 MB), one of them and
     several: each arrives, and nothing outside the pinned memory is touched."""
     exe = str(tmp_path / "pitched_check")
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", HERE, "-I", os.path.join(ROOT, "include"), "-I",
