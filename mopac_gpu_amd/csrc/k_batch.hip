@@ -885,7 +885,10 @@ struct mhip_batch {
   DevBuf nf0, norb, woff, wcum, w1off, ccol, heavy, light, nhb, nlb;
   DevBuf args, mols, cnv, st, act, doeig, mode, niter, shift, ee, partial, scal, orboff;
   DevBuf pdiag, st0;  // starting diagonals and control states, where every run begins
-  hipStream_t cs[4] = {};  // a stream per size class: the classes fill each other's tails
+  int device = 0;  // that everything here belongs to
+  // a stream and an event per size class that runs a workgroup to a molecule:
+  // the classes fill each other's tails
+  hipStream_t cs[4] = {};
   hipEvent_t ev[5] = {};
   DevBuf atom_mol, atom_idx, row_mol, row_idx;
   int n_atom_blk = 0, n_row_blk = 0;
@@ -954,11 +957,29 @@ void launch_scf_class(mhip_batch* b, hipStream_t s, int cls, int offset, int cap
   MHIP_LAUNCH_CHECK();
 }
 
+// For the first n classes, where they have a molecule.
+void ensure_class_streams(mhip_batch* b, int n) {
+  for (int c = 0; c < n; ++c) {
+    if (b->cls_count[c] == 0) continue;
+    if (!b->cs[c]) MHIP_CHECK(hipStreamCreateWithFlags(&b->cs[c], hipStreamNonBlocking));
+    if (!b->ev[c]) MHIP_CHECK(hipEventCreateWithFlags(&b->ev[c], hipEventDisableTiming));
+  }
+}
+
 // A and T of every molecule, and C of those that have none in the default form,
 // for the form with its matrices in memory.  They are left out until it is
 // chosen: 3 n^2 beside the 4 npad^2 that the block-Jacobi form works in.
 void ensure_global_form(mhip_batch* b) {
   if (b->global.ptr) return;
+  struct OnDevice {
+    int before = 0;
+    explicit OnDevice(int device) {
+      MHIP_CHECK(hipGetDevice(&before));
+      MHIP_CHECK(hipSetDevice(device));
+    }
+    ~OnDevice() { (void)hipSetDevice(before); }
+  } on(b->device);
+  ensure_class_streams(b, 4);
   size_t len = 0;
   for (const BatchMol& q : b->mol_h) len += (size_t)q.n * q.n * (q.C ? 2 : 3);
   b->global.ensure(sizeof(double) * len);
@@ -1071,8 +1092,8 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
     auto* b = new mhip_batch();
     b->nmol = nmol;
     MHIP_CHECK(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking));
-    for (auto& c : b->cs) MHIP_CHECK(hipStreamCreateWithFlags(&c, hipStreamNonBlocking));
-    for (auto& e : b->ev) MHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    MHIP_CHECK(hipGetDevice(&b->device));
+    MHIP_CHECK(hipEventCreateWithFlags(&b->ev[4], hipEventDisableTiming));
     // ---- host tables, then one upload per array
     std::vector<long long> o_w(nmol), o_mp(nmol), o_nn(nmol), o_n(nmol), o_at(nmol), o_cc(nmol);
     long long tw = 0, tmp = 0, tnn = 0, tn = 0, tat = 0, tcc = 0;
@@ -1178,6 +1199,7 @@ int mhip_batch_create(int nmol, const mhip_batch_molecule* mols, mhip_batch** ou
           b->cls_count[c]++;
           b->cls_nmax[c] = std::max(b->cls_nmax[c], b->n_h[m]);
         }
+    ensure_class_streams(b, 2);
     // the largest of each class first: they take the longest
     for (int c = 0, o = 0; c < 4; o += b->cls_count[c++])
       std::stable_sort(order.begin() + o, order.begin() + o + b->cls_count[c],
@@ -1418,8 +1440,10 @@ void mhip_batch_destroy(mhip_batch* b) {
   if (!b) return;
   (void)hipStreamSynchronize(b->s);
   bj_destroy(b->bj);
-  for (auto c : b->cs) (void)hipStreamDestroy(c);
-  for (auto e : b->ev) (void)hipEventDestroy(e);
+  for (auto c : b->cs)
+    if (c) (void)hipStreamSynchronize(c), (void)hipStreamDestroy(c);
+  for (auto e : b->ev)
+    if (e) (void)hipEventDestroy(e);
   for (DevBuf* x : {&b->w, &b->h, &b->f, &b->p, &b->pa, &b->pold, &b->p1, &b->C, &b->global, &b->eig, &b->jrow,
                     &b->jcol, &b->nf0, &b->norb, &b->woff, &b->wcum, &b->w1off, &b->ccol, &b->heavy, &b->light,
                     &b->nhb, &b->nlb, &b->args, &b->mols, &b->cnv, &b->st, &b->act, &b->doeig, &b->mode, &b->niter,
