@@ -191,20 +191,23 @@ def main():
     dhf = abs(fast_last["escf"] - ref["escf"]) if ref else None
     dp = float(np.max(np.abs(fast_last["p"] - ref["p"]))) if ref else None
 
-    # ---- roofline: dominant kernel of the measured (fast) form, HIP events on
-    # the stream every kernel is launched on
+    # ---- roofline: dominant kernel class of the measured (fast) form, HIP events
+    # on the stream every kernel is launched on
     n = s.norbs
     jv = [ctypes.c_double(), ctypes.c_longlong(), ctypes.c_double(), ctypes.c_longlong(),
           ctypes.c_double(), ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_longlong(),
           ctypes.c_longlong()]
     jrefs = [ctypes.byref(v) for v in jv]
-    nk = 4
+    nk = 5
     kms, kl, kf, kb = (np.zeros(nk), np.zeros(nk, dtype=np.int64), np.zeros(nk), np.zeros(nk))
-    lib.mhip_kernel_timing(ctx.h, 1, *jrefs)
+    # every class as the fast SCF launches it
     lib.mhip_kernel_stats(ctx.h, 1, nk, None, None, None, None)
     run_fast()
     lib.mhip_kernel_stats(ctx.h, -1, nk, L.ptr(kms), L.ptr(kl), L.ptr(kf), L.ptr(kb))
     lib.mhip_kernel_stats(ctx.h, 0, nk, None, None, None, None)
+    # the parts of the Jacobi steps one after another, and what they processed
+    lib.mhip_kernel_timing(ctx.h, 1, *jrefs)
+    run_fast()
     lib.mhip_kernel_timing(ctx.h, 0, *jrefs)
     solve_ms, n_solve, apply_ms, n_apply, applyc_ms, n_applyc, tiles, pairs, rotations = [v.value for v in jv]
     npad = ((n + 63) // 64) * 64
@@ -214,11 +217,13 @@ def main():
     # its group (the exit diagonalization's occupied or virtual one); solve = the
     # rotations the library counted (32 x 32 cross rounds per pair, plus 2 x 496
     # inside the blocks once per sweep) x (64 + 64 + 64 element pairs) x 6 flops
-    entries = [
-        ("k_jac_solve", "mfma", solve_ms, n_solve, rotations * 3.0 * 64 * 6, 0.0),
-        ("k_jac_apply_a_mfma", "mfma", apply_ms, n_apply, tiles * 2.0 * 2.0 * 64 ** 3, 0.0),
-        ("k_jac_apply_c_mfma", "mfma", applyc_ms, n_applyc, pairs * 2.0 * c_rows * 64 * 64, 0.0),
+    parts = [
+        ("solves", "mfma", solve_ms, n_solve, rotations * 3.0 * 64 * 6, 0.0),
+        ("tiles of A", "mfma", apply_ms, n_apply, tiles * 2.0 * 2.0 * 64 ** 3, 0.0),
+        ("tiles of C", "mfma", applyc_ms, n_applyc, pairs * 2.0 * c_rows * 64 * 64, 0.0),
     ]
+    kf[4] = sum(e[4] for e in parts)
+    entries = []
     for i in range(nk):
         name = lib.mhip_kernel_class_name(i).decode()
         bound = "hbm" if "fock" in name else "mfma"
@@ -228,8 +233,9 @@ def main():
             return None
         return round((e[5] / 1e9 if e[1] == "hbm" else e[4] / 1e12) / (e[2] * 1e-3), 2)
 
-    breakdown = {e[0]: {"ms": round(e[2], 3), "launches": int(e[3]),
-                        ("GB/s" if e[1] == "hbm" else "TFLOP/s"): rate(e)} for e in entries if e[3] > 0}
+    def table(es):
+        return {e[0]: {"ms": round(e[2], 3), "launches": int(e[3]),
+                       ("GB/s" if e[1] == "hbm" else "TFLOP/s"): rate(e)} for e in es if e[3] > 0}
     name, bound, tot_ms, nl, flops, nbytes = max(entries, key=lambda e: e[2])
     avg_s = (tot_ms / max(nl, 1)) * 1e-3
     if bound == "hbm":
@@ -261,7 +267,8 @@ def main():
             "algorithmic_bytes_per_launch": round(nbytes / max(nl, 1)) if nbytes else None, "kernel": name,
             "avg_launch_us": round(avg_s * 1e6, 2), "launches": int(nl),
             "algorithmic_per_launch": round((nbytes if bound == "hbm" else flops) / max(nl, 1)),
-            "kernel_ms_in_one_fast_scf": breakdown}
+            "kernel_ms_in_one_fast_scf": table(entries),
+            "k_jac_step_parts_launched_one_by_one": table(parts)}
 
     # ---- CPU baseline: the FP64 restatement (MKL dsyevd) on host cores
     cpu = None

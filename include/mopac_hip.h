@@ -531,8 +531,9 @@ int mhip_set_tuning(mhip_ctx* ctx, int kernel_variant, int max_inner, double tol
 int mhip_set_jacobi_schedule(int schedule);
 /* Block-Jacobi sweeps used by the last eigensolve of this context. */
 int mhip_last_sweeps(mhip_ctx* ctx);
-/* HIP-event timing of the block-Jacobi solve / A-update / C-update launches
- * on the context's stream.  Returns the accumulated milliseconds and launch
+/* HIP-event timing of the block-Jacobi solves, A updates and C updates on the
+ * context's stream, which run together in a step's one launch and one after
+ * another while this is on.  Returns the accumulated milliseconds and launch
  * counts, the 64x64 tiles / block pairs the timed launches actually
  * processed and the 2x2 rotations of the timed pair solves; enable = 1 or 0
  * resets and switches timing on or off, -1 only reads. */
@@ -541,10 +542,11 @@ int mhip_kernel_timing(mhip_ctx* ctx, int enable, double* solve_ms, long long* n
                        long long* n_applyc, long long* active_tiles, long long* active_pairs,
                        long long* rotations);
 
-/* Process-wide HIP-event timing of the other kernel classes (FP64 GEMM,
- * split-BF16 GEMM, packed density, fock2), on the stream each launch uses.
+/* Process-wide HIP-event timing of kernel classes (FP64 GEMM, split-BF16 GEMM,
+ * packed density, fock2, the block-Jacobi steps as the eigensolver launches
+ * them), on the stream each launch uses.
  * enable = 1 / 0 resets and switches it on / off; -1 fills, per class
- * (index < max_classes, at most 4), the summed milliseconds, launches,
+ * (index < max_classes, at most 5), the summed milliseconds, launches,
  * algorithmic flops and algorithmic HBM bytes of the recorded launches. */
 int mhip_kernel_stats(mhip_ctx* ctx, int enable, int max_classes, double* ms, long long* launches,
                       double* flops, double* bytes);

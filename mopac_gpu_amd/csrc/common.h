@@ -69,6 +69,7 @@ enum KClass {
   K_GEMM_SPLIT,      // gemm_split_bf16: 2 m n k (FP64-equivalent) flops
   K_SYRK_F64,        // packed density: n (n + 1) k flops
   K_FOCK,            // fock_build (row + column pass): 8 (n2elec + 4 mpack) bytes
+  K_JACOBI,          // a block-Jacobi step (its flops depend on the pairs that rotate)
   K_NCLASS
 };
 struct KTimer {

@@ -2,11 +2,12 @@
 //
 // The matrix (padded to a multiple of 64 with decoupled large diagonal
 // entries) is split into 32-wide blocks.  A sweep visits every block pair once
-// in round-robin order; each step
-//   1. diagonalizes the 64x64 submatrix of every pair in LDS (inner cyclic
-//      Jacobi, one workgroup per pair) giving an orthogonal Q_pair,
-//   2. applies A <- Qt^T A Qt tile by tile (two 64^3 products per tile),
-//   3. applies C <- C Qt to the eigenvector accumulator.
+// in round-robin order; a step turns every pair's two blocks by the orthogonal
+// Q_pair that its 64x64 submatrix asks for (a workgroup per pair, in its LDS):
+// A <- Qt^T A Qt tile by tile (two 64^3 products per tile), C <- C Qt.  One
+// launch (k_jac_step) applies a step to A and C and solves the pairs of the
+// next.  The comparison form (schedule 0: cyclic Jacobi over all 64 indices)
+// takes three launches a step.
 // In the SCF the solver starts from the previous eigenvectors (A = C^T F C is
 // then nearly diagonal and one to three sweeps converge it); the first call
 // starts from C = I.  Stopping test: max |A_ij| (i != j) <= tol * max|A_ii|.
@@ -612,7 +613,8 @@ static int sweeps_in_range(hipStream_t s, JacobiPlan& plan, double*& A, double*&
   // used keeps every workgroup alone.  SCFs at 1020 orbitals (408 workgroups)
   // 53.3 -> 49.4 ms, 1200 (570) 71.2 -> 66.4, 1500 (900) equal, 1800 (1305)
   // 133 -> 160.
-  const size_t alone = npairs + ntiles + nctiles <= 3 * 256 ? 16384 : 0;
+  const int total = npairs + ntiles + nctiles;
+  const size_t alone = total <= 3 * 256 ? 16384 : 0;
   auto launch_step = [&](int step, double skip_abs, int from, int to, SweepTest test) {
     const int next = (step + 1) % nsteps;
     const JacStep a{A,          ahead ? A2 : A,  C,                lda,
@@ -621,10 +623,13 @@ static int sweeps_in_range(hipStream_t s, JacobiPlan& plan, double*& A, double*&
                     intra_of(next), plan.where.as<int>() + (size_t)step * plan.nb, qslot(slot ^ 1), aslot(slot ^ 1),
                     dslot(slot), dslot(slot ^ 1), inner_tol,       skip_abs,
                     inner,      crows};
-    hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from, test);
-    MHIP_LAUNCH_CHECK();
+    auto launch = [&] {
+      hipLaunchKernelGGL(k_jac_step, dim3(to - from), dim3(CROSS_THREADS), alone, s, a, from, test);
+      MHIP_LAUNCH_CHECK();
+    };
+    if (ahead && to - from == total) timed(s, K_JACOBI, 0.0, 0.0, launch);
+    else launch();
   };
-  const int total = npairs + ntiles + nctiles;
   plan.ensure_test_event(s);
   for (int sw = 0; sw <= max_sweeps; ++sw) {
     hipLaunchKernelGGL(k_offmax_partial, dim3(plan.n), dim3(256), 0, s, plan.n, A, lda,

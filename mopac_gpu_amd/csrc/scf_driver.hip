@@ -390,8 +390,9 @@ static void pulay_step(mhip_ctx* c, PulayState& st, double* pl_out) {
   // FP - PF (P = alpha density), packed as the reference packs it
   unpack_sym(s, n, c->pa.as<double>(), c->fd.as<double>(), np, np, 0.0);
   unpack_sym(s, n, c->f.as<double>(), c->T.as<double>(), np, np, 0.0);
-  // with the padding (zero), whose size divides the large tiles: 96 -> 17 us
-  // at 462 orbitals
+  // with the padding, whose size divides the large tiles: 96 -> 17 us at 462
+  // orbitals.  Of it only the diagonals are not zero, and the products they
+  // make stay there.
   gemm(s, 'N', 'N', np, np, np, 1.0, c->fd.as<double>(), np, c->T.as<double>(), np, 0.0,
        c->A.as<double>(), np);
   pack_antisym(s, n, c->A.as<double>(), np, eh + (size_t)(lfock - 1) * mp);
@@ -1062,7 +1063,8 @@ int mhip_last_sweeps(mhip_ctx* c) { return c ? c->last_sweeps : 0; }
 // disable (0) and reset; read back accumulated milliseconds and launch counts.
 const char* mhip_kernel_class_name(int cls) {
   static const char* names[K_NCLASS] = {"k_gemm_mfma (FP64 GEMM)", "k_gemm_split_bf16 (split-BF16 GEMM)",
-                                        "k_syrk_packed_mfma (density)", "k_fock_rows+k_fock_cols (fock2)"};
+                                        "k_syrk_packed_mfma (density)", "k_fock_rows+k_fock_cols (fock2)",
+                                        "k_jac_step (block-Jacobi step)"};
   return (cls >= 0 && cls < K_NCLASS) ? names[cls] : "";
 }
 
