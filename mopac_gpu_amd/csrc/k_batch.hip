@@ -705,7 +705,7 @@ __device__ double2 cnvg_diag_wave(int n, double* __restrict__ pnew, double* __re
 // run.  No molecule waits for another: in lockstep, a launch per phase over
 // all molecules, every iteration took the longest eigensolve of its size
 // class and twenty launches, and 64 molecules took 109 ms where they now take
-// 15 (400: 137 -> 25, 4096: 403 -> 222).  With M.fexit, a finished molecule is
+// 13 (400: 137 -> 23, 4096: 403 -> 213).  With M.fexit, a finished molecule is
 // diagonalized once more to 1e-12, as iter does at its exit, and phase_lock'ed
 // if asked.
 template <int NT, bool LDS>

@@ -1,4 +1,4 @@
-"""GPU tests of the batched SCF (one captured graph for many molecules):
+"""GPU tests of the batched SCF (many molecules in one call):
 every molecule's heat of formation, iteration count and density against the
 CPU oracle running the reference's loop on the same molecule."""
 import numpy as np
